@@ -9,10 +9,11 @@
 // of the f64 sum.  Ranking: highest score first, equal scores by the lower row
 // index, so the result is deterministic.
 //
-// registry_tile_kernel: a workgroup scores a 64 x 256 (queries x rows)
-// tile and writes each query's best k rows of it as candidates;
-// registry_merge_kernel: one workgroup per query takes the best k of its
-// ceil(N/256) * k candidates.
+// registry_score_kernel: the scores on f64 MFMA (v_mfma_f64_16x16x4), a
+// workgroup's chunk of rows staged in LDS and its best k rows per query picked
+// there; one sorted candidate list per query and chunk goes out.
+// registry_merge_kernel: one workgroup per query picks the best k of its
+// candidates.
 #include <cfloat>
 
 #include "common.hpp"
@@ -21,7 +22,14 @@
 namespace vdk {
 namespace {
 
-constexpr int kTQ = 64, kTR = 256, kDC = 32, kMaxK = 64, kMergeMax = 32;
+constexpr int kMaxK = 64;
+// Rows per workgroup of the score kernel, i.e. per candidate list: 256, or 64
+// up to 16384 rows, where 256 would leave most CUs idle (1 x 3000 x 256, k = 5:
+// 12 workgroups against 47).  A caller's workspace sized for lists of 256 rows
+// is enough: the lists are then 256 rows long.
+constexpr int kRows = 256, kRowsSmall = 64, kSmallN = 16384;
+
+typedef double double4v __attribute__((ext_vector_type(4)));
 
 // (s, i) ranks before (t, j): higher score, then lower index
 __device__ __forceinline__ bool ranks_before(double s, int i, double t, int j) {
@@ -39,159 +47,362 @@ __device__ __forceinline__ void lane_best(double& s, int& i) {
     }
 }
 
-// A workgroup scores 64 queries x 256 rows, 8 x 8 per thread (thread
-// ty*32 + tx: queries 8*ty.., rows 8*tx..), over D in chunks of 32 staged
-// through LDS as f32 (converted to f64 at use; the products are exact).
-// Then the 32 threads of a query group (one half-wave) pick each of their 8
-// queries' best k rows of the tile: k rounds of (each thread's best row that
-// ranks after the previous pick, then a half-wave arg-max).
-__global__ __launch_bounds__(256) void registry_tile_kernel(const float* __restrict__ q, int B,
-                                                            const float* __restrict__ reg, int N, int D, int k,
-                                                            double* __restrict__ cand_s, int* __restrict__ cand_i) {
-    __shared__ __attribute__((aligned(16))) float sq[kDC][kTQ + 4];   // [dim][query]
-    __shared__ __attribute__((aligned(16))) float sr[kDC][kTR + 4];   // [dim][row]
-    const int tid = threadIdx.x, tx = tid & 31, ty = tid >> 5;
-    const int q0 = blockIdx.y * kTQ, n0 = blockIdx.x * kTR;
+// A pick of the best k out of many, used by both kernels below.  The values
+// are dealt out to G >= k groups; the k-th best of the groups' maxima ranks at
+// or after the k-th best value, so every value of the answer ranks at or
+// before it ("the bar"), and few others do (k = 10 of 256 with 16 groups: 16).
+// Those few are listed and each one's rank among them counted.  Groups are
+// strided over the rows, so runs of equal scores (rows of zeros, duplicates)
+// raise the bar to their k-th row instead of listing them all.
 
-    double acc[8][8];
-#pragma unroll
-    for (int i = 0; i < 8; ++i)
-#pragma unroll
-        for (int j = 0; j < 8; ++j) acc[i][j] = 0.0;
+// A wave scores 16 * RT rows x 16 * QT queries, the workgroup 16 * NW * RT
+// rows.  Lane l = 16 g + c feeds row / query c of each 16-wide block:
+// one 16-byte load covers its 4 values of a 16-dim step (dims 4 g .. 4 g + 3,
+// converted to f64 at use; the products are exact), of which MFMA j takes
+// value j, so a score is summed over the dims in the order (step, j, g)
+// whatever the launch's shape.  Loads go straight to registers, P steps ahead:
+// a step's QT + RT loads feed 4 * QT * RT MFMAs of 64 cycles, so neither LDS
+// nor L1 bandwidth matters and f64 MFMA is the bound (64 x 100000 x 192:
+// 37 us at the 67 TFLOP/s that MFMAs alone reach; this kernel 79 us at k = 10,
+// of which the pick is 12; the f64 FMA kernel it replaces 171 us, bound by its
+// LDS reads, conversions and its k rounds of arg-max exchanges).
+template <int NW, int QT, int RT, int P, int G>
+__global__ __launch_bounds__(NW * 64) void registry_score_kernel(const float* __restrict__ q, int B,
+                                                             const float* __restrict__ reg, int N, int D, int k,
+                                                             double* __restrict__ cand_s, int* __restrict__ cand_i) {
+    constexpr int NQ = 16 * QT, NR = 16 * NW * RT, LD = NR + 8;   // + 64 bytes: neighbouring queries on other banks
+    constexpr int TPQ = NW * 64 / NQ, RPT = NR / TPQ, GPT = G / TPQ;   // threads per query, rows / groups per thread
+    static_assert(TPQ <= 64 && GPT >= 1 && GPT <= RPT && RPT % GPT == 0 && NR <= 256, "selection shape");
+    extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
+    double* const sc = reinterpret_cast<double*>(smem);                        // [NQ][LD] scores
+    uint8_t* const list = smem + sizeof(double) * NQ * LD;                     // [NQ][NR] rows past the bar
+    int* const count = reinterpret_cast<int*>(list + NQ * NR);                 // [NQ]
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, c = lane & 15, g = lane >> 4;
+    const int q0 = blockIdx.y * NQ, b0 = blockIdx.x * NR, n0 = b0 + wave * 16 * RT;
 
-    for (int d0 = 0; d0 < D; d0 += kDC) {
-        // 16-byte loads (D % 4 == 0), stored transposed
-        for (int e = tid; e < kTQ * kDC / 4; e += 256) {
-            const int r = e / (kDC / 4), c = (e - r * (kDC / 4)) * 4, d = d0 + c;
-            const float4v v = (q0 + r < B && d < D) ? *reinterpret_cast<const float4v*>(q + (size_t)(q0 + r) * D + d)
-                                                    : float4v{0.0f, 0.0f, 0.0f, 0.0f};
+    double4v acc[RT][QT];
 #pragma unroll
-            for (int t = 0; t < 4; ++t) sq[c + t][r] = v[t];
-        }
-        for (int e = tid; e < kTR * kDC / 4; e += 256) {
-            const int r = e / (kDC / 4), c = (e - r * (kDC / 4)) * 4, d = d0 + c;
-            const float4v v = (n0 + r < N && d < D) ? *reinterpret_cast<const float4v*>(reg + (size_t)(n0 + r) * D + d)
-                                                    : float4v{0.0f, 0.0f, 0.0f, 0.0f};
+    for (int r = 0; r < RT; ++r)
 #pragma unroll
-            for (int t = 0; t < 4; ++t) sr[c + t][r] = v[t];
-        }
-        __syncthreads();
-#pragma unroll 2
-        for (int c = 0; c < kDC; ++c) {
-            const float4v a0 = *reinterpret_cast<const float4v*>(&sq[c][ty * 8]);
-            const float4v a1 = *reinterpret_cast<const float4v*>(&sq[c][ty * 8 + 4]);
-            const float4v b0 = *reinterpret_cast<const float4v*>(&sr[c][tx * 8]);
-            const float4v b1 = *reinterpret_cast<const float4v*>(&sr[c][tx * 8 + 4]);
-            double a[8], b[8];
+        for (int t = 0; t < QT; ++t) acc[r][t] = double4v{0.0, 0.0, 0.0, 0.0};
+
+    if (n0 < N) {   // (wave-uniform)
+        // rows and queries past the end read the last one; they are masked below
+        const float *rp[RT], *qp[QT];
 #pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                a[e] = a0[e]; a[e + 4] = a1[e];
-                b[e] = b0[e]; b[e + 4] = b1[e];
+        for (int r = 0; r < RT; ++r) rp[r] = reg + (size_t)min(n0 + 16 * r + c, N - 1) * D + 4 * g;
+#pragma unroll
+        for (int t = 0; t < QT; ++t) qp[t] = q + (size_t)min(q0 + 16 * t + c, B - 1) * D + 4 * g;
+        const int ns = (D + 15) >> 4;
+        const float4v zero{0.0f, 0.0f, 0.0f, 0.0f};
+        float4v rv[2][P][RT], qv[2][P][QT];
+        auto load = [&](int buf, int s0) {
+#pragma unroll
+            for (int p = 0; p < P; ++p) {
+                const int d = (s0 + p) * 16;
+                const bool on = d + 4 * g < D;   // D % 4 == 0
+#pragma unroll
+                for (int r = 0; r < RT; ++r)
+                    rv[buf][p][r] = on ? *reinterpret_cast<const float4v*>(rp[r] + d) : zero;
+#pragma unroll
+                for (int t = 0; t < QT; ++t)
+                    qv[buf][p][t] = on ? *reinterpret_cast<const float4v*>(qp[t] + d) : zero;
             }
+        };
+        auto compute = [&](int buf) {
 #pragma unroll
-            for (int i = 0; i < 8; ++i)
+            for (int p = 0; p < P; ++p)
 #pragma unroll
-                for (int j = 0; j < 8; ++j) acc[i][j] = fma(a[i], b[j], acc[i][j]);
+                for (int j = 0; j < 4; ++j) {
+                    double b[QT];
+#pragma unroll
+                    for (int t = 0; t < QT; ++t) b[t] = (double)qv[buf][p][t][j];
+#pragma unroll
+                    for (int r = 0; r < RT; ++r) {
+                        const double a = (double)rv[buf][p][r][j];
+#pragma unroll
+                        for (int t = 0; t < QT; ++t)
+                            acc[r][t] = __builtin_amdgcn_mfma_f64_16x16x4f64(a, b[t], acc[r][t], 0, 0, 0);
+                    }
+                }
+        };
+        load(0, 0);
+#pragma unroll 1
+        for (int s = 0; s < ns; s += 2 * P) {
+            load(1, s + P);   // past the end: zeros, not loads
+            compute(0);
+            load(0, s + 2 * P);
+            compute(1);
         }
-        __syncthreads();
     }
 
-    const int nchunks = gridDim.x;
+    // accumulator i of lane (g, c) is row 4 i + g of its block, query c; scores
+    // that are not finite are never picked
+    const double kNone = -__builtin_inf();
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-        const int qq = q0 + ty * 8 + i;   // uniform over the half-wave
-        if (qq >= B) break;
-        double last_s = DBL_MAX;
-        int last_i = -1;
-        for (int r = 0; r < k; ++r) {
-            double bs = -DBL_MAX;
-            int bi = INT_MAX;
+    for (int t = 0; t < QT; ++t)
 #pragma unroll
-            for (int j = 0; j < 8; ++j) {
-                const int row = n0 + tx * 8 + j;
-                const double sj = acc[i][j];
-                if (row < N && ranks_before(last_s, last_i, sj, row) && ranks_before(sj, row, bs, bi)) {
-                    bs = sj;
-                    bi = row;
+        for (int r = 0; r < RT; ++r)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const int row = (wave * RT + r) * 16 + 4 * i + g;
+                const double v = acc[r][t][i];
+                sc[(16 * t + c) * LD + row] = b0 + row < N && v >= -DBL_MAX && v <= DBL_MAX ? v : kNone;
+            }
+    if (tid < NQ) count[tid] = 0;
+    __syncthreads();
+
+    const int qi = tid / TPQ, t = tid - qi * TPQ;   // (a query's threads are neighbours in one wave)
+    const double* const sq = sc + qi * LD;
+    // the maxima of this thread's groups (row t + TPQ * j is in group j % GPT), lower rows first
+    double gs[GPT];
+    int gr[GPT];
+#pragma unroll
+    for (int u = 0; u < GPT; ++u) { gs[u] = kNone; gr[u] = INT_MAX; }
+#pragma unroll
+    for (int j = 0; j < RPT; ++j) {
+        const double v = sq[t + TPQ * j];
+        if (v > gs[j % GPT]) { gs[j % GPT] = v; gr[j % GPT] = t + TPQ * j; }
+    }
+    // the bar: the k-th best maximum (nothing is barred while fewer than k groups hold a score)
+    int rank[GPT];
+#pragma unroll
+    for (int u = 0; u < GPT; ++u) rank[u] = 0;
+#pragma unroll 4
+    for (int o = 0; o < TPQ; ++o)
+#pragma unroll
+        for (int w = 0; w < GPT; ++w) {
+            const double os = __shfl(gs[w], o, TPQ);
+            const int orow = __shfl(gr[w], o, TPQ);
+#pragma unroll
+            for (int u = 0; u < GPT; ++u) rank[u] += ranks_before(os, orow, gs[u], gr[u]) ? 1 : 0;
+        }
+    double bar = kNone;
+    int bar_row = INT_MAX;
+#pragma unroll
+    for (int u = 0; u < GPT; ++u)
+        if (rank[u] == k - 1) { bar = gs[u]; bar_row = gr[u]; }
+#pragma unroll
+    for (int off = TPQ / 2; off > 0; off >>= 1) {
+        const double os = __shfl_xor(bar, off, TPQ);
+        const int orow = __shfl_xor(bar_row, off, TPQ);
+        if (os > bar) { bar = os; bar_row = orow; }
+    }
+#pragma unroll
+    for (int j = 0; j < RPT; ++j) {
+        const int row = t + TPQ * j;
+        const double v = sq[row];
+        if (v > bar || (v == bar && row <= bar_row && v > kNone)) list[qi * NR + atomicAdd(&count[qi], 1)] = (uint8_t)row;
+    }
+    __syncthreads();
+    if (q0 + qi >= B) return;
+    const int n = count[qi];
+    const uint8_t* const lq = list + qi * NR;
+    const size_t o = ((size_t)(q0 + qi) * gridDim.x + blockIdx.x) * k;
+    if (G > 16 && n > k) {
+        // many past the bar (k = 64 of 256: 166): a score that exactly k exceed, by
+        // bisection between the bar and the best (n * n / TPQ comparisons to
+        // rank them all took 750 us at 64 x 100000, k = 64)
+        double lo = bar, hi = kNone;
+#pragma unroll
+        for (int u = 0; u < GPT; ++u) hi = fmax(hi, gs[u]);
+#pragma unroll
+        for (int off = TPQ / 2; off > 0; off >>= 1) hi = fmax(hi, __shfl_xor(hi, off, TPQ));
+        int found = -1;
+        for (int it = 0; it < 48; ++it) {
+            const double mid = 0.5 * lo + 0.5 * hi;
+            int above = 0;
+#pragma unroll
+            for (int j = 0; j < RPT; ++j) above += sq[t + TPQ * j] > mid ? 1 : 0;
+#pragma unroll
+            for (int off = TPQ / 2; off > 0; off >>= 1) above += __shfl_xor(above, off, TPQ);
+            found = above == k ? 1 : found;
+            if (found < 0 && above > k) lo = mid;
+            if (found < 0 && above < k) hi = mid;
+            if (found > 0) lo = hi = mid;   // (stays)
+            if (__all(found > 0)) break;
+        }
+        if (found > 0) {   // (the same for a query's threads)
+            int at = 0;
+#pragma unroll
+            for (int j = 0; j < RPT; ++j) at += sq[t + TPQ * j] > hi ? 1 : 0;
+            int before = at;   // exclusive prefix over the query's threads
+#pragma unroll
+            for (int off = 1; off < TPQ; off <<= 1) {
+                const int x = __shfl_up(before, off, TPQ);
+                before += t >= off ? x : 0;
+            }
+            size_t w = o + before - at;
+#pragma unroll
+            for (int j = 0; j < RPT; ++j) {
+                const double v = sq[t + TPQ * j];
+                if (v > hi) {
+                    cand_s[w] = v;
+                    cand_i[w++] = b0 + t + TPQ * j;
                 }
             }
-            lane_best<32>(bs, bi);
-            if (tx == 0) {
-                const size_t o = ((size_t)qq * nchunks + blockIdx.x) * k + r;
-                cand_s[o] = bs;
-                cand_i[o] = bi;   // INT_MAX when the tile has fewer than k rows left
-            }
-            last_s = bs;
-            last_i = bi;
+            return;
         }
+    }
+    for (int e = t; e < n; e += TPQ) {
+        const int row = lq[e];
+        const double v = sq[row];
+        int r = 0;
+#pragma unroll 4
+        for (int m = 0; m < n; ++m) {
+            const int orow = lq[m];
+            r += ranks_before(sq[orow], orow, v, row) ? 1 : 0;
+        }
+        if (r < k) {
+            cand_s[o + r] = v;
+            cand_i[o + r] = b0 + row;
+        }
+    }
+    for (int r = n + t; r < k; r += TPQ) {   // the chunk has fewer than k rows left
+        cand_s[o + r] = -DBL_MAX;
+        cand_i[o + r] = INT_MAX;
     }
 }
 
-// One workgroup per query: k rounds of a block-wide arg-max over the
-// candidates that rank after the previous pick.  Up to 256 * kMergeMax
-// candidates are held in registers (32 per thread); beyond that each round
-// scans them in global memory.
-__global__ __launch_bounds__(256) void registry_merge_kernel(const double* __restrict__ cand_s,
-                                                             const int* __restrict__ cand_i, int ncand, int k,
-                                                             int* __restrict__ out_i, float* __restrict__ out_s) {
-    __shared__ double ws[4];
-    __shared__ int wi[4];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, qq = blockIdx.x;
-    const double* cs = cand_s + (size_t)qq * ncand;
-    const int* ci = cand_i + (size_t)qq * ncand;
-    const bool in_regs = ncand <= kMergeMax * 256;
-    double mys[kMergeMax];
-    int myi[kMergeMax];
+// One workgroup of NT threads per query picks the best k of its n <= NT * M
+// candidates (M = 0: any number, re-read) by the bar of 64 groups; should more
+// than kMergeList pass the bar, by k rounds of a workgroup arg-max.  Bound by its
+// latencies (one round trip to memory, then ~1000 instructions in a row): 64
+// queries x 391 lists of 10 take 10 us, 21.8 with the rounds alone.
+constexpr int kMergeList = 2048;
+template <int NT, int M>
+__global__ __launch_bounds__(NT) void registry_merge_kernel(const double* __restrict__ cand_s,
+                                                            const int* __restrict__ cand_i, int n, int k,
+                                                            int* __restrict__ out_i, float* __restrict__ out_s) {
+    constexpr int NW = NT / 64;
+    __shared__ double gs[NW][64], ls[kMergeList], bar_s;
+    __shared__ int gi[NW][64], li[kMergeList], bar_i, count;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const double* const cs = cand_s + (size_t)blockIdx.x * n;
+    const int* const ci = cand_i + (size_t)blockIdx.x * n;
+    out_i += (size_t)blockIdx.x * k;
+    out_s += (size_t)blockIdx.x * k;
+    // the thread's candidates: M in registers, or (M = 0) re-read on each pass
+    double v[M ? M : 1];
+    int id[M ? M : 1];
+    if constexpr (M > 0) {
 #pragma unroll
-    for (int m = 0; m < kMergeMax; ++m) {
-        const int c = tid + m * 256;
-        mys[m] = in_regs && c < ncand ? cs[c] : -DBL_MAX;
-        myi[m] = in_regs && c < ncand ? ci[c] : INT_MAX;
+        for (int m = 0; m < M; ++m) {
+            const int e = tid + m * NT;
+            v[m] = e < n ? cs[e] : -DBL_MAX;
+            id[m] = e < n ? ci[e] : INT_MAX;
+        }
+    }
+    auto each = [&](auto f) {
+        if constexpr (M > 0) {
+#pragma unroll
+            for (int m = 0; m < M; ++m) f(v[m], id[m]);
+        } else {
+#pragma unroll 4
+            for (int e = tid; e < n; e += NT) f(cs[e], ci[e]);
+        }
+    };
+    if (tid == 0) count = 0;
+    double s = -DBL_MAX;
+    int i = INT_MAX;
+    each([&](double x, int xi) {
+        if (ranks_before(x, xi, s, i)) { s = x; i = xi; }
+    });
+    gs[wave][lane] = s;
+    gi[wave][lane] = i;
+    __syncthreads();
+    if (wave == 0) {
+#pragma unroll
+        for (int w = 1; w < NW; ++w)
+            if (ranks_before(gs[w][lane], gi[w][lane], s, i)) { s = gs[w][lane]; i = gi[w][lane]; }
+        int rank = 0;
+#pragma unroll 8
+        for (int o = 0; o < 64; ++o) {
+            const double os = __shfl(s, o);
+            const int oi = __shfl(i, o);
+            // empty groups (INT_MAX) are told apart by their lanes
+            rank += ranks_before(os, oi, s, i) || (i == INT_MAX && oi == INT_MAX && o < lane) ? 1 : 0;
+        }
+        if (rank == k - 1) { bar_s = s; bar_i = i; }   // (i == INT_MAX: nothing is barred)
+    }
+    __syncthreads();
+    const double bs = bar_s;
+    const int bi = bar_i;
+    each([&](double x, int xi) {
+        if (xi != INT_MAX && !ranks_before(bs, bi, x, xi)) {
+            const int at = atomicAdd(&count, 1);
+            if (at < kMergeList) { ls[at] = x; li[at] = xi; }
+        }
+    });
+    __syncthreads();
+    const int nl = count;
+    if (nl <= kMergeList) {
+        for (int e = tid; e < nl; e += NT) {
+            int r = 0;
+#pragma unroll 4
+            for (int m = 0; m < nl; ++m) r += ranks_before(ls[m], li[m], ls[e], li[e]) ? 1 : 0;
+            if (r < k) {
+                out_i[r] = li[e];
+                out_s[r] = (float)ls[e];
+            }
+        }
+        for (int r = nl + tid; r < k; r += NT) {   // fewer than k finite scores
+            out_i[r] = INT_MAX;
+            out_s[r] = (float)-DBL_MAX;
+        }
+        return;
     }
     double last_s = DBL_MAX;
     int last_i = -1;
     for (int r = 0; r < k; ++r) {
-        double bs = -DBL_MAX;
-        int bi = INT_MAX;
-        if (in_regs) {
-#pragma unroll
-            for (int m = 0; m < kMergeMax; ++m)
-                if (myi[m] != INT_MAX && ranks_before(last_s, last_i, mys[m], myi[m]) &&
-                    ranks_before(mys[m], myi[m], bs, bi)) {
-                    bs = mys[m];
-                    bi = myi[m];
-                }
-        } else {
-            for (int c = tid; c < ncand; c += 256) {
-                const double sc = cs[c];
-                const int ic = ci[c];
-                if (ic != INT_MAX && ranks_before(last_s, last_i, sc, ic) && ranks_before(sc, ic, bs, bi)) {
-                    bs = sc;
-                    bi = ic;
-                }
+        double b = -DBL_MAX;
+        int j = INT_MAX;
+        each([&](double x, int xi) {
+            if (xi != INT_MAX && ranks_before(last_s, last_i, x, xi) && ranks_before(x, xi, b, j)) {
+                b = x;
+                j = xi;
             }
-        }
-        lane_best<64>(bs, bi);
-        if (lane == 0) { ws[wave] = bs; wi[wave] = bi; }
+        });
+        lane_best<64>(b, j);
+        __syncthreads();   // the previous round's maxima are read
+        if (lane == 0) { gs[wave][0] = b; gi[wave][0] = j; }
         __syncthreads();
-        bs = ws[0];
-        bi = wi[0];
 #pragma unroll
-        for (int w = 1; w < 4; ++w)
-            if (ranks_before(ws[w], wi[w], bs, bi)) { bs = ws[w]; bi = wi[w]; }
-        __syncthreads();
+        for (int w = 0; w < NW; ++w)
+            if (ranks_before(gs[w][0], gi[w][0], b, j)) { b = gs[w][0]; j = gi[w][0]; }
         if (tid == 0) {
-            out_i[(size_t)qq * k + r] = bi;
-            out_s[(size_t)qq * k + r] = (float)bs;
+            out_i[r] = j;
+            out_s[r] = (float)b;
         }
-        last_s = bs;
-        last_i = bi;
+        last_s = b;
+        last_i = j;
     }
 }
 
-size_t workspace_bytes(int B, int N, int k) {
-    const size_t nchunks = (size_t)(N + kTR - 1) / kTR;
-    return (size_t)B * nchunks * k * (sizeof(double) + sizeof(int)) + 256;
+size_t workspace_bytes(int B, int N, int k, int rows) {
+    const size_t lists = (size_t)(N + rows - 1) / rows;
+    return (size_t)B * lists * k * (sizeof(double) + sizeof(int)) + 256;
+}
+
+template <int NW, int QT, int RT, int P, int G>
+void launch_score(const float* q, int B, const float* reg, int N, int D, int k, double* cand_s, int* cand_i,
+                  hipStream_t s) {
+    constexpr int NQ = 16 * QT, NR = 16 * NW * RT;
+    constexpr int lds = sizeof(double) * NQ * (NR + 8) + NQ * NR + sizeof(int) * NQ;
+    if (lds > 64 * 1024)
+        VDK_HIP(hipFuncSetAttribute((const void*)registry_score_kernel<NW, QT, RT, P, G>,
+                                    hipFuncAttributeMaxDynamicSharedMemorySize, lds));
+    hipLaunchKernelGGL((registry_score_kernel<NW, QT, RT, P, G>), dim3(cdiv(N, NR), cdiv(B, NQ)),
+                       dim3(NW * 64), lds, s, q, B,
+                       reg, N, D, k, cand_s, cand_i);
+    VDK_HIP(hipGetLastError());
+}
+
+template <int NW, int QT, int RT, int P>
+void launch_score_k(const float* q, int B, const float* reg, int N, int D, int k, double* cand_s, int* cand_i,
+                    hipStream_t s) {
+    if (k <= 16) launch_score<NW, QT, RT, P, 16>(q, B, reg, N, D, k, cand_s, cand_i, s);
+    else launch_score<NW, QT, RT, P, 64>(q, B, reg, N, D, k, cand_s, cand_i, s);
 }
 
 }  // namespace
@@ -201,7 +412,7 @@ using namespace vdk;
 
 extern "C" size_t vdk_registry_topk_workspace_size(int B, int N, int k) {
     if (B <= 0 || N <= 0 || k <= 0) return 0;
-    return workspace_bytes(B, N, k);
+    return workspace_bytes(B, N, k, N <= kSmallN ? kRowsSmall : kRows);
 }
 
 extern "C" int vdk_registry_topk(const float* d_queries, int B, const float* d_registry, int N, int D, int k,
@@ -215,16 +426,35 @@ extern "C" int vdk_registry_topk(const float* d_queries, int B, const float* d_r
         require(k >= 1 && k <= kMaxK, "registry_topk: k must be in 1..64");
         require(k <= N, "registry_topk: k exceeds the registry size");
         require((size_t)N * D < (1ull << 31) && (size_t)B * D < (1ull << 31), "registry_topk: registry too large");
-        require(work_bytes >= workspace_bytes(B, N, k), "registry_topk: workspace too small");
-        const int nchunks = (N + kTR - 1) / kTR;
+        require(work_bytes >= workspace_bytes(B, N, k, kRows), "registry_topk: workspace too small");
+        const bool small = N <= kSmallN && work_bytes >= workspace_bytes(B, N, k, kRowsSmall);
+        const int rows = small ? kRowsSmall : kRows, lists = (N + rows - 1) / rows;
         double* cand_s = static_cast<double*>(d_work);
-        int* cand_i = reinterpret_cast<int*>(cand_s + (size_t)B * nchunks * k);
+        int* cand_i = reinterpret_cast<int*>(cand_s + (size_t)B * lists * k);
         hipStream_t s = static_cast<hipStream_t>(stream);
-        hipLaunchKernelGGL(registry_tile_kernel, dim3(nchunks, cdiv(B, kTQ)), dim3(256), 0, s, d_queries, B,
-                           d_registry, N, D, k, cand_s, cand_i);
-        VDK_HIP(hipGetLastError());
-        hipLaunchKernelGGL(registry_merge_kernel, dim3(B), dim3(256), 0, s, cand_s, cand_i, nchunks * k, k, d_idx,
-                           d_score);
+        // up to 16 queries one block of them per wave, two above (64 x 100000 x 192,
+        // k = 10, us: 8 waves of 2 x 2 blocks 79, 4 waves of 4 x 2 92, of 4 x 4
+        // 93; 1 query: 4 waves of 4 x 1 28)
+        if (small) {
+            if (B <= 16) launch_score_k<4, 1, 1, 4>(d_queries, B, d_registry, N, D, k, cand_s, cand_i, s);
+            else launch_score_k<4, 2, 1, 2>(d_queries, B, d_registry, N, D, k, cand_s, cand_i, s);
+        } else {
+            if (B <= 16) launch_score_k<4, 1, 4, 2>(d_queries, B, d_registry, N, D, k, cand_s, cand_i, s);
+            else launch_score_k<8, 2, 2, 1>(d_queries, B, d_registry, N, D, k, cand_s, cand_i, s);
+        }
+        const int n = lists * k;
+        if (n <= 256 * 2)
+            hipLaunchKernelGGL((registry_merge_kernel<256, 2>), dim3(B), dim3(256), 0, s, cand_s, cand_i, n, k, d_idx,
+                               d_score);
+        else if (n <= 1024 * 4)
+            hipLaunchKernelGGL((registry_merge_kernel<1024, 4>), dim3(B), dim3(1024), 0, s, cand_s, cand_i, n, k,
+                               d_idx, d_score);
+        else if (n <= 1024 * 16)
+            hipLaunchKernelGGL((registry_merge_kernel<1024, 16>), dim3(B), dim3(1024), 0, s, cand_s, cand_i, n, k,
+                               d_idx, d_score);
+        else
+            hipLaunchKernelGGL((registry_merge_kernel<1024, 0>), dim3(B), dim3(1024), 0, s, cand_s, cand_i, n, k, d_idx,
+                               d_score);
         VDK_HIP(hipGetLastError());
     });
 }
