@@ -1,0 +1,141 @@
+"""The GEMM kernel's tiles for small launches: same bits as the wide tiles.
+
+A layer with few output pixels runs on the smallest tile whose workgroups fit
+the chip in one round; the K order (taps, planes, 16-channel steps) is the same
+in every tile, so its result equals the LDS-DMA / register-staged tiles' bit
+for bit, and the default pick's.  Compared against f64 as well.
+"""
+import numpy as np
+import pytest
+
+import pyoracle as O
+from gpu_util import announce
+from vdamd import lib
+
+pytestmark = pytest.mark.gpu
+
+SMALL = list(range(92, 102))
+
+
+def run_tiles(d, dy, shape, tiles):
+    outs = {}
+    for t in tiles:
+        d.tile = t
+        if t >= 0 and not lib.lib().vdk_conv2d_tile_fits_ex(t, d):
+            continue
+        lib.check(lib.lib().vdk_conv2d_ex(d, None))
+        lib.check(lib.lib().vdk_synchronize())
+        outs[t] = dy.to_array(np.uint16, shape)
+    return outs
+
+
+# pixels around the 32 / 64 / 128 tile edges, outputs that no tile divides,
+# one and several K chunks, 1-D strides and taps, and a 2-D stride-2 3x3
+CASES = [
+    # B, H, W, IC, OC, KH, KW, stride, pad, residual
+    (1, 1, 1, 128, 32, 1, 1, 1, 0, False),
+    (1, 1, 31, 128, 40, 1, 1, 1, 0, True),
+    (1, 1, 159, 768, 768, 1, 1, 1, 0, True),
+    (3, 1, 53, 256, 200, 1, 1, 1, 0, False),
+    (2, 1, 129, 64, 72, 1, 1, 1, 0, True),
+    (5, 1, 259, 96, 136, 1, 5, 1, 0, False),
+    (1, 1, 639, 512, 512, 1, 3, 2, 0, False),
+    (2, 1, 600, 512, 128, 1, 2, 2, 0, False),
+    (1, 20, 75, 128, 256, 3, 3, 2, 1, False),
+    (1, 21, 33, 64, 128, 3, 3, 2, 1, False),
+    (1, 40, 37, 32, 32, 3, 3, 2, 1, False),
+]
+
+
+@pytest.mark.parametrize("case", CASES)
+def test_small_tiles_bitwise(case):
+    B, H, W, IC, OC, KH, KW, stride, pad, res = case
+    rng = np.random.default_rng(sum(case[:9]))
+    announce(f"small launch {case}")
+    x = rng.standard_normal((B, H, W, IC)).astype(np.float16)
+    w = (rng.standard_normal((OC, KH, KW, IC)) * np.sqrt(2.0 / (KH * KW * IC))).astype(np.float16)
+    b = rng.uniform(-0.5, 0.5, OC).astype(np.float32)
+    sh = stride if KH > 1 else 1
+    Ho = (H + 2 * (pad if KH > 1 else 0) - KH) // sh + 1
+    Wo = (W + 2 * pad - KW) // stride + 1
+    keep = [lib.DeviceBuffer.from_array(v) for v in (x, w, b)]
+    d = lib.ConvDesc()
+    d.x, d.batch, d.H, d.W, d.IC = keep[0].ptr, B, H, W, IC
+    d.w, d.OC, d.KH, d.KW = keep[1].ptr, OC, KH, KW
+    d.stride_h, d.stride_w, d.pad_h, d.pad_w = sh, stride, pad if KH > 1 else 0, pad
+    d.dil_h = d.dil_w = 1
+    d.bias, d.act = keep[2].ptr, lib.ACT_RELU
+    if res:
+        r = rng.standard_normal((B, Ho, Wo, OC)).astype(np.float16)
+        keep.append(lib.DeviceBuffer.from_array(r))
+        d.residual = keep[3].ptr
+    dy = lib.DeviceBuffer(B * Ho * Wo * OC * 2)
+    d.y = dy.ptr
+    ref_tile = 18 if IC % 64 == 0 else 39      # LDS-DMA tiles with 64- / 32-channel chunks
+    outs = run_tiles(d, dy, (B, Ho, Wo, OC), [ref_tile, -1] + SMALL)
+    assert sum(t >= 92 for t in outs) >= 2, sorted(outs)
+    for t, o in outs.items():
+        assert np.array_equal(o, outs[ref_tile]), f"tile {t}"
+    # f16 products are exact in f32; K f32 additions (half an ulp each) and the f16 store
+    xp = np.pad(x.astype(np.float64), ((0, 0), (d.pad_h, d.pad_h), (d.pad_w, d.pad_w), (0, 0)))
+    want = np.zeros((B, Ho, Wo, OC))
+    mag = np.zeros((B, Ho, Wo, OC))
+    for kh in range(KH):
+        for kw in range(KW):
+            xs = xp[:, kh:kh + (Ho - 1) * sh + 1:sh, kw:kw + (Wo - 1) * stride + 1:stride]
+            want += xs @ w[:, kh, kw].astype(np.float64).T
+            mag += np.abs(xs) @ np.abs(w[:, kh, kw].astype(np.float64)).T
+    want += b
+    mag += np.abs(b)
+    if res:
+        want += r
+        mag += np.abs(r)
+    want = np.maximum(want, 0)
+    got = outs[-1].view(np.float16).astype(np.float64)
+    K = KH * KW * IC
+    assert (np.abs(got - want) <= K * 2.0 ** -24 * mag + 2.0 ** -11 * np.abs(want) + 2.0 ** -24).all()
+
+
+@pytest.mark.parametrize("split,KH,stride,IC,OC", [(1, 1, 1, 128, 64), (1, 1, 1, 64, 32), (2, 3, 2, 64, 128),
+                                                   (1, 3, 2, 128, 72), (2, 1, 1, 32, 64)])
+def test_small_tiles_split_bitwise(split, KH, stride, IC, OC):
+    """Split-f16 inputs (two or three plane terms per tap), 1x1 and the stride-2
+    3x3 downsamples, against the LDS-DMA tile with the same chunk width."""
+    rng = np.random.default_rng(split + KH + IC + OC)
+    B, H, W = 2, 10, 91
+    announce(f"small launch split {split} K {KH} s {stride} {IC}->{OC}")
+    x = rng.standard_normal((B, H, W, IC)).astype(np.float32)
+    w = (rng.standard_normal((OC, KH, KH, IC)) * np.sqrt(2.0 / (KH * KH * IC))).astype(np.float32)
+    if split == 2:
+        w = w.astype(np.float16).astype(np.float32)
+
+    def halves(v):
+        hi = v.astype(np.float16)
+        return hi, (v - hi.astype(np.float32)).astype(np.float16)
+
+    wh, wl = halves(w)
+    pack = np.concatenate([wh, wh] if split == 2 else [wh, wh, wl], axis=3)
+    bias = rng.uniform(-0.5, 0.5, OC).astype(np.float32)
+    keep = [lib.DeviceBuffer.from_array(np.ascontiguousarray(v)) for v in
+            (np.concatenate(halves(x), axis=3), pack, bias)]
+    pad = KH // 2
+    Ho, Wo = (H + 2 * pad - KH) // stride + 1, (W + 2 * pad - KH) // stride + 1
+    d = lib.ConvDesc()
+    d.x, d.batch, d.H, d.W, d.IC, d.x_stride, d.x_lo = keep[0].ptr, B, H, W, IC, 2 * IC, IC
+    d.w, d.OC, d.KH, d.KW = keep[1].ptr, OC, KH, KH
+    d.stride_h = d.stride_w = stride
+    d.pad_h = d.pad_w = pad
+    d.dil_h = d.dil_w = 1
+    d.bias, d.act, d.split = keep[2].ptr, lib.ACT_NONE, split
+    dy = lib.DeviceBuffer(B * Ho * Wo * 2 * OC * 2)
+    d.y, d.y_stride, d.y_lo = dy.ptr, 2 * OC, OC
+    ref_tile = 18 if IC % 64 == 0 else 39
+    outs = run_tiles(d, dy, (B, Ho, Wo, 2 * OC), [ref_tile, -1] + SMALL)
+    assert sum(t >= 92 for t in outs) >= 2, sorted(outs)
+    for t, o in outs.items():
+        assert np.array_equal(o, outs[ref_tile]), f"tile {t}"
+    o = outs[-1].view(np.float16).astype(np.float64)
+    got = o[..., :OC] + o[..., OC:]
+    want = np.stack([O.conv2d_g(x[c].transpose(2, 0, 1), np.ascontiguousarray(w.transpose(0, 3, 1, 2)), sh=stride,
+                                sw=stride, ph=pad, pw=pad, bias=bias, f64=True) for c in range(B)])
+    assert np.abs(got.transpose(0, 3, 1, 2) - want).max() <= 2e-6 * np.abs(want).max()

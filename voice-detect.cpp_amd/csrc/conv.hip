@@ -260,11 +260,18 @@ __device__ __forceinline__ void finish_staged(const ConvArgs& a, const float* sT
 // run on one XCD (xcd_swizzle), and the output-channel tiles of a pixel tile
 // are consecutive in it, so the workgroups that read the same input pixels
 // run at about the same time under the same L2: the input leaves HBM once,
-// not once per output-channel tile.
-__device__ __forceinline__ void tile_ids(int& ptile, int& otile) {
+// not once per output-channel tile.  A layer with more weights than input
+// pixels (a transformer's linears on one short clip) runs the other way
+// round, the pixel tiles of an output-channel tile consecutive.
+__device__ __forceinline__ void tile_ids(const ConvArgs& a, int& ptile, int& otile) {
     const int lid = xcd_swizzle(blockIdx.x + gridDim.x * blockIdx.y, gridDim.x * gridDim.y);
-    ptile = lid / gridDim.y;
-    otile = lid - ptile * gridDim.y;
+    if (a.OC * a.KH * a.KW > a.npix_in) {
+        otile = lid / gridDim.x;
+        ptile = lid - otile * gridDim.x;
+    } else {
+        ptile = lid / gridDim.y;
+        otile = lid - ptile * gridDim.y;
+    }
 }
 
 // Staged epilogue of an implicit-GEMM tile (BM channels x BN consecutive
@@ -373,7 +380,7 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64) void conv_igemm_kernel(
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int wm = wave % NWM, wn = wave / NWM;
     int ptile, otile;
-    tile_ids(ptile, otile);
+    tile_ids(a, ptile, otile);
     const int p0 = ptile * BN;
     const int oc0 = otile * BM;
     const int HoWo = a.Ho * a.Wo;
@@ -590,8 +597,9 @@ __device__ __forceinline__ int swz(int r, int c) {
     // cycle; an MFMA operand read has 16 lanes on 16 consecutive rows and one
     // chunk column, so the key makes those 16 (row, chunk) pairs hit distinct
     // 16-byte bank groups.  KC=64: 128-byte rows, key = (r/2) % 8.
-    // KC=32: 64-byte rows, key = (r/4) % 4.
-    if constexpr (KC == 64) return c ^ ((r >> 1) & 7);
+    // KC=32: 64-byte rows, key = (r/4) % 4.  KC=128: 256-byte rows, key = r % 16.
+    if constexpr (KC == 128) return c ^ (r & 15);
+    else if constexpr (KC == 64) return c ^ ((r >> 1) & 7);
     else return c ^ ((r >> 2) & 3);
 }
 
@@ -620,7 +628,7 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64) void conv_dma_kernel(Co
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wm = wave % NWM, wn = wave / NWM;
     int ptile, otile;
-    tile_ids(ptile, otile);
+    tile_ids(a, ptile, otile);
     const int p0 = ptile * BN;
     const int oc0 = otile * BM;
     const int HoWo = a.Ho * a.Wo;
@@ -932,7 +940,7 @@ struct GemmWs {
     static constexpr int CPR = KC / 8, RB = KC * 2;
     static constexpr int NINS = (BM + BN) * CPR / 64, IPP = NINS / NP;   // DMA instructions per chunk / producer
     static constexpr int STAGE = NINS * 1024;
-    static_assert(KC == 32 || KC == 64, "KC");
+    static_assert(KC == 32 || KC == 64 || KC == 128, "KC");
     static_assert(NINS % NP == 0 && (BM * CPR) % 64 == 0, "whole DMA instructions, split evenly over the producers");
     static_assert(NST >= 2 && NST * STAGE <= 163840, "the ring fits the 160 KB of LDS");
     static_assert(TM >= 1 && TN >= 1, "wave tiles of whole 32 x 32 blocks");
@@ -946,7 +954,7 @@ struct GemmWs {
 template <int BM, int BN, int WMG, int WNG, int KC, int NST, int NP, bool PRO = false, bool SEGS = false>
 __global__ __launch_bounds__((WMG * WNG + NP) * 64) void gemm_ws_kernel(ConvArgs a) {
     using G = GemmWs<BM, BN, WMG, WNG, KC, NST, NP>;
-    constexpr int TM = G::TM, TN = G::TN, RB = G::RB, CPR = G::CPR;
+    constexpr int TM = G::TM, TN = G::TN, RB = G::RB;
     constexpr int SMEM_E = G::WN * (BM + 4) * 4;   // one epilogue pass of a wave's pixel columns
     constexpr int SMEM = NST * G::STAGE > SMEM_E ? NST * G::STAGE : SMEM_E;
     constexpr int PRO_MAX = 1024;                  // input channels with a staged prologue
@@ -962,7 +970,7 @@ __global__ __launch_bounds__((WMG * WNG + NP) * 64) void gemm_ws_kernel(ConvArgs
         __syncthreads();
     }
     int ptile, otile;
-    tile_ids(ptile, otile);
+    tile_ids(a, ptile, otile);
     const int p0 = ptile * BN, oc0 = otile * BM;
     // chunks per tap (split-f16: over the [hi | lo | hi] plane terms)
     const int ncpt = (a.split ? (a.split == 2 ? 2 : 3) * a.IC : a.IC) / KC;
@@ -2722,7 +2730,9 @@ struct TileCfg {
 // same order as its 5-row bands, so the same bits, on 5x the workgroups), 80
 // the register-staged 64x64 tile with 64-channel chunks, 81-84 the 1x1 GEMM
 // kernel with producer / compute waves, 85-88 narrow tiles of that kernel
-// with the prologue / segment-sum variants.
+// with the prologue / segment-sum variants, 92-101 the GEMM kernel's tiles for
+// launches that leave the chip partly idle (deep rings of 64- and 128-channel
+// chunks; pick_small_tile).
 
 // Tile table.  Wave tiles are WM x WN = (bm / waves_m) x (bn / waves_n) with
 // 4 waves per workgroup; entries are selected per layer by pick_tile().
@@ -2819,6 +2829,16 @@ const TileCfg kTiles[] = {
     {128, 256, 64, launch_gemm_ws<128, 256, 2, 4, 64, 3, 4, true>, false, 0, 0, 0, true, true},   // 89: wide, + prologue
     {256, 128, 64, launch_gemm_ws<256, 128, 4, 2, 64, 3, 4, true>, false, 0, 0, 0, true, true},   // 90
     {128, 384, 32, launch_gemm_ws<128, 384, 2, 4, 32, 4, 4, true>, false, 0, 0, 0, true, true},   // 91
+    {32, 32, 128, launch_gemm_ws<32, 32, 1, 1, 128, 4, 4, true>, false, 0, 0, 0, true, true},     // 92: small launches
+    {32, 32, 64, launch_gemm_ws<32, 32, 1, 1, 64, 8, 2, true>, false, 0, 0, 0, true, true},       // 93
+    {32, 32, 32, launch_gemm_ws<32, 32, 1, 1, 32, 16, 2, true>, false, 0, 0, 0, true, true},      // 94
+    {64, 32, 128, launch_gemm_ws<64, 32, 2, 1, 128, 3, 4>, false, 0, 0, 0, true},                 // 95
+    {64, 64, 128, launch_gemm_ws<64, 64, 2, 2, 128, 4, 4, true>, false, 0, 0, 0, true, true},     // 96
+    {64, 64, 128, launch_gemm_ws<64, 64, 2, 2, 128, 2, 4>, false, 0, 0, 0, true},                 // 97
+    {64, 64, 64, launch_gemm_ws<64, 64, 2, 2, 64, 4, 4, true>, false, 0, 0, 0, true, true},       // 98
+    {32, 64, 32, launch_gemm_ws<32, 64, 1, 2, 32, 8, 2>, false, 0, 0, 0, true},                   // 99
+    {128, 64, 128, launch_gemm_ws<128, 64, 2, 2, 128, 3, 4>, false, 0, 0, 0, true},               // 100
+    {128, 128, 64, launch_gemm_ws<128, 128, 4, 2, 64, 4, 4>, false, 0, 0, 0, true},               // 101
 };
 constexpr int kNumTiles = (int)(sizeof(kTiles) / sizeof(kTiles[0]));
 
@@ -2826,6 +2846,7 @@ bool is_s1_3x3(const ConvArgs& a) {
     return a.KH == 3 && a.KW == 3 && a.sh == 1 && a.sw == 1 && a.ph == 1 && a.pw == 1 && a.dh == 1 && a.dw == 1;
 }
 
+constexpr int kFirstSmall = 92;   // the GEMM kernel's small-launch tiles
 constexpr int kFirstDma = 14;   // then the halo tiles from 26, 8-wave DMA tiles from 33
 
 // The register-weight kernels take the plain epilogue only: bias, residual,
@@ -2872,17 +2893,17 @@ bool tile_fits(const TileCfg& t, const ConvArgs& a) {
     // take the register-staged kernel
     if (a.KH * a.KW > 32 && a.KH != 1 && !igemm_tile(idx)) return false;
     if (t.sp_ic) return a.IC == t.sp_ic && a.OC == t.bm && split_epilogue(a);
-    // the GEMM kernel: split-f16 inputs for 1x1 convs only (the plane terms
-    // are consecutive chunks of one tap), channel groups whole per chunk
-    // (prologue / segment sums: the EXT tiles, 1x1 without padding, up to
+    // the GEMM kernel: channel groups whole per chunk, split-f16 plane terms
+    // as consecutive chunks of a tap (2-D taps: the small-launch tiles; prologue / segment sums: the EXT tiles, 1x1 without padding, up to
     // 1024 input channels, pixel tiles at most seg_len wide)
     if (t.gemm) {
         const bool one = a.KH * a.KW == 1 && a.ph == 0 && a.pw == 0;
         if ((a.in_scale || a.segsum) && !(t.gemm_ext && one && !a.split)) return false;
         if (a.in_scale && a.IC > 1024) return false;
         if (a.segsum && t.bn > a.seg_len) return false;
-        return (!a.split || a.KH * a.KW == 1) && !a.reflect && !a.wq && t.kc % (1 << a.xgl) == 0 &&
-               a.IC % t.kc == 0 && a.xs % 8 == 0 && (!a.split || a.x_lo % 8 == 0);
+        if (a.split && a.KH * a.KW != 1 && idx < kFirstSmall) return false;
+        return !a.reflect && !a.wq && t.kc % (1 << a.xgl) == 0 && a.IC % t.kc == 0 && a.xs % 8 == 0 &&
+               (!a.split || a.x_lo % 8 == 0);
     }
     // 16-channel group strides: the LDS-DMA kernel's offsets and the shared store
     if ((a.xgs != (1 << a.xgl) || a.ygs != (1 << a.ygl)) && (igemm_tile(idx) || t.halo || t.rw_ic || t.band_w))
@@ -2905,6 +2926,54 @@ int tile_override() {
     return v;
 }
 
+// Layers whose output a 128 x 128 (or wider) tiling spreads over fewer
+// workgroups than there are CUs: the time is then one workgroup's own walk
+// along K (a chunk's load latency and barrier per step), not the chip's MFMA
+// rate, so the tile is the smallest whose workgroups still fit the 256 CUs in
+// one round (64 KB rings: two per CU), with the longest K chunk the channels
+// allow.  Every tile sums K in the same order (taps, planes, 16-channel
+// steps), so the choice changes no bit and a clip's result does not depend on
+// its batch.  From a sweep of every fitting tile over the layers of all four
+// embedders and wav2vec2-base at 17 batch x length pairs, inputs flushed to
+// HBM, single launches (us, of which about 4.5 are the launch itself), before
+// -> now: 159 pixels, 768 -> 768 22.5 -> 8.7 and 3072 -> 768 45 -> 14.5 (92);
+// 159 pixels, 768 -> 3072 27 -> 9.9 (95); 1279 pixels, 3 x 512 -> 512 30 ->
+// 13.0 (96); 1295 pixels, 1024 -> 1024 36 -> 14.3 (97) and 3072 -> 1536 43 ->
+// 26.5 (100); 4768 pixels, 3072 -> 768 54 -> 41 (101); split-f16, 1000 pixels,
+// 1024 -> 128 41 -> 16 (92) and 29120 pixels, 256 -> 32 28 -> 19 (98).  Past
+// the limits below the wide tiles' fewer operand reads win.
+int pick_small_tile(const ConvArgs& a) {
+    if (is_s1_3x3(a) || a.KH * a.KW > 32) return -1;   // their own kernels (below)
+    const auto wgs = [&](int bm, int bn) { return (long)cdiv(a.OC, bm) * cdiv(a.npix, bn); };
+    const bool c64 = a.IC % 64 == 0, c128 = a.IC % 128 == 0;
+    const int K = a.KH * a.KW * a.IC * (a.split ? (a.split == 2 ? 2 : 3) : 1);
+    const long w32 = wgs(32, 32), w64 = wgs(64, 64), w128 = wgs(128, 128);
+    int t = -1;
+    if (w32 <= 256) t = c128 ? 92 : (c64 ? 93 : 94);
+    else if (a.in_scale || a.segsum) {   // CAM++'s linear1 / transits
+        if (c128 && w64 <= 256 && a.OC > 128) t = 96;
+        else if (w32 <= 512) t = c128 ? 92 : (c64 ? 93 : 94);
+        else if (c64 && w64 <= 256) t = c128 ? 96 : 98;
+    } else if (!c64 || a.OC % 64 != 0) {
+        // narrow outputs and 32-channel chunks
+        if (c64 && a.split && w64 <= 1000) t = 98;
+        else if (wgs(32, 64) <= 700) t = 99;
+    } else if (c128 && wgs(64, 32) <= 256) t = 95;
+    else if (c128 && w64 <= 256) t = 96;
+    else if (!c128 && wgs(64, 32) <= 256) t = 93;
+    else if (w128 >= 140 && w128 <= 256 && K >= 512) t = 101;
+    else if (c128 && K >= 1536 && wgs(128, 64) <= 256) t = 100;
+    else if (c128 && K >= 512 && w64 <= 640 && !a.split) t = 97;
+    else if (w64 <= (a.split ? 1000 : 640)) t = 98;
+    return t >= 0 && tile_fits(kTiles[t], a) ? t : -1;
+}
+
+// Rounds of workgroups over 256 CUs x a tile's area: what a GEMM tile costs
+// when the launch is a few rounds long.
+long round_cost(const ConvArgs& a, int t) {
+    return cdiv(cdiv(a.npix, kTiles[t].bn) * cdiv(a.OC, kTiles[t].bm), 256) * (long)kTiles[t].bm * kTiles[t].bn;
+}
+
 // Per-layer-class defaults, from a sweep of every ResNet34 conv shape at
 // batch 64 on MI355X (64-channel 3x3 stride-1 layers with the plain
 // epilogue: the register-weight kernel; 128-channel ones whose map is 39-76
@@ -2918,6 +2987,8 @@ int tile_override() {
 int pick_tile(const ConvArgs& a) {
     const int o = tile_override();
     if (o >= 0 && o < kNumTiles && tile_fits(kTiles[o], a)) return o;
+    const int small = pick_small_tile(a);
+    if (small >= 0) return small;
     const int bm = a.OC % 128 == 0 ? 128 : (a.OC % 64 == 0 ? 64 : 32);
     if (a.in_scale) {   // register-staged tiles for a few ten thousand pixels (CAM++'s
         // linear1: the LDS-DMA tiles, faster in isolation, measured slower in the model):
@@ -2974,6 +3045,14 @@ int pick_tile(const ConvArgs& a) {
             // qkv 768 -> 2304 on the 8-wave LDS-DMA tile, 60.9 -> 55.8 us; ECAPA's
             // 1024 -> 1024 TDNNs the same, 88.5 -> 84.6 us)
             if (a.npix < 16384 && a.OC == 2304 && a.IC == 768 && tile_fits(kTiles[40], a)) return 40;
+            // 5960 / 11920 pixels: 1024 -> 1024 40 -> 26 us on 256 x 128, 3072 ->
+            // 1536 94 -> 68 / 151 -> 134 us on 128 x 288, where the narrower
+            // tile's rounds cover the map with less left over
+            if (a.npix < 16384 && a.OC == 1024 && tile_fits(kTiles[83], a) && round_cost(a, 83) < round_cost(a, 82))
+                return 83;
+            if (a.npix < 16384 && a.IC >= 2048 && a.OC % 256 == 0 && tile_fits(kTiles[84], a) &&
+                round_cost(a, 84) < round_cost(a, 83))
+                return 84;
             if (a.npix < 16384 && (a.OC == 1024 || a.OC == 2304) && tile_fits(kTiles[82], a)) return 82;
             if (a.npix >= 16384 && a.OC == 1024 && a.IC == 1024 && tile_fits(kTiles[40], a)) return 40;
             if (a.IC >= 2048) return a.OC % 256 == 0 ? 83 : 81;
@@ -2987,11 +3066,18 @@ int pick_tile(const ConvArgs& a) {
         if (a.sw == 2 && a.KW <= 3 && a.IC == 512 && a.OC == 512 && tile_fits(kTiles[83], a)) {
             if (a.npix >= 65536 || a.npix < 16384) return 83;
             if (a.KW == 2 && a.npix >= 16384 && a.npix < 32768 && tile_fits(kTiles[82], a)) return 82;
+            // 3-tap ones between: the tile whose rounds cover the map best (19k
+            // pixels 62 -> 56 us on 128 x 384, 29k 87 -> 67, 58k 150 -> 132 on 256 x 256)
+            if (a.KW == 3) return round_cost(a, 82) < round_cost(a, 38) ? 82 : 38;
         }
         // ECAPA's block0 (k = 5 over the 96 padded mel channels, 1024 out) on
         // the 128x256 8-wave tile (52.9 against 69.2 us at batch 64 x 4 s),
         // and asp.tdnn's 1536 -> 128 GEMM on the 128x64 tile (398 workgroups
         // instead of 199: 25.0 against 38.7 us)
+        // (under 8192 pixels the 128x64 one: 3357 pixels 25 -> 17, 5960 26 -> 22 us)
+        if (a.KW == 5 && a.IC % 32 == 0 && a.OC >= 512 && a.OC % 128 == 0 && a.npix < 8192 &&
+            tile_fits(kTiles[48], a))
+            return 48;
         if (a.KW == 5 && a.IC % 32 == 0 && a.OC >= 512 && a.OC % 128 == 0 && tile_fits(kTiles[36], a)) return 36;
         // CAM++'s TDNN (k = 5, stride 2, 320 -> 128) on the 128x32 tile (in-model: 30.2 -> 19.2 us)
         if (a.KW == 5 && a.sw == 2 && a.OC == 128 && a.IC % 64 == 0 && tile_fits(kTiles[52], a)) return 52;
