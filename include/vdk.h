@@ -331,6 +331,12 @@ typedef struct {
 } vdk_res2_weights;
 int vdk_res2_block(void* d_buf, int stride, int batch, int T, int G, int scale, int dil,
                    const vdk_res2_weights* w, void* stream);
+/* The same block into a buffer of its own: y [B][T][y_stride] = [y_1 | x_0 |
+ * y_2 .. y_{scale-1}] in slots 0 .. scale - 1, x left as it was; x and y must
+ * not overlap, y 16-byte aligned.  (In place, clips of several time tiles go
+ * through a side buffer, allocated and freed on the stream.) */
+int vdk_res2_block_out(const void* d_x, int stride, int batch, int T, int G, int scale, int dil,
+                       const vdk_res2_weights* w, void* d_y, int y_stride, void* stream);
 /* out [B][T+2*pad][G] = reflect_pad(a (+ b)) over time: the Res2Net group
  * input x_i + y_{i-1} of src/encoder.cpp:174-200 padded for its dilated conv.
  * d_b may be NULL. */

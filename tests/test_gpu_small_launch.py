@@ -139,3 +139,46 @@ def test_small_tiles_split_bitwise(split, KH, stride, IC, OC):
     want = np.stack([O.conv2d_g(x[c].transpose(2, 0, 1), np.ascontiguousarray(w.transpose(0, 3, 1, 2)), sh=stride,
                                 sw=stride, ph=pad, pw=pad, bias=bias, f64=True) for c in range(B)])
     assert np.abs(got.transpose(0, 3, 1, 2) - want).max() <= 2e-6 * np.abs(want).max()
+
+
+@pytest.mark.parametrize("batch,T,dil,scale", [(1, 5, 4, 8), (1, 32, 2, 8), (1, 95, 2, 8), (5, 259, 4, 8),
+                                              (2, 333, 3, 4), (40, 301, 4, 8), (1, 1198, 3, 8)])
+def test_res2_block_out_tiles(batch, T, dil, scale):
+    """One ECAPA Res2Net block over many short tiles: every split into time
+    tiles gives the bits of the block run in place, one clip at a time (few
+    tiles or one), and x stays as it was."""
+    rng = np.random.default_rng(batch + T + dil + scale)
+    G, L = 128, lib.lib()
+    S = (scale + 1) * G
+    announce(f"res2 block out B={batch} T={T} dil={dil} scale={scale}")
+    x = rng.standard_normal((batch, T, S), dtype=np.float32).astype(np.float16)
+    keep, rw = [], lib.Res2Weights()
+    for j in range(scale - 1):
+        w = (rng.standard_normal((G, 3, G)) * np.sqrt(2.0 / (3 * G))).astype(np.float16)
+        vec = [rng.uniform(lo, hi, G).astype(np.float32) for lo, hi in ((-0.1, 0.1), (0.5, 1.0), (-0.2, 0.2))]
+        bufs = [lib.DeviceBuffer.from_array(v) for v in [w] + vec]
+        keep += bufs
+        rw.w[j], rw.bias[j], rw.scale[j], rw.shift[j] = (b.ptr for b in bufs)
+    dx = lib.DeviceBuffer.from_array(x)
+    ys = scale * G + 64
+    dy = lib.DeviceBuffer.from_array(np.zeros((batch, T, ys), np.float16))
+    lib.check(L.vdk_res2_block_out(dx.ptr, S, batch, T, G, scale, dil, rw, dy.ptr, ys, None))
+    lib.check(L.vdk_synchronize())
+    got = dy.to_array(np.uint16, (batch, T, ys))
+    assert np.array_equal(dx.to_array(np.uint16, (batch, T, S)), x.view(np.uint16))
+    assert not got[:, :, scale * G:].any()
+    for c in sorted({0, batch // 2, batch - 1}):
+        one = lib.DeviceBuffer.from_array(x[c:c + 1])
+        lib.check(L.vdk_res2_block(one.ptr, S, 1, T, G, scale, dil, rw, None))
+        lib.check(L.vdk_synchronize())
+        assert np.array_equal(got[c, :, :scale * G], one.to_array(np.uint16, (1, T, S))[0, :, :scale * G])
+    # the first group against f64 (f32 sums of 3 * 128 products, then the f16 store)
+    c = batch - 1
+    w, b, sc, sh = (k.to_array(t, s).astype(np.float64) for k, t, s in
+                    zip(keep[:4], (np.float16,) + (np.float32,) * 3, ((G, 3, G), (G,), (G,), (G,))))
+    xp = np.pad(x[c, :, 2 * G:3 * G].astype(np.float64), ((dil, dil), (0, 0)), mode="reflect")
+    taps = [xp[k * dil:k * dil + T] for k in range(3)]
+    want = np.maximum(sum(v @ w[:, k].T for k, v in enumerate(taps)) + b, 0) * sc + sh
+    mag = (sum(np.abs(v) @ np.abs(w[:, k]).T for k, v in enumerate(taps)) + np.abs(b)) * sc + np.abs(sh)
+    err = np.abs(got[c, :, :G].view(np.float16).astype(np.float64) - want)
+    assert (err <= 3 * G * 2.0 ** -24 * mag + 2.0 ** -11 * np.abs(want) + 2.0 ** -24).all()

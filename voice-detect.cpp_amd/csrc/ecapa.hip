@@ -15,7 +15,9 @@
 //    (src/encoder.cpp:262-295): global mean/std (clamp 1e-12), softmax over
 //    time per channel, weighted mean/std.
 // Sums are accumulated in f64.
+#include <algorithm>
 #include <cmath>
+#include <type_traits>
 
 #include "common.hpp"
 #include "vdk.h"
@@ -467,24 +469,35 @@ bool al16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
 // clip; D the dilation), so the tile's halo shrinks by D per group and no
 // other workgroup's result is ever read.  Its input in_j (x_1, then
 // f16(v_{j-1} + x_j) with v the previous group's f32 output) lives in one of
-// two LDS buffers and the next one is written by the group's epilogue; the
-// weights stream through LDS one tap (128 x 128 f16) at a time in a
-// two-stage DMA ring; y_j = f16(v_j) leaves for its slot of the Res2Net
-// buffer for the tile's own frames.  Per group the conv runs exactly like the
-// one-group DMA conv (taps outer, 16-channel k-steps inner, accumulators from
-// zero, bias -> ReLU -> BN scale, shift, the same reflect rule), so the
-// results are the same bits as the chain of single-group launches.
-// Layout of the buffer (stride S per frame): x_m in slot m + 1 (m = 0 ..
-// scale - 1, slots of G = 128 channels), y_1 written to slot 0, y_j (j >= 2)
-// to slot j.
+// two LDS buffers: x_{j+1} is DMA'd into the other one while group j computes,
+// and the group's epilogue adds v to it in place.  The weights stream through
+// LDS one tap (128 x 128 f16) at a time in an NST-stage DMA ring, and
+// y_j = f16(v_j) leaves for its slot of the output for the tile's own frames.
+// Per group the conv runs exactly like the one-group DMA conv (taps outer,
+// 16-channel k-steps inner, accumulators from zero, bias -> ReLU -> BN scale,
+// shift, the same reflect rule), so the results are the same bits as the
+// chain of single-group launches.
+//
+// The input (stride S per frame) holds x_m in slot m + 1 (m = 0 .. scale - 1,
+// slots of G = 128 channels); the output (stride ys) y_1 in slot 0, y_j in
+// slot j and, with copy0, x_0 in slot 1.  Other tiles read x on their halos
+// whenever they come to run, so the output must not overlap the input when a
+// clip has several tiles.
+//
+// Bound by the LDS reads of its 21 dependent tap steps.  With a branch per
+// frame block between the operand reads every MFMA waited out an LDS round
+// trip (2.4 us a step whatever the tile's length: 50 us alone at 5 x 259
+// frames, D = 3); with a tap's reads issued together the wide tiles take 43
+// us.  Small launches take 96-row buffers, which leave LDS for a third weight
+// stage, and as many tiles of at least 32 frames as the chip has CUs: 35 us.
 // ---------------------------------------------------------------------------
 constexpr int kR2G = 128;          // channels per group
-constexpr int kR2Rows = 160;       // frames an input buffer holds (t1 - t0 + 2 L D <= 160)
 constexpr int kR2MaxL = 7;
 
 struct Res2Args {
-    half_t* t1;                    // [B][T][S]
-    int S, T, D, L, Tt, nt;
+    const half_t* x;               // [B][T][S]
+    half_t* y;                     // [B][T][ys]
+    int S, ys, T, D, L, Tt, nt, copy0;
     const half_t* w[kR2MaxL];      // [G][3][G] per group
     const float* bias[kR2MaxL];
     const float* scale[kR2MaxL];
@@ -501,9 +514,13 @@ __device__ __forceinline__ int r2_refl(int s, int T) {
 // distinct 16-byte bank groups)
 __device__ __forceinline__ int r2_off(int r, int c) { return r * 256 + ((c ^ (r & 15)) << 4); }
 
+// ROWS: frames an input buffer holds (t1 - t0 + 2 L D <= ROWS)
+template <int ROWS, int NST>
 __global__ __launch_bounds__(512) void res2_block_kernel(Res2Args a) {
-    __shared__ __attribute__((aligned(1024))) uint8_t s_in[2][kR2Rows * 256];
-    __shared__ __attribute__((aligned(1024))) uint8_t s_w[2][kR2G * 256];
+    static_assert(ROWS % 32 == 0 && (NST == 2 || NST == 3), "whole DMA rounds; x lands with the group's last tap");
+    constexpr int NB = (ROWS / 32 + 1) / 2;    // 32-frame blocks per wave
+    __shared__ __attribute__((aligned(1024))) uint8_t s_in[2][ROWS * 256];
+    __shared__ __attribute__((aligned(1024))) uint8_t s_w[NST][kR2G * 256];
     __shared__ float s_ep[kR2MaxL][3][kR2G];   // bias, scale, shift
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -514,13 +531,10 @@ __global__ __launch_bounds__(512) void res2_block_kernel(Res2Args a) {
     auto lo = [&](int j) { const int v = t0 - (L - j) * D; return v > 0 ? v : 0; };
     auto hi = [&](int j) { const int v = t1 + (L - j) * D; return v < T ? v : T; };
     const int base = lo(0);
-    half_t* const clip = a.t1 + (size_t)b * T * S;
+    const half_t* const clip = a.x + (size_t)b * T * S;
+    half_t* const yclip = a.y + (size_t)b * T * a.ys;
+    const int4v xr = dma_rsrc(clip + (size_t)base * S, (uint32_t)((T - base < ROWS ? T - base : ROWS) * S * 2));
 
-    for (int i = tid; i < L * 3 * kR2G; i += 512) {
-        const int j = i / (3 * kR2G), r = i - j * 3 * kR2G, q = r / kR2G, c = r - q * kR2G;
-        const float* src = q == 0 ? a.bias[j] : (q == 1 ? a.scale[j] : a.shift[j]);
-        s_ep[j][q][c] = src ? src[c] : (q == 1 ? 1.0f : 0.0f);
-    }
     // weights of tap k of group j: 2048 16-byte slots, 4 DMA instructions per wave
     auto issue_w = [&](int c) {
         const int j = c / 3, k = c - j * 3;
@@ -528,34 +542,54 @@ __global__ __launch_bounds__(512) void res2_block_kernel(Res2Args a) {
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             const int ins = wave * 4 + i, s = ins * 64 + lane, r = s >> 4, pc = s & 15, lc = pc ^ (r & 15);
-            dma16(s_w[c & 1] + ins * 1024, rs, (uint32_t)(((r * 3 + k) * kR2G + lc * 8) * 2));
+            dma16(s_w[c % NST] + ins * 1024, rs, (uint32_t)(((r * 3 + k) * kR2G + lc * 8) * 2));
         }
     };
-    issue_w(0);
-    // in_1 = x_1 (slot 2) on R_0
-    {
-        const int n = (hi(0) - base) * 16;
-        for (int i = tid; i < n; i += 512) {
-            const int r = i >> 4, c = i & 15;
-            *reinterpret_cast<half8*>(s_in[0] + r2_off(r, c)) =
-                *reinterpret_cast<const half8*>(clip + (size_t)(base + r) * S + 2 * kR2G + c * 8);
+    // frames [f0, f1) of input slot `slot` into rows f - base of dst (whole
+    // groups of 4 rows, 4 per instruction); returns this wave's instructions
+    auto issue_x = [&](uint8_t* dst, int slot, int f0, int f1) {
+        int n = 0;
+#pragma unroll
+        for (int i = 0; i < ROWS / 32; ++i) {
+            const int ins = wave + 8 * i;
+            if (ins * 4 + 4 <= f0 - base || ins * 4 >= f1 - base) continue;
+            const int s = ins * 64 + lane, r = s >> 4, lc = (s & 15) ^ (r & 15);
+            dma16(dst + ins * 1024, xr, base + r < T ? (uint32_t)((r * S + slot * kR2G + lc * 8) * 2) : kOOB);
+            ++n;
+        }
+        return n;
+    };
+    issue_x(s_in[0], 2, base, hi(0));   // in_1 = x_1 on R_0
+#pragma unroll
+    for (int c = 0; c < NST - 1; ++c)
+        if (c < 3 * L) issue_w(c);
+    for (int i = tid; i < L * 3 * kR2G; i += 512) {
+        const int j = i / (3 * kR2G), r = i - j * 3 * kR2G, q = r / kR2G, c = r - q * kR2G;
+        const float* src = q == 0 ? a.bias[j] : (q == 1 ? a.scale[j] : a.shift[j]);
+        s_ep[j][q][c] = src ? src[c] : (q == 1 ? 1.0f : 0.0f);
+    }
+    if (a.copy0) {
+        for (int i = tid; i < (t1 - t0) * 16; i += 512) {
+            const int f = t0 + (i >> 4), c = kR2G + (i & 15) * 8;
+            *reinterpret_cast<half8*>(yclip + (size_t)f * a.ys + c) =
+                *reinterpret_cast<const half8*>(clip + (size_t)f * S + c);
         }
     }
 
     const int ob = wave & 3, fb0 = wave >> 2;   // 32-channel block, first frame block (then every second)
-    float16v acc[3];
-    int fcol[3];        // per frame block: this lane's frame (masked columns: a valid one)
-    half4 xn[3][4];     // x_{j+1} of the epilogue's (frame, 4 channels)
+    float16v acc[NB];
+    int fcol[NB];       // per frame block: this lane's frame (masked columns: a valid one)
     int nfb = 0, lo_j = 0, hi_j = 0, nx = 0;
     for (int c = 0; c < 3 * L; ++c) {
         const int j = c / 3 + 1, k = c - (j - 1) * 3;
         const uint8_t* const in = s_in[(j - 1) & 1];
+        uint8_t* const out = s_in[j & 1];
         if (k == 0) {
             lo_j = lo(j);
             hi_j = hi(j);
             nfb = (hi_j - lo_j + 31) >> 5;
 #pragma unroll
-            for (int i = 0; i < 3; ++i) {
+            for (int i = 0; i < NB; ++i) {
                 const int fb = fb0 + 2 * i;
                 const int f = lo_j + fb * 32 + lrow;
                 fcol[i] = f < hi_j ? f : hi_j - 1;   // masked columns: any valid row, result dropped
@@ -563,51 +597,53 @@ __global__ __launch_bounds__(512) void res2_block_kernel(Res2Args a) {
                 for (int r = 0; r < 16; ++r) acc[i][r] = 0.0f;
             }
         }
-        // chunk c (issued one step ago, or before the loop) has landed; after
-        // the barrier every wave is past chunk c - 1, so its stage is free,
-        // and the previous group's epilogue writes of `in` are complete
-        if (k == 0 || nx == 0) wait_vmcnt<0>();
-        else wait_vmcnt_le(nx);
+        // Chunk c's own instructions have landed (waited for before the
+        // previous group's stores when k == 0).  Younger ones may fly: the
+        // NST - 2 chunks after it and, where they went out after it, x_{j+1}'s.
+        // At k = 2 the wait covers x_{j+1}, issued before this chunk.
+        const int ahead = 3 * L - 1 - c < NST - 2 ? 3 * L - 1 - c : NST - 2;
+        if (k != 0 || c == 0) wait_vmcnt_le(4 * ahead + (NST == 3 && k == 1 ? nx : 0));
+        // after the barrier every wave is past chunk c - 1, so its stage is
+        // free, and the previous group's epilogue writes of `in` are complete
         lds_barrier();
-        if (c + 1 < 3 * L) issue_w(c + 1);
-        nx = 0;
-        if (k == 0 && j < L) {   // x_{j+1} for this group's epilogue, in flight behind the weights
+        if (k == 0) nx = j < L ? issue_x(out, j + 2, lo_j, hi_j) : 0;   // `out` held in_{j-1}
+        if (c + NST - 1 < 3 * L) issue_w(c + NST - 1);
+        const uint8_t* const wt = s_w[c % NST];
+        int rk[NB];   // per frame block: the LDS input row of tap k (reflected into the clip)
 #pragma unroll
-            for (int i = 0; i < 3; ++i) {
-                const int fb = fb0 + 2 * i;
-                if (fb >= nfb) continue;
-                const int f = lo_j + fb * 32 + lrow;
+        for (int i = 0; i < NB; ++i) rk[i] = r2_refl(fcol[i] + (k - 1) * D, T) - base;
+        // the tap's operands all leave LDS ahead of its MFMAs (the block count
+        // is a compile-time one per case: a branch between the reads would
+        // make every MFMA wait out an LDS round trip)
+        auto mfmas = [&](auto nblocks) {
+            constexpr int N = decltype(nblocks)::value;
+            half8 af[8], bf[N][8];
 #pragma unroll
-                for (int g = 0; g < 4; ++g) {
-                    const int oc = ob * 32 + g * 8 + lhalf * 4;
-                    xn[i][g] = f < hi_j ? *reinterpret_cast<const half4*>(clip + (size_t)f * S + (j + 2) * kR2G + oc)
-                                        : half4{0, 0, 0, 0};
-                    ++nx;
-                }
+            for (int ks = 0; ks < 8; ++ks) {
+                const int ch = ks * 2 + lhalf;
+                af[ks] = *reinterpret_cast<const half8*>(wt + r2_off(ob * 32 + lrow, ch));
+#pragma unroll
+                for (int i = 0; i < N; ++i) bf[i][ks] = *reinterpret_cast<const half8*>(in + r2_off(rk[i], ch));
             }
-        }
-        const uint8_t* const wt = s_w[c & 1];
-        int rk[3];   // per frame block: the LDS input row of tap k (reflected into the clip)
 #pragma unroll
-        for (int i = 0; i < 3; ++i) rk[i] = r2_refl(fcol[i] + (k - 1) * D, T) - base;
+            for (int ks = 0; ks < 8; ++ks)
 #pragma unroll
-        for (int ks = 0; ks < 8; ++ks) {
-            const int ch = ks * 2 + lhalf;
-            const half8 af = *reinterpret_cast<const half8*>(wt + r2_off(ob * 32 + lrow, ch));
-#pragma unroll
-            for (int i = 0; i < 3; ++i) {
-                if (fb0 + 2 * i >= nfb) continue;
-                const half8 bf = *reinterpret_cast<const half8*>(in + r2_off(rk[i], ch));
-                acc[i] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af, bf, acc[i], 0, 0, 0);
-            }
-        }
+                for (int i = 0; i < N; ++i)
+                    acc[i] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[ks], bf[i][ks], acc[i], 0, 0, 0);
+        };
+        const int mine = (nfb - fb0 + 1) >> 1;   // this wave's frame blocks
+        if (mine == 1) mfmas(std::integral_constant<int, 1>());
+        if (mine == 2) mfmas(std::integral_constant<int, 2>());
+        if constexpr (NB == 3)
+            if (mine == 3) mfmas(std::integral_constant<int, 3>());
         if (k < 2) continue;
+        // the next chunk before this group's stores, which then drain behind it
+        if (c + 1 < 3 * L) wait_vmcnt_le(4 * (3 * L - 2 - c < NST - 2 ? 3 * L - 2 - c : NST - 2));
         // epilogue of group j: bias -> ReLU -> BN; y_j out for the tile's frames,
-        // in_{j+1} = f16(v + x_{j+1}) into the other input buffer on R_j
-        uint8_t* const out = s_in[j & 1];
-        half_t* const yslot = clip + (j == 1 ? 0 : j) * kR2G;
+        // in_{j+1} = f16(v + x_{j+1}) over x_{j+1} on R_j
+        half_t* const yslot = yclip + (j == 1 ? 0 : j) * kR2G;
 #pragma unroll
-        for (int i = 0; i < 3; ++i) {
+        for (int i = 0; i < NB; ++i) {
             const int fb = fb0 + 2 * i;
             if (fb >= nfb) continue;
             const int f = lo_j + fb * 32 + lrow;
@@ -615,6 +651,8 @@ __global__ __launch_bounds__(512) void res2_block_kernel(Res2Args a) {
 #pragma unroll
             for (int g = 0; g < 4; ++g) {
                 const int oc = ob * 32 + g * 8 + lhalf * 4;
+                half4* const xi = reinterpret_cast<half4*>(out + r2_off(f - base, oc >> 3) + (oc & 7) * 2);
+                const half4 xn = j < L ? *xi : half4{0, 0, 0, 0};
                 half4 yv, iv;
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
@@ -623,13 +661,67 @@ __global__ __launch_bounds__(512) void res2_block_kernel(Res2Args a) {
                     v = v * s_ep[j - 1][1][oc + e];
                     v = v + s_ep[j - 1][2][oc + e];
                     yv[e] = (half_t)v;
-                    iv[e] = (half_t)(v + (float)xn[i][g][e]);
+                    iv[e] = (half_t)(v + (float)xn[e]);
                 }
-                if (f >= t0 && f < t1) *reinterpret_cast<half4*>(yslot + (size_t)f * S + oc) = yv;
-                if (j < L) *reinterpret_cast<half4*>(out + r2_off(f - base, oc >> 3) + (oc & 7) * 2) = iv;
+                if (f >= t0 && f < t1) *reinterpret_cast<half4*>(yslot + (size_t)f * a.ys + oc) = yv;
+                if (j < L) *xi = iv;
             }
         }
     }
+}
+
+// In-place results of a side buffer [B*T][(L + 1) G] (slots 0 and 2 .. L) into
+// buf's slots of the same numbers.
+__global__ __launch_bounds__(256) void res2_copy_kernel(const half_t* __restrict__ y, half_t* __restrict__ buf, long rows,
+                                                        int L, int S) {
+    const int ch = (L + 1) * (kR2G / 8);
+    const long i = (long)blockIdx.x * 256 + threadIdx.x;
+    if (i >= rows * ch) return;
+    const long r = i / ch;
+    const int c = (int)(i - r * ch) * 8;
+    if (c / kR2G == 1) return;
+    *reinterpret_cast<half8*>(buf + r * S + c) = *reinterpret_cast<const half8*>(y + r * (L + 1) * kR2G + c);
+}
+
+// Tiles of a launch: 96-row buffers with three weight stages while their tiles
+// fit the CUs in one round, as many of at least 32 frames as there are CUs
+// (5 x 259 frames, D = 2 / 3 / 4: 53 / 45 / 46 us on 160 rows, 36 / 36 / 37 on
+// 96; 32 x 298, D = 3: 50 / 41); else 160 rows, whose longer tiles recompute
+// less halo (64 x 398: 768 narrow tiles took three rounds, 930 -> 740 us over
+// a whole 32 x 3 s pass).
+void launch_res2(Res2Args& a, int batch, hipStream_t s) {
+    const int halo = 2 * a.L * a.D, t96 = 96 - halo, t160 = 160 - halo;
+    require(t160 >= 32, "res2_block: dilation too large for the LDS tile");
+    const bool narrow = t96 >= 32 && (long)batch * cdiv(a.T, t96) <= 256;
+    a.nt = cdiv(a.T, narrow ? t96 : t160);
+    if (narrow) a.nt = std::max(a.nt, std::min(cdiv(a.T, 32), 256 / batch));
+    a.Tt = cdiv(a.T, a.nt);
+    a.nt = cdiv(a.T, a.Tt);
+    if (narrow) hipLaunchKernelGGL((res2_block_kernel<96, 3>), dim3(batch * a.nt), dim3(512), 0, s, a);
+    else hipLaunchKernelGGL((res2_block_kernel<160, 2>), dim3(batch * a.nt), dim3(512), 0, s, a);
+    VDK_HIP(hipGetLastError());
+}
+
+Res2Args res2_args(const void* d_x, int stride, int batch, int T, int G, int scale, int dil,
+                   const vdk_res2_weights* wts) {
+    require(d_x && wts, "res2_block: NULL pointer");
+    require(G == kR2G, "res2_block: groups of 128 channels only");
+    require(scale >= 2 && scale - 1 <= kR2MaxL, "res2_block: scale must be 2 .. 8");
+    require(batch > 0 && T > dil && dil >= 1, "res2_block: T must exceed the dilation");
+    require(stride >= (scale + 1) * G && stride % 8 == 0 && al16(d_x), "res2_block: bad buffer stride / alignment");
+    require((size_t)batch * T * stride < (1ull << 31), "res2_block: buffer too large for one launch");
+    require((scale - 1) * dil <= 64, "res2_block: dilation too large for the LDS tile");
+    Res2Args a{};
+    a.x = static_cast<const half_t*>(d_x);
+    a.S = stride; a.T = T; a.D = dil; a.L = scale - 1;
+    for (int j = 0; j < a.L; ++j) {
+        require(wts->w[j] && wts->bias[j] && al16(wts->w[j]), "res2_block: missing group weights");
+        a.w[j] = static_cast<const half_t*>(wts->w[j]);
+        a.bias[j] = wts->bias[j];
+        a.scale[j] = wts->scale[j];
+        a.shift[j] = wts->shift[j];
+    }
+    return a;
 }
 
 }  // namespace
@@ -715,31 +807,48 @@ extern "C" int vdk_se_scale_residual(const void* d_x, int x_stride, const float*
     return vdk::se_residual(d_x, x_stride, d_scale, false, d_res, res_stride, batch, T, C, d_y, y_stride, stream);
 }
 
+extern "C" int vdk_res2_block_out(const void* d_x, int stride, int batch, int T, int G, int scale, int dil,
+                                  const vdk_res2_weights* wts, void* d_y, int y_stride, void* stream) {
+    return guarded([&] {
+        Res2Args a = res2_args(d_x, stride, batch, T, G, scale, dil, wts);
+        require(d_y && al16(d_y) && y_stride >= scale * G && y_stride % 8 == 0,
+                "res2_block_out: bad output / stride / alignment");
+        const uintptr_t x0 = reinterpret_cast<uintptr_t>(d_x), y0 = reinterpret_cast<uintptr_t>(d_y);
+        require(x0 + (size_t)batch * T * stride * 2 <= y0 || y0 + (size_t)batch * T * y_stride * 2 <= x0,
+                "res2_block_out: the output must not overlap the input");
+        a.y = static_cast<half_t*>(d_y);
+        a.ys = y_stride;
+        a.copy0 = 1;
+        launch_res2(a, batch, static_cast<hipStream_t>(stream));
+    });
+}
+
 extern "C" int vdk_res2_block(void* d_buf, int stride, int batch, int T, int G, int scale, int dil,
                               const vdk_res2_weights* wts, void* stream) {
     return guarded([&] {
-        require(d_buf && wts, "res2_block: NULL pointer");
-        require(G == kR2G, "res2_block: groups of 128 channels only");
-        require(scale >= 2 && scale - 1 <= kR2MaxL, "res2_block: scale must be 2 .. 8");
-        require(batch > 0 && T > dil && dil >= 1, "res2_block: T must exceed the dilation");
-        require(stride >= (scale + 1) * G && stride % 8 == 0 && al16(d_buf), "res2_block: bad buffer stride / alignment");
-        require((size_t)batch * T * stride < (1ull << 31), "res2_block: buffer too large for one launch");
-        Res2Args a{};
-        a.t1 = static_cast<half_t*>(d_buf);
-        a.S = stride; a.T = T; a.D = dil; a.L = scale - 1;
-        const int tmax = kR2Rows - 2 * a.L * dil;
-        require(tmax >= 32, "res2_block: dilation too large for the LDS tile");
-        a.nt = cdiv(T, tmax);
-        a.Tt = cdiv(T, a.nt);
-        for (int j = 0; j < a.L; ++j) {
-            require(wts->w[j] && wts->bias[j] && al16(wts->w[j]), "res2_block: missing group weights");
-            a.w[j] = static_cast<const half_t*>(wts->w[j]);
-            a.bias[j] = wts->bias[j];
-            a.scale[j] = wts->scale[j];
-            a.shift[j] = wts->shift[j];
+        Res2Args a = res2_args(d_buf, stride, batch, T, G, scale, dil, wts);
+        hipStream_t s = static_cast<hipStream_t>(stream);
+        if (T <= 160 - 2 * a.L * dil) {   // one tile per clip reads all its input before it is overwritten
+            a.y = static_cast<half_t*>(d_buf);
+            a.ys = stride;
+            a.nt = 1;
+            a.Tt = T;
+            hipLaunchKernelGGL((res2_block_kernel<160, 2>), dim3(batch), dim3(512), 0, s, a);
+            VDK_HIP(hipGetLastError());
+            return;
         }
-        hipLaunchKernelGGL(res2_block_kernel, dim3(batch * a.nt), dim3(512), 0, static_cast<hipStream_t>(stream), a);
+        // several tiles: y_j's slot holds x_{j-1}, which a neighbour that starts
+        // late still reads on its halo, so the results go through a side buffer
+        void* tmp = nullptr;
+        const long rows = (long)batch * T;
+        VDK_HIP(hipMallocAsync(&tmp, (size_t)rows * scale * G * 2, s));
+        a.y = static_cast<half_t*>(tmp);
+        a.ys = scale * G;
+        launch_res2(a, batch, s);
+        hipLaunchKernelGGL(res2_copy_kernel, dim3(cdiv(rows * scale * (G / 8), 256)), dim3(256), 0, s, a.y,
+                           static_cast<half_t*>(d_buf), rows, a.L, stride);
         VDK_HIP(hipGetLastError());
+        VDK_HIP(hipFreeAsync(tmp, s));
     });
 }
 

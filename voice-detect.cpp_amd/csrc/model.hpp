@@ -279,8 +279,8 @@ private:
         void* fc_work = nullptr;
         size_t fc_work_bytes = 0;
         // ECAPA: time-major f16 activations and f32 per-clip vectors
-        void *x0p = nullptr, *h0 = nullptr, *t1 = nullptr, *t2 = nullptr, *s2b[2] = {nullptr, nullptr}, *cat = nullptr,
-             *mfa = nullptr, *a1 = nullptr;
+        void *x0p = nullptr, *h0 = nullptr, *t1 = nullptr, *t2 = nullptr, *t3 = nullptr,
+             *s2b[2] = {nullptr, nullptr}, *cat = nullptr, *mfa = nullptr, *a1 = nullptr;
         float *logits = nullptr, *se_m = nullptr, *se_h = nullptr, *se_g = nullptr, *stats = nullptr,
               *pb = nullptr;
         // CAM++

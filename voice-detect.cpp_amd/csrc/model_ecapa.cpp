@@ -223,6 +223,7 @@ void Model::alloc_ecapa_workspace(int batch, int T) {
     w.s2b[0] = ws_alloc(2 * BT * e.group);
     w.s2b[1] = ws_alloc(2 * BT * e.group);
     w.t2 = ws_alloc(2 * BT * e.C);
+    w.t3 = e.group == 128 && e.scale <= 8 ? ws_alloc(2 * BT * e.C) : nullptr;
     w.cat = ws_alloc(2 * BT * nb * e.C);
     w.mfa = ws_alloc(2 * BT * e.mfa);
     w.a1 = ws_alloc(2 * BT * e.att);
@@ -322,8 +323,11 @@ void Model::encode_ecapa(int batch, int T) {
         const int S = C + G;
         uint8_t* t1 = static_cast<uint8_t*>(w.t1);
         tdnn("ecapa_tdnn1", b.tdnn1, xin, xs, batch, T, 1, b.tdnn1.b, 0, 1, 0, t1 + gB, S, 0);
-        if (G == 128 && e.scale <= 8 && (e.scale - 1) * b.dil <= 64) {
-            // all groups in one launch per time tile, the same bits as the chain below
+        const void* r2 = w.t1;   // [y_1 | x_0 | y_2 ..] and its stride
+        int r2s = S;
+        if (w.t3 && (e.scale - 1) * b.dil <= 64) {
+            // all groups in one launch, the same bits as the chain below, into
+            // t3: other time tiles still read x from t1
             vdk_res2_weights rw{};
             for (int j = 0; j + 1 < e.scale; ++j) {
                 rw.w[j] = b.res[j].w;
@@ -336,8 +340,10 @@ void Model::encode_ecapa(int batch, int T) {
                 prof_begin("conv.ecapa_res2_block", n * 2.0 * 3 * G * G * npix,
                            2.0 * npix * G * (2.0 * n) + n * 2.0 * 3 * G * G);
             }
-            check_rc(vdk_res2_block(w.t1, S, batch, T, G, e.scale, b.dil, &rw, stream_));
+            check_rc(vdk_res2_block_out(w.t1, S, batch, T, G, e.scale, b.dil, &rw, w.t3, C, stream_));
             prof_end();
+            r2 = w.t3;
+            r2s = C;
         } else {
             for (int j = 1; j < e.scale; ++j) {
                 const bool last = j + 1 == e.scale;
@@ -346,7 +352,7 @@ void Model::encode_ecapa(int batch, int T) {
                           last ? nullptr : t1 + (j + 2) * gB, S, last ? nullptr : w.s2b[(j + 1) & 1]);
             }
         }
-        tdnn("ecapa_tdnn2", b.tdnn2, w.t1, S, batch, T, 1, b.tdnn2.b, 0, 1, 0, w.t2, C, 0);
+        tdnn("ecapa_tdnn2", b.tdnn2, r2, r2s, batch, T, 1, b.tdnn2.b, 0, 1, 0, w.t2, C, 0);
         // SE (src/encoder.cpp:207-219) and the residual (src/encoder.cpp:243)
         prof_begin("ecapa_se_mean", 0.0, 2.0 * batch * (double)T * C);
         check_rc(vdk_channel_mean(w.t2, C, batch, T, C, w.se_m, stream_));
