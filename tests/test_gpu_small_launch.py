@@ -182,3 +182,55 @@ def test_res2_block_out_tiles(batch, T, dil, scale):
     mag = (sum(np.abs(v) @ np.abs(w[:, k]).T for k, v in enumerate(taps)) + np.abs(b)) * sc + np.abs(sh)
     err = np.abs(got[c, :, :G].view(np.float16).astype(np.float64) - want)
     assert (err <= 3 * G * 2.0 ** -24 * mag + 2.0 ** -11 * np.abs(want) + 2.0 ** -24).all()
+
+
+@pytest.mark.parametrize("B,H,W,IC,OC,res,relu", [
+    (1, 20, 75, 128, 128, True, True),      # one segment, the 5-row band's own width
+    (2, 7, 76, 128, 128, False, True),      # just past it: two segments of 38
+    (1, 6, 151, 64, 128, True, False),      # three segments, the last one narrower
+    (3, 5, 13, 256, 256, True, True),       # narrow map, ragged bands
+    (1, 1, 1, 16, 128, False, False),       # one pixel, one chunk
+    (1, 10, 39, 256, 384, True, True),      # three output groups, two segments of 20
+])
+def test_band_tiles_bitwise(B, H, W, IC, OC, res, relu):
+    """The stride-1 3x3 band kernels at any width: the 32 x 32 tiles and every
+    band height and segment width give the same bits (so the batch may choose),
+    with and without the chunk-major weights, and agree with f64."""
+    rng = np.random.default_rng(B + H + W + IC + OC)
+    announce(f"bands B={B} H={H} W={W} {IC}->{OC} res={res}")
+    x = rng.standard_normal((B, H, W, IC)).astype(np.float16)
+    w = (rng.standard_normal((OC, 3, 3, IC)) * np.sqrt(2.0 / (9 * IC))).astype(np.float16)
+    b = rng.uniform(-0.5, 0.5, OC).astype(np.float32)
+    r = rng.standard_normal((B, H, W, OC)).astype(np.float16)
+    wc = np.ascontiguousarray(w.reshape(OC, 9, IC // 16, 16).transpose(2, 1, 0, 3))
+    keep = [lib.DeviceBuffer.from_array(v) for v in (x, w, b, r, wc)]
+    d = lib.ConvDesc()
+    d.x, d.batch, d.H, d.W, d.IC = keep[0].ptr, B, H, W, IC
+    d.w, d.OC, d.KH, d.KW = keep[1].ptr, OC, 3, 3
+    d.stride_h = d.stride_w = d.pad_h = d.pad_w = d.dil_h = d.dil_w = 1
+    d.bias, d.act = keep[2].ptr, lib.ACT_RELU if relu else lib.ACT_NONE
+    if res:
+        d.residual = keep[3].ptr
+    dy = lib.DeviceBuffer(B * H * W * OC * 2)
+    d.y = dy.ptr
+    outs = run_tiles(d, dy, (B, H, W, OC), [-1] + list(range(102, 109)))
+    assert len(outs) == 8, sorted(outs)
+    d.w_chunked = keep[4].ptr
+    chunked = run_tiles(d, dy, (B, H, W, OC), [-1] + list(range(102, 109)))
+    for o in (outs, chunked):
+        for t in o:
+            assert np.array_equal(o[t], outs[103]), f"tile {t}"
+    xp = np.pad(x.astype(np.float64), ((0, 0), (1, 1), (1, 1), (0, 0)))
+    want, mag = b + np.zeros((B, H, W, OC)), np.abs(b) + np.zeros((B, H, W, OC))
+    for kh in range(3):
+        for kw in range(3):
+            xs = xp[:, kh:kh + H, kw:kw + W]
+            want += xs @ w[:, kh, kw].astype(np.float64).T
+            mag += np.abs(xs) @ np.abs(w[:, kh, kw].astype(np.float64)).T
+    if res:
+        want += r
+        mag += np.abs(r)
+    if relu:
+        want = np.maximum(want, 0)
+    got = outs[-1].view(np.float16).astype(np.float64)
+    assert (np.abs(got - want) <= 9 * IC * 2.0 ** -24 * mag + 2.0 ** -11 * np.abs(want) + 2.0 ** -24).all()

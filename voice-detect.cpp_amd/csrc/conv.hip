@@ -68,6 +68,7 @@ struct ConvArgs {
     int axs, ax_lo, adss, ads_lo;
     int xgl = 4, ygl = 4;      // log2 of the channels per group of x / y (16 or 32)
     int xgs = 16, ygs = 16;    // elements between channel groups of x / y (= group size: contiguous)
+    int nseg = 1;              // column segments of a band (band kernels with producer / compute waves)
 };
 
 // Element offset of channel c in a layout of 2^gl-channel groups gs elements
@@ -2392,9 +2393,10 @@ void launch_band(const ConvArgs& a, hipStream_t s) {
 }
 
 // ---------------------------------------------------------------------------
-// conv3x3_bandws_kernel: stride-1 3x3 conv (pad 1) for maps up to MAXW wide
-// and OC % 128 == 0, one workgroup per band of TH full rows x 128 output
-// channels (flattened 32-pixel MFMA blocks), with the waves split by role:
+// conv3x3_bandws_kernel: stride-1 3x3 conv (pad 1) for OC % 128 == 0, one
+// workgroup per band of TH rows x 128 output channels (flattened 32-pixel MFMA
+// blocks); maps wider than MAXW are cut into column segments of equal width,
+// each with its own halo.  The waves are split by role:
 //  * NCW compute waves in a WMG x WNG grid, each holding 4/WMG 32-channel A
 //    blocks x NJ 32-pixel B blocks of accumulators; they only read LDS and
 //    run MFMAs, never a global load, so no MFMA stream stalls behind the
@@ -2465,9 +2467,12 @@ __global__ __launch_bounds__((WMG * WNG + NP) * 64) void conv3x3_bandws_kernel(C
 
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int H = a.H, W = a.W, IC = a.IC, HW = W + 2;
+    // the workgroup's rows r0 .. r0 + TH - 1, columns cs .. cs + W - 1 (W: the
+    // segment's width) of clip b
+    const int H = a.H, FW = a.W, W = (FW + a.nseg - 1) / a.nseg, IC = a.IC, HW = W + 2;
     const int bands = (H + TH - 1) / TH;
-    const int b = blockIdx.x / bands, r0 = (blockIdx.x - b * bands) * TH;
+    const int bb = blockIdx.x / a.nseg, cs = (blockIdx.x - bb * a.nseg) * W;
+    const int b = bb / bands, r0 = (bb - b * bands) * TH;
     const int oc0 = blockIdx.y * G::OCB;
     const int npx = TH * W;                           // band pixels (rows past H are computed and dropped)
     const bool has_res = a.res != nullptr;
@@ -2491,9 +2496,9 @@ __global__ __launch_bounds__((WMG * WNG + NP) * 64) void conv3x3_bandws_kernel(C
                 const int s = xi * 64 + lane;
                 const int q = s >> 1, hr = div_small(q, inv_hw), hc = q - hr * HW;
                 const int ghalf = (s & 1) ^ ((q >> 3) & 1);
-                const int ih = r0 - 1 + hr, iw = hc - 1;
-                if (hr < TH + 2 && ih >= 0 && ih < H && iw >= 0 && iw < W)
-                    xoff[i] = (int)(((size_t)(b * H + ih) * W + iw) * a.xs * 2) + ghalf * 16;
+                const int ih = r0 - 1 + hr, iw = cs + hc - 1;
+                if (hr < TH + 2 && ih >= 0 && ih < H && iw >= 0 && iw < FW)
+                    xoff[i] = (int)(((size_t)(b * H + ih) * FW + iw) * a.xs * 2) + ghalf * 16;
             }
         }
         const __amdgpu_buffer_rsrc_t wr = __builtin_amdgcn_make_buffer_rsrc(
@@ -2527,9 +2532,9 @@ __global__ __launch_bounds__((WMG * WNG + NP) * 64) void conv3x3_bandws_kernel(C
                     const int sl = ri * 64 + lane;
                     const int pr = half * G::HALF_ROWS + sl / G::SPR, ch = sl % G::SPR;
                     const int r = div_small(pr, inv_w), c = pr - r * W;
-                    const bool ok = ch < 16 && pr < npx && r0 + r < H;
+                    const bool ok = ch < 16 && pr < npx && r0 + r < H && cs + c < FW;
                     const uint32_t off =
-                        ok ? (uint32_t)(((((size_t)(b * H + r0 + r) * W + c) * a.rs + oc0) * 2) + ch * 16) : kOOB;
+                        ok ? (uint32_t)(((((size_t)(b * H + r0 + r) * FW + cs + c) * a.rs + oc0) * 2) + ch * 16) : kOOB;
                     __builtin_amdgcn_raw_ptr_buffer_load_lds(rr, (lds_void*)(dst + ri * 1024), 16, off, 0, 0, 0);
                 }
             }
@@ -2676,18 +2681,163 @@ __global__ __launch_bounds__((WMG * WNG + NP) * 64) void conv3x3_bandws_kernel(C
         const int pr = pg * NJ * 32 + (it * 64 + lane) / G::CPR;
         const half8 v8 = *reinterpret_cast<const half8*>(rrow(pr) + cg0 * 2 + ch * 16);
         const int r = div_small(pr, inv_w), c = pr - r * W;
-        if (pr < npx && r0 + r < H)
-            *reinterpret_cast<half8*>(y + ((size_t)(b * H + r0 + r) * W + c) * a.ys + ch * 8) = v8;
+        if (pr < npx && r0 + r < H && cs + c < FW)
+            *reinterpret_cast<half8*>(y + ((size_t)(b * H + r0 + r) * FW + cs + c) * a.ys + ch * 8) = v8;
     }
 }
 
 template <int TH, int MAXW, int WMG, int WNG, int NJ, int NP>
-void launch_bandws(const ConvArgs& a, hipStream_t s) {
+void launch_bandws(const ConvArgs& args, hipStream_t s) {
+    ConvArgs a = args;
+    a.nseg = cdiv(a.W, MAXW);
     const int B = a.npix / (a.Ho * a.Wo);
-    hipLaunchKernelGGL((conv3x3_bandws_kernel<TH, MAXW, WMG, WNG, NJ, NP>), dim3(B * cdiv(a.H, TH), a.OC / 128),
+    hipLaunchKernelGGL((conv3x3_bandws_kernel<TH, MAXW, WMG, WNG, NJ, NP>), dim3(B * cdiv(a.H, TH) * a.nseg, a.OC / 128),
                        dim3((WMG * WNG + NP) * 64), 0, s, a);
 }
 
+
+// ---------------------------------------------------------------------------
+// conv3x3_slim_kernel: the band kernels' stride-1 3x3 conv (pad 1, the plain
+// epilogue) for launches whose bands leave most of the chip idle: a workgroup
+// computes 32 output channels of 32 consecutive pixels (flattened over the
+// launch) with one compute wave, fed by two producer waves.  Per 16-channel
+// chunk the weights of the 9 taps and the 9 taps' im2col pixel rows go into
+// an NST-stage LDS ring, one DMA instruction per tap ([32 rows][16 channels],
+// the 16-byte halves swapped on odd groups of 8 rows as in the band kernels),
+// from lane offsets that stay fixed over the chunks.  The sums run in the band
+// kernels' order (chunks, taps; accumulators from the bias; the residual
+// through identity-operand MFMAs), so the results are the same bits.
+// Bound by the latency of a chunk's way through LDS.
+// ---------------------------------------------------------------------------
+constexpr int kSlimStages = 4;   // 72 KB: two workgroups per CU (8 stages, one per CU: 9.6 -> 13.7 us at batch 2)
+
+__global__ __launch_bounds__(192) void conv3x3_slim_kernel(ConvArgs a) {
+    constexpr int NST = kSlimStages, STAGE = 18 * 1024;
+    __shared__ __attribute__((aligned(1024))) uint8_t smem[NST * STAGE];
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    int ptile, otile;
+    tile_ids(a, ptile, otile);
+    const int p0 = ptile * 32, oc0 = otile * 32;
+    const int H = a.H, W = a.W, IC = a.IC, nk = IC / 16;
+
+    if (wave > 0) {
+        // ---------------- producers: wave 1 weights, wave 2 pixels ----------------
+        const int row = lane >> 1, half = (lane & 1) ^ ((row >> 3) & 1);
+        const bool wts = wave == 1, chunked = a.wc != nullptr;
+        uint32_t off[9];
+#pragma unroll
+        for (int t = 0; t < 9; ++t) off[t] = kOOB;
+        if (wts) {
+#pragma unroll
+            for (int t = 0; t < 9; ++t)
+                off[t] = chunked ? (uint32_t)((t * a.OC + oc0 + row) * 32 + half * 16)
+                                 : (uint32_t)(((oc0 + row) * 9 + t) * IC * 2 + half * 16);
+        } else if (p0 + row < a.npix) {
+            const int P = p0 + row, b = P / (H * W), rem = P - b * (H * W), ih0 = rem / W, iw0 = rem - ih0 * W;
+#pragma unroll
+            for (int t = 0; t < 9; ++t) {
+                const int ih = ih0 + t / 3 - 1, iw = iw0 + t % 3 - 1;
+                if (ih >= 0 && ih < H && iw >= 0 && iw < W)
+                    off[t] = (uint32_t)(((b * H + ih) * W + iw) * a.xs * 2 + half * 16);
+            }
+        }
+        const __amdgpu_buffer_rsrc_t rs =
+            wts ? __builtin_amdgcn_make_buffer_rsrc((void*)(chunked ? a.wc : a.w), 0, (int)((size_t)a.OC * 9 * IC * 2),
+                                                    0x00020000)
+                : __builtin_amdgcn_make_buffer_rsrc((void*)a.x, 0, (int)(((size_t)(a.npix_in - 1) * a.xs + IC) * 2),
+                                                    0x00020000);
+        const int step = wts && chunked ? 9 * a.OC * 32 : 32;   // bytes from chunk to chunk
+        uint8_t* const dst0 = smem + (wts ? 0 : 9 * 1024);
+        auto issue = [&](int k) {
+            const uint32_t ko = (uint32_t)(k * step);
+#pragma unroll
+            for (int t = 0; t < 9; ++t)
+                __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (lds_void*)(dst0 + (k % NST) * STAGE + t * 1024), 16,
+                                                         off[t] == kOOB ? kOOB : off[t] + ko, 0, 0, 0);
+        };
+#pragma unroll
+        for (int k = 0; k < NST - 1; ++k)
+            if (k < nk) issue(k);
+#pragma unroll 1
+        for (int k = 0; k < nk; ++k) {
+            wait_vmcnt_le((nk - 1 - k < NST - 2 ? nk - 1 - k : NST - 2) * 9);   // chunk k has landed
+            lds_barrier();   // chunk k is visible; the compute wave is done with chunk k-1's stage
+            if (k + NST - 1 < nk) issue(k + NST - 1);
+        }
+        return;
+    }
+
+    // ---------------- compute wave ----------------
+    const int lrow = lane & 31, lhalf = lane >> 5;
+    const int P = p0 + lrow;
+    const bool ok = P < a.npix;
+    half8 rv[2] = {};
+    if (a.res && ok) {
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+            rv[h] = *reinterpret_cast<const half8*>(a.res + (size_t)P * a.rs + oc0 + h * 16 + lhalf * 8);
+    }
+    float16v acc;   // register g*4+e of a lane: channel 8g + 4*lhalf + e
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+        const float4v v = a.bias ? *reinterpret_cast<const float4v*>(a.bias + oc0 + g * 8 + lhalf * 4)
+                                 : float4v{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int e = 0; e < 4; ++e) acc[g * 4 + e] = v[e];
+    }
+    const int fo = lrow * 32 + ((lhalf ^ ((lrow >> 3) & 1)) << 4);
+#pragma unroll 1
+    for (int k = 0; k < nk; ++k) {
+        lds_barrier();   // chunk k has landed
+        const uint8_t* const st = smem + (k % NST) * STAGE + fo;
+        half8 af[9], bf[9];
+#pragma unroll
+        for (int t = 0; t < 9; ++t) {
+            af[t] = *reinterpret_cast<const half8*>(st + t * 1024);
+            bf[t] = *reinterpret_cast<const half8*>(st + (9 + t) * 1024);
+        }
+#pragma unroll
+        for (int t = 0; t < 9; ++t) acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[t], bf[t], acc, 0, 0, 0);
+    }
+    if (a.res) {
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            half8 eye;
+#pragma unroll
+            for (int e = 0; e < 8; ++e) eye[e] = (half_t)((lrow == h * 16 + lhalf * 8 + e) ? 1.0f : 0.0f);
+            acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(eye, rv[h], acc, 0, 0, 0);
+        }
+    }
+    // f16, then the lane halves trade 4-channel pieces, so each lane stores
+    // two whole 8-channel chunks of its pixel
+    const bool relu = a.act == VDK_ACT_RELU;
+    half_t* const y = static_cast<half_t*>(a.y) + (size_t)P * a.ys + oc0;
+#pragma unroll
+    for (int g = 0; g < 4; g += 2) {
+        union { half_t h[4]; int d[2]; } own[2], recv;
+#pragma unroll
+        for (int q = 0; q < 2; ++q)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const float v = acc[(g + q) * 4 + e];
+                own[q].h[e] = (half_t)(relu ? fmaxf(v, 0.0f) : v);
+            }
+#pragma unroll
+        for (int d = 0; d < 2; ++d) recv.d[d] = __shfl_xor(lhalf ? own[0].d[d] : own[1].d[d], 32, 64);
+        half8 out;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            out[e] = lhalf ? recv.h[e] : own[0].h[e];
+            out[e + 4] = lhalf ? own[1].h[e] : recv.h[e];
+        }
+        if (ok) *reinterpret_cast<half8*>(y + (g + lhalf) * 8) = out;
+    }
+}
+
+void launch_slim(const ConvArgs& a, hipStream_t s) {
+    hipLaunchKernelGGL(conv3x3_slim_kernel, dim3(cdiv(a.npix, 32), a.OC / 32), dim3(192), 0, s, a);
+}
 
 template <int BM, int BN, int WM, int WN, int KC>
 void launch_igemm(const ConvArgs& a, hipStream_t s) {
@@ -2732,7 +2882,8 @@ struct TileCfg {
 // kernel with producer / compute waves, 85-88 narrow tiles of that kernel
 // with the prologue / segment-sum variants, 92-101 the GEMM kernel's tiles for
 // launches that leave the chip partly idle (deep rings of 64- and 128-channel
-// chunks; pick_small_tile).
+// chunks; pick_small_tile), 102 the band kernels' sums on 32 x 32 tiles, 103-108
+// the producer / compute band kernel on column segments of any map (pick_band).
 
 // Tile table.  Wave tiles are WM x WN = (bm / waves_m) x (bn / waves_n) with
 // 4 waves per workgroup; entries are selected per layer by pick_tile().
@@ -2839,6 +2990,13 @@ const TileCfg kTiles[] = {
     {32, 64, 32, launch_gemm_ws<32, 64, 1, 2, 32, 8, 2>, false, 0, 0, 0, true},                   // 99
     {128, 64, 128, launch_gemm_ws<128, 64, 2, 2, 128, 3, 4>, false, 0, 0, 0, true},               // 100
     {128, 128, 64, launch_gemm_ws<128, 128, 4, 2, 64, 4, 4>, false, 0, 0, 0, true},               // 101
+    {32, 32, 16, launch_slim, true, 0, 1 << 20},       // 102: the band kernels' sums on 32 x 32 tiles
+    {128, 384, 16, launch_bandws<5, 75, 2, 4, 3, 4>, true, 0, 1 << 20},  // 103: bands of column segments (wide maps)
+    {128, 192, 16, launch_bandws<5, 38, 2, 2, 3, 4>, true, 0, 1 << 20},  // 104
+    {128, 256, 16, launch_bandws<3, 75, 2, 4, 2, 4>, true, 0, 1 << 20},  // 105: three-row bands
+    {128, 128, 16, launch_bandws<3, 38, 2, 2, 2, 4>, true, 0, 1 << 20},  // 106
+    {128, 96, 16, launch_bandws<1, 75, 4, 3, 1, 4>, true, 0, 1 << 20},   // 107: one-row bands
+    {128, 64, 16, launch_bandws<1, 38, 4, 1, 2, 4>, true, 0, 1 << 20},   // 108
 };
 constexpr int kNumTiles = (int)(sizeof(kTiles) / sizeof(kTiles[0]));
 
@@ -2972,6 +3130,40 @@ int pick_small_tile(const ConvArgs& a) {
 // when the launch is a few rounds long.
 long round_cost(const ConvArgs& a, int t) {
     return cdiv(cdiv(a.npix, kTiles[t].bn) * cdiv(a.OC, kTiles[t].bm), 256) * (long)kTiles[t].bm * kTiles[t].bn;
+}
+
+// Stride-1 3x3 layers with 128-channel output groups and the plain epilogue:
+// the band kernels, whose tiles all run the same sums in the same order, so
+// the map's width and the batch choose among them freely.  Each takes a fixed
+// time per round of 256 workgroups, base + chunks x per (us over the launch,
+// measured at 128 and 256 channels, single launches with inputs flushed to
+// HBM); the least total wins.  Against the rule before (5-row bands, one-row
+// ones under 48 workgroups, LDS-DMA tiles on maps wider than 75 / 38): 20 x 75
+// x 128 14.6 -> 8.8 us at batch 1 (102), 27.4 -> 16.8 at batch 16 (106), 29.2
+// -> 22.4 at batch 32 (104); 20 x 126 x 128 at batch 16 34.7 -> 22.1 (104);
+// 10 x 38 x 256 16.8 -> 10.8 at batch 1 (102), 27.9 -> 22.6 at batch 16 (106);
+// 10 x 63 x 256 at batch 64 68.8 -> 53.3 (103).
+int pick_band(const ConvArgs& a) {
+    if (!is_s1_3x3(a) || a.OC % 128 != 0 || !plain_epilogue(a) || (long)a.npix * a.OC >= (1L << 30)) return -1;
+    struct BandCost { int tile, th, maxw; float base, per; };
+    static const BandCost kBands[] = {
+        {103, 5, 75, 9.5f, 1.56f}, {104, 5, 38, 6.0f, 1.06f}, {105, 3, 75, 7.5f, 1.06f},
+        {106, 3, 38, 4.5f, 0.81f}, {107, 1, 75, 3.5f, 0.81f}, {108, 1, 38, 3.1f, 0.64f},
+    };
+    const int chunks = a.IC / 16, B = a.npix / (a.Ho * a.Wo);
+    const auto rounds = [](long wgs) { return (float)((wgs + 255) / 256); };
+    int best = -1;
+    float cost = 0.0f;
+    for (const BandCost& c : kBands) {
+        if (!tile_fits(kTiles[c.tile], a)) continue;
+        const float v = rounds((long)B * cdiv(a.H, c.th) * cdiv(a.W, c.maxw) * (a.OC / 128)) * (c.base + c.per * chunks);
+        if (best < 0 || v < cost) best = c.tile, cost = v;
+    }
+    // the 32 x 32 tiles: two workgroups share a CU
+    const long w32 = (long)cdiv(a.npix, 32) * (a.OC / 32);
+    const float slim = w32 <= 256 ? 2.3f + 0.25f * chunks : rounds(w32) * (1.0f + 0.275f * chunks);
+    if (best >= 0 && tile_fits(kTiles[102], a) && slim < cost) best = 102;
+    return best;
 }
 
 // Per-layer-class defaults, from a sweep of every ResNet34 conv shape at
@@ -3162,20 +3354,11 @@ int pick_tile(const ConvArgs& a) {
         if (a.IC == 128 && a.OC == 256) return 40;
         if (a.IC == 256 && a.OC == 512) return 40;
     }
-    if (is_s1_3x3(a) && a.IC == 64 && a.OC == 64 && plain_epilogue(a)) return 66;   // 3-stage ring
-    // small batches (5-row bands on under 48 workgroups): one-row bands, the
-    // same bits on 5x the workgroups; measured on ResNet34's maps: 128->128
-    // 22.1 -> 11.1 us at batch 1, 23.1 -> 15.0 us at batch 8, slower from
-    // batch 16 (64 workgroups); 256->256 23.8 -> 14.8 us at batch 1
-    const long bands5 = (long)(a.npix / (a.Ho * a.Wo)) * cdiv(a.H, 5) * (a.OC / 128);
-    if (is_s1_3x3(a) && a.OC == 128 && a.W > BandTile<5, 3>::MAXW && bands5 < 48 && tile_fits(kTiles[77], a))
-        return 77;
-    if (is_s1_3x3(a) && a.OC >= 256 && a.W <= BandTile<5, 3>::MAXW && bands5 < 48 && tile_fits(kTiles[78], a))
-        return 78;
-    if (is_s1_3x3(a) && a.OC == 128 && a.W > BandTile<5, 3>::MAXW && tile_fits(kTiles[64], a)) return 64;
-    if (is_s1_3x3(a) && a.OC == 128 && a.W > BandTile<5, 3>::MAXW && tile_fits(kTiles[57], a)) return 57;
-    if (is_s1_3x3(a) && a.OC >= 256 && a.W <= BandTile<5, 3>::MAXW && tile_fits(kTiles[65], a)) return 65;
-    if (is_s1_3x3(a) && a.OC >= 256 && a.W <= BandTile<5, 3>::MAXW && tile_fits(kTiles[58], a)) return 58;
+    // (up to 256 64 x 64 tiles: the GEMM kernel's, the same bits; batch 1 10.2 -> 8.8 us)
+    if (is_s1_3x3(a) && a.IC == 64 && a.OC == 64 && plain_epilogue(a))
+        return cdiv(a.npix, 64) <= 256 && tile_fits(kTiles[98], a) ? 98 : 66;   // 66: 3-stage ring
+    const int band = pick_band(a);
+    if (band >= 0) return band;
     // ResNet's stride-2 convs at small batches (under 8192 output pixels, e.g.
     // batch 1), measured: the 3x3s from 64 / 128 channels on the 128x32 DMA
     // tile (18.8 -> 9.6 / 13.7 us), the rest on the 64x64 register-staged tile
