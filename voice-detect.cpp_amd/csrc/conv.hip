@@ -863,18 +863,27 @@ void launch_dma(const ConvArgs& a, hipStream_t s) {
 // (p + NPW * i of the chunk's NINS) fills LDS row r = q / CPR (q = 64 * ins
 // + lane), 16-byte slot s with chunk swz(r, s) of weight row oc0 + r
 // ([OC][KH][KW][IC]) or, past the BM weight rows, of output pixel
-// p0 + r - BM.  A weight slot keeps its byte offset at tap 0 / channel 0
-// (-1: past the weights, reads zeros); a pixel slot its clip's first input
-// row b * H (-1: past the pixels) and the tap-0 input row / column ih0, iw0
-// (with the slot's chunk in the low 4 bits), checked against the map per tap.
+// p0 + r - BM.  Every lane keeps the byte offset of its slot, kOOB where it
+// reads zeros: a weight slot's at K = 0, a pixel slot's in the current tap at
+// channel 0, taken anew when the tap changes; the chunk's place along K is a
+// wave-uniform scalar offset, so a chunk costs the instructions alone.  (With
+// the offsets recomputed per chunk the small-launch tiles' producers held up
+// their one compute wave.)  issue() is called for chunks 0, 1, 2, ... in turn.
 template <int BM, int KC, int IPW, int NPW>
 struct GemmFeed {
     static constexpr int CPR = KC / 8;
-    int p, lane, icw;
-    int off[IPW], ih0[IPW], iw0[IPW], cof[IPW];
+    static constexpr int WI = BM * CPR / 64;   // the weight rows' instructions (whole ones)
+    int p, icw, tap_c0, kw, wk;                // K per tap; the next chunk's channel in its tap, tap column, bytes along K
+    int ih0[IPW], iw0[IPW], base[IPW];         // pixel slots: tap 0's input row / column; element offset of input (0, 0)
+    uint32_t cur[IPW];
     __amdgpu_buffer_rsrc_t wr, xr;
-    __device__ __forceinline__ GemmFeed(const ConvArgs& a, int p_, int lane_, int p0, int oc0) : p(p_), lane(lane_) {
-        // split-f16 (1x1 only): K per tap runs over [x_hi . w_hi | x_lo . w_hi | x_hi . w_lo]
+    // wave-uniform; known at compile time when the weight instructions split
+    // evenly over the feeding waves (ins < WI iff i < WI / NPW)
+    __device__ __forceinline__ bool is_w(int i) const { return WI % NPW == 0 ? i < WI / NPW : p + NPW * i < WI; }
+    __device__ __forceinline__ void init(const ConvArgs& a, int p_, int lane, int p0, int oc0) {
+        p = p_;
+        tap_c0 = kw = wk = 0;
+        // split-f16: K per tap runs over [x_hi . w_hi | x_lo . w_hi | x_hi . w_lo]
         icw = a.split ? (a.split == 2 ? 2 : 3) * a.IC : a.IC;
         const int xext = ((a.IC >> a.xgl) - 1) * a.xgs + (1 << a.xgl);   // a pixel's channels in one plane
         wr = __builtin_amdgcn_make_buffer_rsrc((void*)a.w, 0, (int)((size_t)a.OC * a.KH * a.KW * icw * 2),
@@ -886,50 +895,62 @@ struct GemmFeed {
         for (int i = 0; i < IPW; ++i) {
             const int ins = p + NPW * i;
             const int q = ins * 64 + lane, r = q / CPR, c = swz<KC>(r, q - r * CPR);
-            ih0[i] = iw0[i] = 0;
-            cof[i] = chan_off(c * 8, a.xgl, a.xgs);   // the slot's 8 channels within a chunk
+            ih0[i] = iw0[i] = INT_MIN / 2;   // no pixel: outside the map in every tap
+            base[i] = 0;
+            cur[i] = kOOB;
             if (r < BM) {
-                off[i] = oc0 + r < a.OC ? ((oc0 + r) * a.KH * a.KW * icw + c * 8) * 2 : -1;
+                if (oc0 + r < a.OC) cur[i] = (uint32_t)(((oc0 + r) * a.KH * a.KW * icw + c * 8) * 2);
             } else {
                 const int P = p0 + r - BM;
-                off[i] = -1;
                 if (P < a.npix) {
                     const int b = P / HoWo, rem = P - b * HoWo;
                     const int oh = rem / a.Wo, ow = rem - oh * a.Wo;
-                    off[i] = b * a.H;
                     ih0[i] = oh * a.sh - a.ph;
                     iw0[i] = ow * a.sw - a.pw;
+                    base[i] = b * a.H * a.W * a.xs + chan_off(c * 8, a.xgl, a.xgs);   // the slot's 8 channels in a chunk
                 }
             }
         }
+        set_tap(a);
     }
-    // This wave's instructions of chunk k (tap k / ncpt, K offset (k % ncpt)
-    // * KC) into the stage at dst: branch-free (selects of out-of-range
-    // offsets, the weight / pixel split fixed at compile time), so the loads
-    // go out back to back.  Chunks cover whole channel groups and, split,
-    // lie inside one plane term.
-    __device__ __forceinline__ void issue(const ConvArgs& a, uint8_t* dst, int k, int ncpt) const {
-        const int tap = k / ncpt, c0 = (k - tap * ncpt) * KC;
-        const int kh = tap / a.KW, kw = tap - kh * a.KW;
-        const int term = a.split ? (c0 >= 2 * a.IC ? 2 : (c0 >= a.IC ? 1 : 0)) : 0;
-        const int xc = (term == 1 ? a.x_lo : 0) + chan_off(c0 - term * a.IC, a.xgl, a.xgs);   // the chunk's first channel
-        constexpr int WI = BM * CPR / 64;   // the weight rows' instructions (whole ones)
+    // the pixel slots' offsets in the cursor's tap (ih0 / iw0 are its row and column)
+    __device__ __forceinline__ void set_tap(const ConvArgs& a) {
+#pragma unroll
+        for (int i = 0; i < IPW; ++i)
+            if (!is_w(i)) {
+                const bool in = (unsigned)ih0[i] < (unsigned)a.H && (unsigned)iw0[i] < (unsigned)a.W;
+                cur[i] = in ? (uint32_t)((base[i] + (ih0[i] * a.W + iw0[i]) * a.xs) * 2) : kOOB;
+            }
+    }
+    // This wave's instructions of the next chunk into the stage at dst.
+    // Chunks cover whole channel groups and, split, lie inside one plane term.
+    __device__ __forceinline__ void issue(const ConvArgs& a, uint8_t* dst) {
+        const int term = a.split ? (tap_c0 >= 2 * a.IC ? 2 : (tap_c0 >= a.IC ? 1 : 0)) : 0;
+        const int xk = ((term == 1 ? a.x_lo : 0) + chan_off(tap_c0 - term * a.IC, a.xgl, a.xgs)) * 2;
 #pragma unroll
         for (int i = 0; i < IPW; ++i) {
             const int ins = p + NPW * i;
-            // wave-uniform; known at compile time when the weight instructions
-            // split evenly over the feeding waves (ins < WI iff i < WI / NPW)
-            const bool wrow = WI % NPW == 0 ? i < WI / NPW : ins < WI;
-            if (wrow) {
-                const uint32_t o = off[i] < 0 ? kOOB : (uint32_t)(off[i] + (tap * icw + c0) * 2);
-                __builtin_amdgcn_raw_ptr_buffer_load_lds(wr, (lds_void*)(dst + ins * 1024), 16, o, 0, 0, 0);
+            const uint32_t o = cur[i];
+            const int so = is_w(i) ? wk : xk;
+            if (is_w(i)) {
+                __builtin_amdgcn_raw_ptr_buffer_load_lds(wr, (lds_void*)(dst + ins * 1024), 16, o, so, 0, 0);
             } else {
-                const int ih = ih0[i] + kh * a.dh, iw = iw0[i] + kw * a.dw;
-                const bool in = off[i] >= 0 && (unsigned)ih < (unsigned)a.H && (unsigned)iw < (unsigned)a.W;
-                const uint32_t pos = (uint32_t)((((off[i] + ih) * a.W + iw) * a.xs + xc + cof[i]) * 2);
-                __builtin_amdgcn_raw_ptr_buffer_load_lds(xr, (lds_void*)(dst + ins * 1024), 16, in ? pos : kOOB, 0, 0,
-                                                         0);
+                __builtin_amdgcn_raw_ptr_buffer_load_lds(xr, (lds_void*)(dst + ins * 1024), 16, o, so, 0, 0);
             }
+        }
+        wk += KC * 2;
+        tap_c0 += KC;
+        if (tap_c0 == icw && a.KH * a.KW > 1) {   // the next tap
+            tap_c0 = 0;
+            const bool row = ++kw == a.KW;
+            const int dh = row ? a.dh : 0, dw = row ? -(a.KW - 1) * a.dw : a.dw;
+            if (row) kw = 0;
+#pragma unroll
+            for (int i = 0; i < IPW; ++i) {
+                ih0[i] += dh;
+                iw0[i] += dw;
+            }
+            set_tap(a);
         }
     }
 };
@@ -988,18 +1009,18 @@ __global__ __launch_bounds__((WMG * WNG + NP) * 64) void gemm_ws_kernel(ConvArgs
 
     if (wave >= G::NCW) {
         // ---------------- producers ----------------
-        GemmFeed<BM, KC, G::IPP, NP> feed(a, wave - G::NCW, lane, p0, oc0);
-        auto issue = [&](int k) { feed.issue(a, smem + (k % NST) * G::STAGE, k, ncpt); };
+        GemmFeed<BM, KC, G::IPP, NP> feed;
+        feed.init(a, wave - G::NCW, lane, p0, oc0);
 #pragma unroll
         for (int k = 0; k < NST - 1; ++k)
-            if (k < nk) issue(k);
+            if (k < nk) feed.issue(a, smem + k * G::STAGE);
 #pragma unroll 1
         for (int k = 0; k < nk; ++k) {
             // chunk k has landed once at most min(NST-2, nk-1-k) younger chunks are in flight
             const int younger = nk - 1 - k < NST - 2 ? nk - 1 - k : NST - 2;
             wait_vmcnt_le(younger * G::IPP);
             lds_barrier();   // chunk k is visible; the compute waves are done with chunk k-1's stage
-            if (k + NST - 1 < nk) issue(k + NST - 1);
+            if (k + NST - 1 < nk) feed.issue(a, smem + ((k + NST - 1) % NST) * G::STAGE);
         }
     } else {
         // ---------------- compute waves ----------------
@@ -1017,7 +1038,11 @@ __global__ __launch_bounds__((WMG * WNG + NP) * 64) void gemm_ws_kernel(ConvArgs
         for (int k = 0; k < nk; ++k) {
             lds_barrier();   // chunk k has landed; chunk k-1's reads are done
             const uint8_t* const sa = smem + (k % NST) * G::STAGE;
-            half8 af[2][TM], bf[2][TN];
+// Wave tiles of one or two blocks have too few MFMAs to hide a
+            // fragment read behind: the chunk's reads all go out first.  Larger ones read one k-step ahead, between the MFMAs.
+            constexpr bool kAll = TM * TN <= 2;
+            constexpr int NB = kAll ? KS : 2;
+            half8 af[NB][TM], bf[NB][TN];
             auto load = [&](int kk, int buf) {
                 const int c = kk * 2 + lhalf;
 #pragma unroll
@@ -1028,10 +1053,15 @@ __global__ __launch_bounds__((WMG * WNG + NP) * 64) void gemm_ws_kernel(ConvArgs
                     bf[buf][j] = *reinterpret_cast<const half8*>(
                         sa + boff[j] + swz<KC>(BM + n_off + j * 32 + lrow, c) * 16);
             };
-            load(0, 0);
+            if constexpr (kAll) {
+#pragma unroll
+                for (int kk = 0; kk < KS; ++kk) load(kk, kk);
+            } else {
+                load(0, 0);
+            }
 #pragma unroll
             for (int kk = 0; kk < KS; ++kk) {
-                const int cb = kk & 1;
+                const int cb = kAll ? kk : kk & 1;
                 if constexpr (PRO) {   // BatchNorm + ReLU of the input channels, as the f16 operand
                     const int ch = k * KC + kk * 16 + lhalf * 8;
                     const float4v sc0 = *reinterpret_cast<const float4v*>(s_in + ch);
@@ -1046,12 +1076,13 @@ __global__ __launch_bounds__((WMG * WNG + NP) * 64) void gemm_ws_kernel(ConvArgs
                             bf[cb][j][e + 4] = (half_t)fmaxf((float)bf[cb][j][e + 4] * sc1[e] + sh1[e], 0.0f);
                         }
                 }
-                if (kk + 1 < KS) load(kk + 1, cb ^ 1);
+                if (!kAll && kk + 1 < KS) load(kk + 1, cb ^ 1);
 #pragma unroll
                 for (int i = 0; i < TM; ++i)
 #pragma unroll
                     for (int j = 0; j < TN; ++j)
                         acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[cb][i], bf[cb][j], acc[i][j], 0, 0, 0);
+                if (kAll) continue;
                 if (kk + 1 < KS) {
                     // one MFMA, then one fragment read, in turn
 #pragma unroll
