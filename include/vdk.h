@@ -567,6 +567,12 @@ int vdk_time_mean(const void* d_x, int x_f32, int batch, int T, int C, float* d_
  * the emotion head's weighted layer sum, one hidden state at a time. */
 int vdk_time_mean_acc(const void* d_x, int x_f32, int batch, int T, int C, float w, int accumulate,
                       float* d_out, void* stream);
+/* out [B][C] = sum_i weights[i] * mean over time of state i, states f16
+ * [B][T][C] state_stride elements apart (a multiple of 8), n_states <= 32
+ * (weights on the host; zero ones are skipped): the same values as one
+ * vdk_time_mean_acc call per state in turn. */
+int vdk_time_mean_states(const void* d_x, size_t state_stride, int n_states, int batch, int T, int C,
+                         const float* weights, float* d_out, void* stream);
 
 #ifdef __cplusplus
 }

@@ -5,6 +5,8 @@ the chip in one round; the K order (taps, planes, 16-channel steps) is the same
 in every tile, so its result equals the LDS-DMA / register-staged tiles' bit
 for bit, and the default pick's.  Compared against f64 as well.
 """
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -234,3 +236,46 @@ def test_band_tiles_bitwise(B, H, W, IC, OC, res, relu):
         want = np.maximum(want, 0)
     got = outs[-1].view(np.float16).astype(np.float64)
     assert (np.abs(got - want) <= 9 * IC * 2.0 ** -24 * mag + 2.0 ** -11 * np.abs(want) + 2.0 ** -24).all()
+
+
+@pytest.mark.parametrize("T,H,G,K", [(149, 768, 16, 128), (31, 128, 2, 128), (33, 96, 2, 33), (1, 128, 2, 7)])
+def test_pos_conv_small_launch_bitwise(T, H, G, K):
+    """wav2vec2's positional conv: one clip (32-frame workgroups) gives the
+    bits it has in a batch that fills the chip (192-frame workgroups)."""
+    rng = np.random.default_rng(T + H + K)
+    announce(f"pos_conv small T={T} H={H} G={G} K={K}")
+    B, icg, L = 1 + 256 // (G * ((T + 31) // 32)), H // G, lib.lib()
+    x = rng.standard_normal((B, T, H)).astype(np.float16)
+    w = np.zeros((G, 64, K, icg), np.float16)
+    w[:, :icg] = rng.standard_normal((G, icg, K, icg)) * np.sqrt(1.0 / (icg * K))
+    keep = [lib.DeviceBuffer.from_array(v) for v in (x, w, (0.1 * rng.standard_normal(H)).astype(np.float32))]
+    dy, d1 = lib.DeviceBuffer(B * T * H * 4), lib.DeviceBuffer(T * H * 4)
+    lib.check(L.vdk_pos_conv(keep[0].ptr, B, T, H, G, keep[1].ptr, keep[2].ptr, K, K // 2, dy.ptr, None))
+    for c in (0, B - 1):
+        lib.check(L.vdk_pos_conv(keep[0].ptr + c * T * H * 2, 1, T, H, G, keep[1].ptr, keep[2].ptr, K, K // 2, d1.ptr,
+                                 None))
+        lib.check(L.vdk_synchronize())
+        assert np.array_equal(d1.to_array(np.uint32, (T, H)), dy.to_array(np.uint32, (B, T, H))[c])
+
+
+@pytest.mark.parametrize("n,B,T,C", [(13, 1, 159, 768), (1, 3, 1, 32), (25, 2, 1000, 100), (32, 1, 7, 1024)])
+def test_time_mean_states_equals_one_by_one(n, B, T, C):
+    """The pooled states in one launch: the bits of one accumulating launch per
+    state, zero weights skipped, a gap between the states."""
+    rng = np.random.default_rng(n + T + C)
+    announce(f"time_mean_states n={n} B={B} T={T} C={C}")
+    L, gap = lib.lib(), (B * T * C + 71) // 8 * 8
+    x = rng.standard_normal((n, gap)).astype(np.float16)
+    w = rng.uniform(-1, 1, n).astype(np.float32)
+    w[n // 2 + 1:n // 2 + 2] = 0.0
+    dx, do, dr = lib.DeviceBuffer.from_array(x), lib.DeviceBuffer(B * C * 4), lib.DeviceBuffer(B * C * 4)
+    lib.check(L.vdk_time_mean_states(dx.ptr, gap, n, B, T, C, w.ctypes.data_as(ctypes.POINTER(ctypes.c_float)), do.ptr,
+                                     None))
+    first = True
+    for i in range(n):
+        if w[i] != 0:
+            lib.check(L.vdk_time_mean_acc(dx.ptr + i * gap * 2, 0, B, T, C, ctypes.c_float(w[i]), 0 if first else 1,
+                                          dr.ptr, None))
+            first = False
+    lib.check(L.vdk_synchronize())
+    assert np.array_equal(do.to_array(np.uint32, (B, C)), dr.to_array(np.uint32, (B, C)))

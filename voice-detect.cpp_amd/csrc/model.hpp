@@ -298,7 +298,9 @@ private:
         float *wstats = nullptr, *fe32 = nullptr, *z = nullptr, *acc = nullptr, *wpool = nullptr, *wt1 = nullptr,
               *wt2 = nullptr, *raw = nullptr;
         void *fe[2] = {nullptr, nullptr}, *u = nullptr, *wproj = nullptr, *wh = nullptr, *wh1 = nullptr,
+             *wstates = nullptr, *wlast = nullptr,
              *qkv = nullptr, *att = nullptr, *ffb = nullptr, *c0_work = nullptr;
+        size_t state_rows = 0;   // rows of each hidden state in wstates
         size_t c0_work_bytes = 0;
         int feat_buf = 0;           // which fe[] holds the conv features after a forward
     };

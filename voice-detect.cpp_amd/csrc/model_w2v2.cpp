@@ -280,6 +280,13 @@ void Model::alloc_w2v2_workspace(int batch, int n) {
     w.acc = static_cast<float*>(ws_alloc(4 * BT * H));
     w.wh = ws_alloc(2 * BT * H);
     w.wh1 = ws_alloc(2 * BT * H);
+    // small launches of the post-norm stack keep every hidden state and pool
+    // them in one launch at the end; larger ones pool state by state (their
+    // launches are long, and 13 states of 64 x 10 s would be 0.6 GB)
+    if (!c.stable_layer_norm && c.n_layers + 1 <= 32 && H % 8 == 0) {
+        w.state_rows = std::min<size_t>(BT, 4096);
+        w.wstates = ws_alloc(2 * w.state_rows * H * (c.n_layers + 1));
+    }
     w.qkv = ws_alloc(2 * BT * 3 * H);
     w.att = ws_alloc(2 * BT * H);
     w.ffb = ws_alloc(2 * BT * c.ff);
@@ -426,15 +433,27 @@ void Model::analyze_forward(const float* d_pcm, int batch, int n, float* d_raw) 
     } else {
         // post-norm (src/analyze_w2v2.cpp:429-468): hidden_states[0] is the
         // encoder LN of (projection + pos conv), then every layer's output
-        ln("w2v2_ln", w.z, BT, H, m.enc_n, VDK_LN_X_F32, w.wh, nullptr, 0.0f);
-        pool_state(w.wh, 0, 0);
+        const bool keep = (size_t)BT <= w.state_rows && std::count(sw.begin(), sw.end(), 0.0f) + 1 < (long)sw.size();
+        auto state = [&](int i) -> void* {
+            return keep ? static_cast<uint8_t*>(w.wstates) + 2 * w.state_rows * H * i : w.wh;
+        };
+        ln("w2v2_ln", w.z, BT, H, m.enc_n, VDK_LN_X_F32, state(0), nullptr, 0.0f);
+        if (!keep) pool_state(w.wh, 0, 0);
         for (int li = 0; li < c.n_layers; ++li) {
             const W2Layer& L = m.layers[li];
-            attention(L, w.wh, 0, w.wh, w.z, 1);
+            attention(L, state(li), 0, state(li), w.z, 1);
             ln("w2v2_ln", w.z, BT, H, L.ln1, VDK_LN_X_F32, w.wh1, nullptr, 0.0f);
             feed_forward(L, w.wh1, 0, w.wh1, w.z, 1);
-            ln("w2v2_ln", w.z, BT, H, L.ln2, VDK_LN_X_F32, w.wh, nullptr, 0.0f);
-            pool_state(w.wh, 0, li + 1);
+            ln("w2v2_ln", w.z, BT, H, L.ln2, VDK_LN_X_F32, state(li + 1), nullptr, 0.0f);
+            if (!keep) pool_state(w.wh, 0, li + 1);
+        }
+        w.wlast = state(c.n_layers);
+        if (keep) {
+            prof_begin("w2v2_time_mean", 0.0, 2.0 * BT * H * sw.size());
+            check_rc(vdk_time_mean_states(w.wstates, w.state_rows * H, (int)sw.size(), batch, T, H, sw.data(), w.wpool,
+                                          stream_));
+            prof_end();
+            pooled = true;
         }
     }
     require(pooled, "voicedetect: the analyze head pools no hidden state");
@@ -499,7 +518,7 @@ void Model::analyze_capture(const float* pcm, int batch, int n, float* feat, flo
         if (c.stable_layer_norm)
             VDK_HIP(hipMemcpyAsync(hidden, ws_.acc, 4 * BT * c.hidden, hipMemcpyDeviceToHost, stream_));
         else
-            widen(ws_.wh, BT * c.hidden, hidden);
+            widen(ws_.wlast, BT * c.hidden, hidden);
     }
     if (raw) VDK_HIP(hipMemcpyAsync(raw, ws_.raw, 4 * (size_t)batch * w2_.n_out, hipMemcpyDeviceToHost, stream_));
     VDK_HIP(hipStreamSynchronize(stream_));

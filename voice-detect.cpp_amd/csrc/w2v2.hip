@@ -121,38 +121,52 @@ __global__ __launch_bounds__(256) void conv0_moments_kernel(const float* __restr
     part[((size_t)b * gridDim.x + chunk) * NP + p] = acc;
 }
 
-// Chunk partials -> per-clip moment sums, in chunk order.
-__global__ __launch_bounds__(256) void conv0_moments_reduce_kernel(const double* __restrict__ part, int nchunk,
-                                                                   int NP, double* __restrict__ mom) {
-    const int b = blockIdx.x, p = threadIdx.x;
-    if (p >= NP) return;
-    double s = 0.0;
-    for (int j = 0; j < nchunk; ++j) s += part[((size_t)b * nchunk + j) * NP + p];
-    mom[(size_t)b * NP + p] = s;
-}
+// Chunk partials -> the clip's moments -> the affine of 256 of its channels.
+// The chunks are summed in kMomSlices interleaved slices, each in order, then
+// the slices in order: every workgroup of a clip forms the same moments, and a
+// clip's do not depend on the batch.  (One thread per moment walking all chunks
+// and a second launch took 38 + 11 us for one 3.2 s clip, one load latency
+// after the other; this 8 us.)
+constexpr int kMomMax = kMaxK + kMaxK * (kMaxK + 1) / 2;   // moments per clip
+constexpr int kMomSlices = 1024 / kMomMax > 6 ? 6 : 1024 / kMomMax;
 
-__global__ __launch_bounds__(256) void conv0_finalize_kernel(const double* __restrict__ mom,
-                                                             const float* __restrict__ w,
-                                                             const float* __restrict__ bias, int C, int K, int T0,
-                                                             const float* __restrict__ gamma,
-                                                             const float* __restrict__ beta, float eps,
-                                                             float* __restrict__ scale, float* __restrict__ shift) {
-    const int c = blockIdx.x * 256 + threadIdx.x, b = blockIdx.y;
-    if (c >= C) return;
-    const int NP = K + K * (K + 1) / 2;
-    const double* mb = mom + (size_t)b * NP;
-    double wc[kMaxK], m[kMaxK];
+__global__ __launch_bounds__(1024) void conv0_finalize_kernel(const double* __restrict__ part, int nchunk,
+                                                              const float* __restrict__ w,
+                                                              const float* __restrict__ bias, int C, int K, int T0,
+                                                              const float* __restrict__ gamma,
+                                                              const float* __restrict__ beta, float eps,
+                                                              float* __restrict__ scale, float* __restrict__ shift) {
+    __shared__ double ps[kMomSlices][kMomMax], mb[kMomMax];
+    const int NP = K + K * (K + 1) / 2, tid = threadIdx.x, b = blockIdx.y;
+    const int sl = tid / NP, p = tid - sl * NP;
+    if (sl < kMomSlices) {
+        const double* pb = part + (size_t)b * nchunk * NP + p;
+        double s = 0.0;
+#pragma unroll 8   // eight chunks' loads in flight; the sum keeps its order
+        for (int j = sl; j < nchunk; j += kMomSlices) s += pb[(size_t)j * NP];
+        ps[sl][p] = s;
+    }
+    __syncthreads();
+    if (tid < NP) {
+        double s = 0.0;
+#pragma unroll
+        for (int i = 0; i < kMomSlices; ++i) s += ps[i][tid];
+        mb[tid] = s / T0;
+    }
+    __syncthreads();
+    const int c = blockIdx.x * 256 + tid;
+    if (tid >= 256 || c >= C) return;
+    double wc[kMaxK];
     double mean = bias ? (double)bias[c] : 0.0;
     for (int k = 0; k < K; ++k) {
         wc[k] = (double)w[c * K + k];
-        m[k] = mb[k] / T0;
-        mean += wc[k] * m[k];
+        mean += wc[k] * mb[k];
     }
     double var = 0.0;
     int q = K;
     for (int k1 = 0; k1 < K; ++k1)
         for (int k2 = k1; k2 < K; ++k2, ++q) {
-            const double cov = mb[q] / T0 - m[k1] * m[k2];
+            const double cov = mb[q] - mb[k1] * mb[k2];
             var += (k1 == k2 ? 1.0 : 2.0) * wc[k1] * wc[k2] * cov;
         }
     var = var > 0.0 ? var : 0.0;
@@ -166,7 +180,8 @@ __global__ __launch_bounds__(256) void conv0_finalize_kernel(const double* __res
 // holds their KT taps (zero past K) in registers.  A workgroup covers
 // kApplyFrames frames of one clip: the waveform window and the weights
 // (staged through LDS as [K][C] so every global read is coalesced) are loaded
-// once per workgroup.  norm 0: none; 1: GroupNorm affine from scale/shift
+// once per workgroup.  kApplyFrames is the most a workgroup takes; small
+// batches take fewer (frames), for enough workgroups to fill the chip.  norm 0: none; 1: GroupNorm affine from scale/shift
 // [B][C]; 2: LayerNorm over the frame's C channels (gamma, beta, eps).  Then
 // GELU, stored f16.
 constexpr int kApplyFrames = 256;
@@ -180,13 +195,13 @@ __global__ __launch_bounds__(256) void conv0_apply_kernel(const float* __restric
                                                           const float* __restrict__ scale,
                                                           const float* __restrict__ shift,
                                                           const float* __restrict__ gamma,
-                                                          const float* __restrict__ beta, float eps,
+                                                          const float* __restrict__ beta, float eps, int frames,
                                                           half_t* __restrict__ y) {
     constexpr int C = CPL * 64;
     __shared__ float sx[kApplyWin];
     __shared__ __attribute__((aligned(16))) float sw[KT * C];   // [tap][channel]
-    const int b = blockIdx.y, t0 = blockIdx.x * kApplyFrames;
-    const int nt = T0 - t0 < kApplyFrames ? T0 - t0 : kApplyFrames;
+    const int b = blockIdx.y, t0 = blockIdx.x * frames;
+    const int nt = T0 - t0 < frames ? T0 - t0 : frames;
     const int len = (nt - 1) * S + K;
     load_window(x, n, wstats, b, t0 * S, len, sx);
     for (int i = len + threadIdx.x; i < (nt - 1) * S + KT; i += 256) sx[i] = 0.0f;   // taps K..KT-1
@@ -258,13 +273,13 @@ __global__ __launch_bounds__(256) void conv0_apply_kernel(const float* __restric
 template <int CPL>
 void launch_conv0_apply(dim3 g, hipStream_t s, const float* x, int n, const float* wstats, const float* w,
                         const float* bias, int K, int S, int T0, int norm, const float* scale, const float* shift,
-                        const float* gamma, const float* beta, float eps, half_t* y) {
+                        const float* gamma, const float* beta, float eps, int frames, half_t* y) {
     if (K == 10)
         hipLaunchKernelGGL((conv0_apply_kernel<CPL, 10>), g, dim3(256), 0, s, x, n, wstats, w, bias, K, S, T0, norm,
-                           scale, shift, gamma, beta, eps, y);
+                           scale, shift, gamma, beta, eps, frames, y);
     else
         hipLaunchKernelGGL((conv0_apply_kernel<CPL, kMaxK>), g, dim3(256), 0, s, x, n, wstats, w, bias, K, S, T0,
-                           norm, scale, shift, gamma, beta, eps, y);
+                           norm, scale, shift, gamma, beta, eps, frames, y);
 }
 
 // ---- LayerNorm over rows of C (one wave per row, lane l owns elements
@@ -656,6 +671,86 @@ __global__ __launch_bounds__(192) void pos_conv_kernel(const half_t* __restrict_
     }
 }
 
+// The same conv for launches whose 192-frame workgroups are few: a workgroup
+// takes 32 frames x 64 outputs (two waves, one 32-output block each) and
+// streams the weights eight taps at a time through a two-stage LDS ring by DMA
+// (rows of 8 * ICG halfs, 16-byte chunks XOR-swizzled by row within groups of
+// 16), so there is one barrier per eight taps instead of one per tap.  The
+// same sums in the same order.
+constexpr int kPosST = 32, kPosTaps = 8;
+
+template <int ICG>
+__global__ __launch_bounds__(128) void pos_conv_small_kernel(const half_t* __restrict__ x, const half_t* __restrict__ w,
+                                                             const float* __restrict__ bias, float* __restrict__ y,
+                                                             int T, int H, int K, int pad) {
+    constexpr int RS = ICG + 8, CH = ICG / 8;
+    constexpr int WCH = kPosTaps * CH;          // 16-byte chunks per weight row and stage (a multiple of 16)
+    constexpr int STAGE = 64 * WCH * 16;
+    static_assert(WCH % 16 == 0, "whole swizzle groups");
+    __shared__ __attribute__((aligned(1024))) uint8_t sw[2][STAGE];
+    __shared__ __attribute__((aligned(16))) half_t sx[(kPosST + kPosMaxK - 1) * RS];
+    const int b = blockIdx.z, g = blockIdx.y, t0 = blockIdx.x * kPosST;
+    const int tid = threadIdx.x, lane = tid & 63, lr = lane & 31, hl = lane >> 5;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const size_t cb = (size_t)g * ICG;
+    const half8 zero8 = {0, 0, 0, 0, 0, 0, 0, 0};
+    const int4v wrs = dma_rsrc(w + (size_t)g * 64 * K * ICG, (uint32_t)(64 * K * ICG * 2));
+    // 64 rows * WCH chunks = WCH instructions; taps past K read on into the next
+    // row (or zeros past the last) and are not used
+    uint32_t off[WCH / 2];
+#pragma unroll
+    for (int i = 0; i < WCH / 2; ++i) {
+        const int s = (wave + 2 * i) * 64 + lane, r = s / WCH, pos = s - r * WCH;
+        off[i] = (uint32_t)((r * K * ICG + ((pos & ~15) | ((pos ^ r) & 15)) * 8) * 2);
+    }
+    auto issue = [&](int st, int k0) {
+#pragma unroll
+        for (int i = 0; i < WCH / 2; ++i)
+            dma16(sw[st] + (wave + 2 * i) * 1024, wrs, off[i] + (uint32_t)(k0 * ICG * 2));
+    };
+    issue(0, 0);
+    const int rows = kPosST + K - 1;
+    for (int i = tid; i < rows * CH; i += 128) {
+        const int r = i / CH, c = i - r * CH, f = t0 - pad + r;
+        const half8 v = (f >= 0 && f < T) ? *reinterpret_cast<const half8*>(x + ((size_t)b * T + f) * H + cb + c * 8)
+                                          : zero8;
+        *reinterpret_cast<half8*>(&sx[r * RS + c * 8]) = v;
+    }
+    float16v acc;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) acc[r] = 0.0f;
+    const int o = 32 * wave + lr;   // this lane's B row (output)
+    for (int k0 = 0, st = 0; k0 < K; k0 += kPosTaps, st ^= 1) {
+        wait_vmcnt<0>();            // this wave's share of the stage (issued one stage ago)
+        lds_barrier();              // everyone's; the other stage's reads are done
+        if (k0 + kPosTaps < K) issue(st ^ 1, k0 + kPosTaps);
+        const uint8_t* const wr = sw[st] + o * WCH * 16;
+#pragma unroll
+        for (int k = 0; k < kPosTaps; ++k) {
+            if (k0 + k >= K) break;
+            half8 a[CH / 2], bw[CH / 2];
+#pragma unroll
+            for (int kk = 0; kk < CH / 2; ++kk) {
+                const int c = k * CH + 2 * kk + hl;
+                a[kk] = *reinterpret_cast<const half8*>(&sx[(lr + k0 + k) * RS + 16 * kk + 8 * hl]);
+                bw[kk] = *reinterpret_cast<const half8*>(wr + ((c & ~15) | ((c ^ o) & 15)) * 16);
+            }
+#pragma unroll
+            for (int kk = 0; kk < CH / 2; ++kk)
+                acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[kk], bw[kk], acc, 0, 0, 0);
+        }
+    }
+    if (o >= ICG) return;
+    const float bo = bias[cb + o];
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+        const int t = t0 + 8 * (r >> 2) + 4 * hl + (r & 3);
+        if (t >= T) continue;
+        const size_t i = ((size_t)b * T + t) * H + cb + o;
+        y[i] = (float)x[i] + gelu_erf(acc[r] + bo);
+    }
+}
+
 // ---- per-clip mean over time: out[b][c] = [out +] w * mean_t x[b][t][c] ----
 // A workgroup covers 256 channels of one clip: 64 lanes x 4 channels (one
 // 8- or 16-byte load per row) x 16 time partitions, f64 sums combined in a
@@ -697,13 +792,62 @@ __global__ __launch_bounds__(1024) void time_mean_kernel(const void* __restrict_
     }
 }
 
+// ---- the weighted sum of several states' means over time in one launch:
+// out[b][c] = sum_i w_i * mean_t x_i[b][t][c], states x_i (f16) `state` elements
+// apart, in the order of one vdk_time_mean_acc call per state.  A workgroup
+// covers 32 channels of one clip; a wave takes whole states (8 lanes x 4
+// channels x 8 time partitions).  The f64 sums of f16 values (multiples of
+// 2^-24 below 2^16) are exact, so their order is free and the means are
+// time_mean_kernel's.  (13 launches over 159 frames of 768 channels took 74 us,
+// most of it the launches.)
+constexpr int kMeanStates = 32;
+struct StateWeights {
+    float w[kMeanStates];
+};
+
+__global__ __launch_bounds__(1024) void time_mean_states_kernel(const half_t* __restrict__ x, size_t state, int n, int T,
+                                                                int C, StateWeights sw, float* __restrict__ out) {
+    __shared__ float sm[kMeanStates][32];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, cg = lane & 7;
+    const int c = blockIdx.x * 32 + cg * 4, b = blockIdx.y;
+    for (int i = wave; i < n; i += 16) {
+        double s[4] = {0.0, 0.0, 0.0, 0.0};
+        if (c < C && sw.w[i] != 0.0f) {
+            const half_t* const xi = x + i * state + (size_t)b * T * C + c;
+#pragma unroll 8
+            for (int t = lane >> 3; t < T; t += 8) {
+                const half4 v = *reinterpret_cast<const half4*>(xi + (size_t)t * C);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) s[e] += (double)(float)v[e];
+            }
+        }
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+#pragma unroll
+            for (int m = 8; m < 64; m <<= 1) s[e] += __shfl_xor(s[e], m, 64);
+            if (lane < 8) sm[i][cg * 4 + e] = (float)(s[e] / T);
+        }
+    }
+    __syncthreads();
+    const int cc = blockIdx.x * 32 + threadIdx.x;
+    if (threadIdx.x >= 32 || cc >= C) return;
+    float acc = 0.0f;
+    bool any = false;
+    for (int i = 0; i < n; ++i) {
+        if (sw.w[i] == 0.0f) continue;
+        acc = any ? acc + sw.w[i] * sm[i][threadIdx.x] : sw.w[i] * sm[i][threadIdx.x];
+        any = true;
+    }
+    out[(size_t)b * C + cc] = acc;
+}
+
 bool al16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
 
 int conv0_frames(int n, int K, int S) { return n < K ? 0 : (n - K) / S + 1; }
 
 size_t conv0_work(int batch, int n, int C, int K, int S) {
-    // per-chunk moment partials [B][nchunk][NP] and sums [B][NP] f64
-    // (NP = K + K(K+1)/2), then scale / shift [B][C] f32
+    // per-chunk moment partials [B][nchunk][NP] f64 (NP = K + K(K+1)/2), then
+    // scale / shift [B][C] f32 (the size leaves NP f64 per clip to spare)
     const size_t np = (size_t)K + (size_t)K * (K + 1) / 2;
     const size_t nchunk = (size_t)(conv0_frames(n, K, S) + kFrames - 1) / kFrames;
     return (size_t)batch * (np * 8 * (nchunk + 1) + (size_t)C * 8) + 256;
@@ -752,34 +896,35 @@ extern "C" int vdk_w2v2_conv0(const float* d_x, int batch, int n, const float* d
             const int NP = K + K * (K + 1) / 2;
             const int nchunk = (T0 + kFrames - 1) / kFrames;
             double* part = static_cast<double*>(d_work);
-            double* mom = part + (size_t)batch * nchunk * NP;
-            float* sc = reinterpret_cast<float*>(mom + (size_t)batch * NP);
+            float* sc = reinterpret_cast<float*>(part + (size_t)batch * nchunk * NP);
             float* sh = sc + (size_t)batch * C;
             hipLaunchKernelGGL(conv0_moments_kernel, dim3(nchunk, batch), dim3(256), 0, s, d_x, n, d_stats, K, S, T0,
                                part);
             VDK_HIP(hipGetLastError());
-            hipLaunchKernelGGL(conv0_moments_reduce_kernel, dim3(batch), dim3(256), 0, s, part, nchunk, NP, mom);
-            VDK_HIP(hipGetLastError());
-            hipLaunchKernelGGL(conv0_finalize_kernel, dim3(cdiv(C, 256), batch), dim3(256), 0, s, mom, d_w, d_bias,
-                               C, K, T0, d_gamma, d_beta, eps, sc, sh);
+            hipLaunchKernelGGL(conv0_finalize_kernel, dim3(cdiv(C, 256), batch), dim3(1024), 0, s, part, nchunk, d_w,
+                               d_bias, C, K, T0, d_gamma, d_beta, eps, sc, sh);
             VDK_HIP(hipGetLastError());
             scale = sc;
             shift = sh;
         }
         half_t* y = static_cast<half_t*>(d_y);
-        const dim3 g(cdiv(T0, kApplyFrames), batch);
+        // 256 frames a workgroup, halved down to 32 while that leaves fewer than
+        // 512 workgroups (one 3.2 s clip: 40 workgroups 45 us, 320 10 us)
+        int frames = kApplyFrames;
+        while (frames > 32 && (long)batch * cdiv(T0, frames) < 512) frames /= 2;
+        const dim3 g(cdiv(T0, frames), batch);
         switch (C) {
             case 256:
                 launch_conv0_apply<4>(g, s, d_x, n, d_stats, d_w, d_bias, K, S, T0, norm, scale, shift, d_gamma,
-                                      d_beta, eps, y);
+                                      d_beta, eps, frames, y);
                 break;
             case 512:
                 launch_conv0_apply<8>(g, s, d_x, n, d_stats, d_w, d_bias, K, S, T0, norm, scale, shift, d_gamma,
-                                      d_beta, eps, y);
+                                      d_beta, eps, frames, y);
                 break;
             default:
                 launch_conv0_apply<16>(g, s, d_x, n, d_stats, d_w, d_bias, K, S, T0, norm, scale, shift, d_gamma,
-                                       d_beta, eps, y);
+                                       d_beta, eps, frames, y);
                 break;
         }
         VDK_HIP(hipGetLastError());
@@ -875,6 +1020,24 @@ extern "C" int vdk_time_mean(const void* d_x, int x_f32, int batch, int T, int C
     });
 }
 
+extern "C" int vdk_time_mean_states(const void* d_x, size_t state_stride, int n_states, int batch, int T, int C,
+                                    const float* weights, float* d_out, void* stream) {
+    return guarded([&] {
+        require(d_x && d_out && weights, "time_mean_states: NULL pointer");
+        require(batch > 0 && batch <= 65535 && T > 0 && C > 0 && C % 4 == 0,
+                "time_mean_states: C must be a positive multiple of 4");
+        require(n_states > 0 && n_states <= kMeanStates, "time_mean_states: 1 .. 32 states");
+        require(al16(d_x) && state_stride % 8 == 0 && state_stride >= (size_t)batch * T * C,
+                "time_mean_states: states must be 16-byte aligned and apart");
+        StateWeights sw{};
+        for (int i = 0; i < n_states; ++i) sw.w[i] = weights[i];
+        hipLaunchKernelGGL(time_mean_states_kernel, dim3(cdiv(C, 32), batch), dim3(1024), 0,
+                           static_cast<hipStream_t>(stream), static_cast<const half_t*>(d_x), state_stride, n_states, T,
+                           C, sw, d_out);
+        VDK_HIP(hipGetLastError());
+    });
+}
+
 extern "C" int vdk_pos_conv(const void* d_x, int batch, int T, int H, int groups, const void* d_w, const float* d_bias,
                             int K, int pad, float* d_y, void* stream) {
     return guarded([&] {
@@ -886,11 +1049,18 @@ extern "C" int vdk_pos_conv(const void* d_x, int batch, int T, int H, int groups
         require(al16(d_x) && al16(d_w), "pos_conv: buffers must be 16-byte aligned");
         require((size_t)batch * T * H < (1ull << 31), "pos_conv: too many frames for one launch");
         require(batch <= 65535 && groups <= 65535, "pos_conv: grid too large");
-        const dim3 grid(cdiv(T, kPosTT), groups, batch);
+        const dim3 grid(cdiv(T, kPosTT), groups, batch), fine(cdiv(T, kPosST), groups, batch);
         hipStream_t s = static_cast<hipStream_t>(stream);
+        // one round of the 32-frame workgroups (one 3.2 s clip 70 -> 27 us); four clips
+        // of 3 s and more are no faster on them
+        const bool small = (long)fine.x * groups * batch <= 256;
         const half_t* x = static_cast<const half_t*>(d_x);
         const half_t* w = static_cast<const half_t*>(d_w);
-        if (icg == 48)
+        if (small && icg == 48)
+            hipLaunchKernelGGL(pos_conv_small_kernel<48>, fine, dim3(128), 0, s, x, w, d_bias, d_y, T, H, K, pad);
+        else if (small)
+            hipLaunchKernelGGL(pos_conv_small_kernel<64>, fine, dim3(128), 0, s, x, w, d_bias, d_y, T, H, K, pad);
+        else if (icg == 48)
             hipLaunchKernelGGL(pos_conv_kernel<48>, grid, dim3(192), 0, s, x, w, d_bias, d_y, T, H, K, pad);
         else
             hipLaunchKernelGGL(pos_conv_kernel<64>, grid, dim3(192), 0, s, x, w, d_bias, d_y, T, H, K, pad);

@@ -139,6 +139,8 @@ _SIGS = {
     "vdk_layer_norm": (C.c_int, [_vp, C.c_int, C.c_int, _vp, _vp, C.c_float, C.c_int, _vp, _vp, C.c_float, _vp]),
     "vdk_attention": (C.c_int, [_vp, C.c_int, C.c_int, C.c_int, C.c_int, C.c_float, _vp, _vp]),
     "vdk_time_mean": (C.c_int, [_vp, C.c_int, C.c_int, C.c_int, C.c_int, _vp, _vp]),
+    "vdk_time_mean_states": (C.c_int, [_vp, C.c_size_t, C.c_int, C.c_int, C.c_int, C.c_int, C.POINTER(C.c_float), _vp,
+                                       _vp]),
     "vdk_time_mean_acc": (C.c_int, [_vp, C.c_int, C.c_int, C.c_int, C.c_int, C.c_float, C.c_int, _vp, _vp]),
     "vdk_pos_conv": (C.c_int, [_vp, C.c_int, C.c_int, C.c_int, C.c_int, _vp, _vp, C.c_int, C.c_int, _vp, _vp]),
     "vdk_resblock3x3": (C.c_int, [_vp, C.c_int, C.c_int, C.c_int, C.c_int, _vp, _vp, _vp, _vp, _vp, _vp]),
