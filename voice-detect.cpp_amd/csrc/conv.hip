@@ -2486,7 +2486,9 @@ __device__ __forceinline__ int div_small(int n, float inv_d) {
     return (int)(((float)n + 0.5f) * inv_d);
 }
 
-template <int TH, int MAXW, int WMG, int WNG, int NJ, int NP>
+// SEG: maps of several column segments (one segment: the arithmetic of the
+// columns compiles away, 3 % of the 5-row bands at batch 64)
+template <int TH, int MAXW, int WMG, int WNG, int NJ, int NP, bool SEG>
 __global__ __launch_bounds__((WMG * WNG + NP) * 64) void conv3x3_bandws_kernel(ConvArgs a) {
     using G = BandWsTile<TH, MAXW, WMG, WNG, NJ, NP>;
     constexpr int MI = G::MI;
@@ -2500,9 +2502,9 @@ __global__ __launch_bounds__((WMG * WNG + NP) * 64) void conv3x3_bandws_kernel(C
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     // the workgroup's rows r0 .. r0 + TH - 1, columns cs .. cs + W - 1 (W: the
     // segment's width) of clip b
-    const int H = a.H, FW = a.W, W = (FW + a.nseg - 1) / a.nseg, IC = a.IC, HW = W + 2;
+    const int H = a.H, FW = a.W, W = SEG ? (FW + a.nseg - 1) / a.nseg : FW, IC = a.IC, HW = W + 2;
     const int bands = (H + TH - 1) / TH;
-    const int bb = blockIdx.x / a.nseg, cs = (blockIdx.x - bb * a.nseg) * W;
+    const int bb = SEG ? blockIdx.x / a.nseg : blockIdx.x, cs = SEG ? (blockIdx.x - bb * a.nseg) * W : 0;
     const int b = bb / bands, r0 = (bb - b * bands) * TH;
     const int oc0 = blockIdx.y * G::OCB;
     const int npx = TH * W;                           // band pixels (rows past H are computed and dropped)
@@ -2563,7 +2565,7 @@ __global__ __launch_bounds__((WMG * WNG + NP) * 64) void conv3x3_bandws_kernel(C
                     const int sl = ri * 64 + lane;
                     const int pr = half * G::HALF_ROWS + sl / G::SPR, ch = sl % G::SPR;
                     const int r = div_small(pr, inv_w), c = pr - r * W;
-                    const bool ok = ch < 16 && pr < npx && r0 + r < H && cs + c < FW;
+                    const bool ok = ch < 16 && pr < npx && r0 + r < H && (!SEG || cs + c < FW);
                     const uint32_t off =
                         ok ? (uint32_t)(((((size_t)(b * H + r0 + r) * FW + cs + c) * a.rs + oc0) * 2) + ch * 16) : kOOB;
                     __builtin_amdgcn_raw_ptr_buffer_load_lds(rr, (lds_void*)(dst + ri * 1024), 16, off, 0, 0, 0);
@@ -2712,7 +2714,7 @@ __global__ __launch_bounds__((WMG * WNG + NP) * 64) void conv3x3_bandws_kernel(C
         const int pr = pg * NJ * 32 + (it * 64 + lane) / G::CPR;
         const half8 v8 = *reinterpret_cast<const half8*>(rrow(pr) + cg0 * 2 + ch * 16);
         const int r = div_small(pr, inv_w), c = pr - r * W;
-        if (pr < npx && r0 + r < H && cs + c < FW)
+        if (pr < npx && r0 + r < H && (!SEG || cs + c < FW))
             *reinterpret_cast<half8*>(y + ((size_t)(b * H + r0 + r) * FW + cs + c) * a.ys + ch * 8) = v8;
     }
 }
@@ -2722,8 +2724,11 @@ void launch_bandws(const ConvArgs& args, hipStream_t s) {
     ConvArgs a = args;
     a.nseg = cdiv(a.W, MAXW);
     const int B = a.npix / (a.Ho * a.Wo);
-    hipLaunchKernelGGL((conv3x3_bandws_kernel<TH, MAXW, WMG, WNG, NJ, NP>), dim3(B * cdiv(a.H, TH) * a.nseg, a.OC / 128),
-                       dim3((WMG * WNG + NP) * 64), 0, s, a);
+    const dim3 grid(B * cdiv(a.H, TH) * a.nseg, a.OC / 128), block((WMG * WNG + NP) * 64);
+    if (a.nseg == 1)
+        hipLaunchKernelGGL((conv3x3_bandws_kernel<TH, MAXW, WMG, WNG, NJ, NP, false>), grid, block, 0, s, a);
+    else
+        hipLaunchKernelGGL((conv3x3_bandws_kernel<TH, MAXW, WMG, WNG, NJ, NP, true>), grid, block, 0, s, a);
 }
 
 
@@ -3141,7 +3146,7 @@ int pick_small_tile(const ConvArgs& a) {
     if (w32 <= 256) t = c128 ? 92 : (c64 ? 93 : 94);
     else if (a.in_scale || a.segsum) {   // CAM++'s linear1 / transits
         if (c128 && w64 <= 256 && a.OC > 128) t = 96;
-        else if (w32 <= 512) t = c128 ? 92 : (c64 ? 93 : 94);
+        else if (w32 <= 512) t = c64 ? 93 : 87;   // (16 x 249 frames, 256 / 608 -> 128: 10.8 / 14.3 us; 92: 15.0)
         else if (c64 && w64 <= 256) t = c128 ? 96 : 98;
     } else if (!c64 || a.OC % 64 != 0) {
         // narrow outputs and 32-channel chunks
@@ -3213,26 +3218,21 @@ int pick_tile(const ConvArgs& a) {
     const int small = pick_small_tile(a);
     if (small >= 0) return small;
     const int bm = a.OC % 128 == 0 ? 128 : (a.OC % 64 == 0 ? 64 : 32);
-    if (a.in_scale) {   // register-staged tiles for a few ten thousand pixels (CAM++'s
-        // linear1: the LDS-DMA tiles, faster in isolation, measured slower in the model):
-        // 64-channel chunks from 256 input channels (half the chunk steps, each a
-        // load round trip) on the 64x64 tile (B=32 x 499 frames: 12.8 / 16.6 /
-        // 19.9 -> 12.0 / 15.8 / 19.5 us at 256 / 512 / 768 channels against the
-        // 128x64 one), else the 64x64 tile with 32-channel chunks
-        // the GEMM kernel's narrow tiles from 800 channels (B=32 x 499 frames,
-        // interleaved: 800 22.5 -> 21.2 us, 1024 23.5 -> 22.1 us)
+    if (a.in_scale) {
         // CAM++'s 1024 -> 512 transits (B=32 x 499 frames): the GEMM kernel's
-        // 256x128 prologue tile, 55.5 -> 31.8 us (512 -> 256: no gain)
-        if (a.KH * a.KW == 1 && a.IC >= 1024 && a.OC >= 512 && a.OC % 256 == 0 && !a.segsum &&
-            tile_fits(kTiles[90], a))
-            return 90;
+        // 256x128 prologue tile, 55.5 -> 31.8 us (512 -> 256: no gain); up to
+        // one round of them the 128x64 one (16 x 249 frames: 28.4 -> 17.6 us)
+        if (a.KH * a.KW == 1 && a.IC >= 1024 && a.OC >= 512 && a.OC % 256 == 0 && !a.segsum) {
+            if ((long)cdiv(a.npix, 64) * (a.OC / 128) <= 256 && tile_fits(kTiles[86], a)) return 86;
+            if (tile_fits(kTiles[90], a)) return 90;
+        }
         // the 512 -> 256 transit on the 128x64 LDS-DMA tile (in-model: 21.3 -> 16.8 us)
         if (a.KH * a.KW == 1 && a.IC == 512 && a.OC == 256 && !a.segsum && tile_fits(kTiles[18], a)) return 18;
-        if (a.IC >= 800 && a.OC == 128 && a.npix < 65536) {
-            if (a.IC % 64 == 0 && tile_fits(kTiles[86], a)) return 86;
-            if (tile_fits(kTiles[85], a)) return 85;
-        }
-        if (a.IC >= 256 && a.IC % 64 == 0 && a.OC == 128 && a.npix < 65536 && tile_fits(kTiles[80], a)) return 80;
+        // linear1 (128 .. 992 -> 128 with the segment sums) on the GEMM kernel's
+        // 128x64 tile (B=32 x 499 frames, launches of 4.5 us included: 12.2 ->
+        // 11.8 us at 128 channels, 19.0 -> 16.2 at 576, 23.0 -> 17.7 at 736
+        // against the register-staged 64x64 tiles)
+        if (a.OC == 128 && a.npix < 65536 && tile_fits(kTiles[85], a)) return 85;
         if (a.IC % 32 == 0) return bm >= 64 ? (a.npix < 32768 ? 63 : (bm == 128 ? 5 : 2)) : 10;
         return bm == 128 ? 13 : (bm == 64 ? 12 : 11);
     }
