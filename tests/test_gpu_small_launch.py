@@ -279,3 +279,46 @@ def test_time_mean_states_equals_one_by_one(n, B, T, C):
             first = False
     lib.check(L.vdk_synchronize())
     assert np.array_equal(do.to_array(np.uint32, (B, C)), dr.to_array(np.uint32, (B, C)))
+
+
+@pytest.mark.parametrize("B,H,W,IC,OC,split,groups", [(2, 10, 91, 128, 128, 2, False), (1, 10, 33, 128, 128, 1, False),
+                                                      (1, 20, 50, 64, 64, 2, False), (1, 1, 1, 64, 32, 2, False),
+                                                      (1, 13, 37, 32, 32, 2, True), (1, 7, 45, 32, 64, 1, False)])
+def test_slim_split_bitwise(B, H, W, IC, OC, split, groups):
+    """Split-f16 stride-1 3x3 convs on 32 x 32 tiles: the halo kernel's bits (or
+    the register-weight kernel's, where the channel groups need it), the
+    default's, and f64 to split-f16's accuracy."""
+    rng = np.random.default_rng(B + H + W + IC + OC)
+    announce(f"slim split B={B} H={H} W={W} {IC}->{OC} split={split} groups={groups}")
+    x = rng.standard_normal((B, H, W, IC)).astype(np.float32)
+    w = (rng.standard_normal((OC, 3, 3, IC)) * np.sqrt(2.0 / (9 * IC))).astype(np.float32)
+    if split == 2:
+        w = w.astype(np.float16).astype(np.float32)
+
+    def halves(v):
+        hi = v.astype(np.float16)
+        return hi, (v - hi.astype(np.float32)).astype(np.float16)
+
+    wh, wl = halves(w)
+    bias = rng.uniform(-0.5, 0.5, OC).astype(np.float32)
+    keep = [lib.DeviceBuffer.from_array(np.ascontiguousarray(v)) for v in
+            (np.concatenate(halves(x), axis=3), np.concatenate([wh, wh] if split == 2 else [wh, wh, wl], axis=3), bias)]
+    d = lib.ConvDesc()
+    d.x, d.batch, d.H, d.W, d.IC, d.x_stride, d.x_lo = keep[0].ptr, B, H, W, IC, 2 * IC, IC
+    d.w, d.OC, d.KH, d.KW = keep[1].ptr, OC, 3, 3
+    d.stride_h = d.stride_w = d.pad_h = d.pad_w = d.dil_h = d.dil_w = 1
+    d.bias, d.act, d.clamp_hi, d.split = keep[2].ptr, lib.ACT_RELU, 20.0, split
+    if groups:   # one 32-channel group, its lo half inside the group stride
+        d.x_group, d.x_group_stride, d.y_group, d.y_group_stride = 32, 64, 32, 64
+    dy = lib.DeviceBuffer(B * H * W * 2 * OC * 2)
+    d.y, d.y_stride, d.y_lo = dy.ptr, 2 * OC, OC
+    outs = run_tiles(d, dy, (B, H, W, 2 * OC), [-1, 26, 28, 30, 72, 74, 75, 109])
+    assert 109 in outs and len(outs) >= 3, sorted(outs)
+    for t, o in outs.items():
+        assert np.array_equal(o, outs[109]), f"tile {t}"
+    o = outs[109].view(np.float16).astype(np.float64)
+    got = o[..., :OC] + o[..., OC:]
+    want = np.stack([O.conv2d_g(x[c].transpose(2, 0, 1), np.ascontiguousarray(w.transpose(0, 3, 1, 2)), ph=1, pw=1,
+                                bias=bias, f64=True) for c in range(B)])
+    want = np.clip(want, 0, 20)
+    assert np.abs(got.transpose(0, 3, 1, 2) - want).max() <= 2e-6 * max(np.abs(want).max(), 1.0)

@@ -2875,6 +2875,117 @@ void launch_slim(const ConvArgs& a, hipStream_t s) {
     hipLaunchKernelGGL(conv3x3_slim_kernel, dim3(cdiv(a.npix, 32), a.OC / 32), dim3(192), 0, s, a);
 }
 
+// ---------------------------------------------------------------------------
+// conv3x3_slim_split_kernel: the halo kernel's stride-1 3x3 conv on split-f16
+// maps (any epilogue) for launches that leave most of the chip idle: the slim
+// kernel's 32 channels x 32 pixels per workgroup, with stages of 32 channels
+// of one plane term x 9 taps (rows of 64 bytes, swizzled as in the GEMM
+// kernels; two producer waves for the weights, two for the pixels).  The sums
+// run in the halo kernel's order (plane terms, 32-channel chunks, taps,
+// 16-channel steps), so the results are the same bits.
+// ---------------------------------------------------------------------------
+__global__ __launch_bounds__(320) void conv3x3_slim_split_kernel(ConvArgs a) {
+    constexpr int NST = 2, STAGE = 36 * 1024;   // 72 KB: two workgroups per CU (4 stages no faster alone, slower past 256)
+    __shared__ __attribute__((aligned(1024))) uint8_t smem[NST * STAGE];
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    int ptile, otile;
+    tile_ids(a, ptile, otile);
+    const int p0 = ptile * 32, oc0 = otile * 32;
+    const int H = a.H, W = a.W, IC = a.IC, icw = (a.split == 2 ? 2 : 3) * IC, nk = icw / 32;
+
+    if (wave > 0) {
+        // ---------------- producers: waves 1, 2 weights, 3, 4 pixels ----------------
+        // instruction i of a pair's wave h: 16 rows (h * 16 ..) of tap i
+        const int h = (wave - 1) & 1, row = h * 16 + (lane >> 2), c = swz<32>(row, lane & 3);
+        const bool wts = wave <= 2;
+        uint32_t off[9];
+#pragma unroll
+        for (int t = 0; t < 9; ++t) off[t] = kOOB;
+        if (wts) {
+            if (oc0 + row < a.OC) {
+#pragma unroll
+                for (int t = 0; t < 9; ++t) off[t] = (uint32_t)((((oc0 + row) * 9 + t) * icw + c * 8) * 2);
+            }
+        } else if (p0 + row < a.npix) {
+            const int P = p0 + row, b = P / (H * W), rem = P - b * (H * W), ih0 = rem / W, iw0 = rem - ih0 * W;
+#pragma unroll
+            for (int t = 0; t < 9; ++t) {
+                const int ih = ih0 + t / 3 - 1, iw = iw0 + t % 3 - 1;
+                if (ih >= 0 && ih < H && iw >= 0 && iw < W)
+                    off[t] = (uint32_t)((((b * H + ih) * W + iw) * a.xs + chan_off(c * 8, a.xgl, a.xgs)) * 2);
+            }
+        }
+        const int xext = ((IC >> a.xgl) - 1) * a.xgs + (1 << a.xgl);
+        const __amdgpu_buffer_rsrc_t rs =
+            wts ? __builtin_amdgcn_make_buffer_rsrc((void*)a.w, 0, (int)((size_t)a.OC * 9 * icw * 2), 0x00020000)
+                : __builtin_amdgcn_make_buffer_rsrc((void*)a.x, 0,
+                                                    (int)(((size_t)(a.npix_in - 1) * a.xs + xext + a.x_lo) * 2), 0x00020000);
+        uint8_t* const dst0 = smem + (wts ? 0 : 18 * 1024) + h * 1024;
+        auto issue = [&](int k) {
+            const int c0 = k * 32, term = c0 >= 2 * IC ? 2 : (c0 >= IC ? 1 : 0);
+            const uint32_t ko =
+                (uint32_t)((wts ? c0 : (term == 1 ? a.x_lo : 0) + chan_off(c0 - term * IC, a.xgl, a.xgs)) * 2);
+#pragma unroll
+            for (int t = 0; t < 9; ++t) {
+                const uint32_t o = off[t] == kOOB ? kOOB : off[t] + ko;
+                __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (lds_void*)(dst0 + (k % NST) * STAGE + t * 2048), 16, o, 0, 0,
+                                                         0);
+            }
+        };
+#pragma unroll
+        for (int k = 0; k < NST - 1; ++k)
+            if (k < nk) issue(k);
+#pragma unroll 1
+        for (int k = 0; k < nk; ++k) {
+            wait_vmcnt_le((nk - 1 - k < NST - 2 ? nk - 1 - k : NST - 2) * 9);   // chunk k has landed
+            lds_barrier();   // chunk k is visible; the compute wave is done with chunk k-1's stage
+            if (k + NST - 1 < nk) issue(k + NST - 1);
+        }
+        return;
+    }
+
+    // ---------------- compute wave ----------------
+    const int lrow = lane & 31, lhalf = lane >> 5;
+    float16v acc;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) acc[r] = 0.0f;
+    int fo[2];
+#pragma unroll
+    for (int kk = 0; kk < 2; ++kk) fo[kk] = lrow * 64 + swz<32>(lrow, kk * 2 + lhalf) * 16;
+#pragma unroll 1
+    for (int k = 0; k < nk; ++k) {
+        lds_barrier();   // chunk k has landed
+        const uint8_t* const st = smem + (k % NST) * STAGE;
+        half8 af[9][2], bf[9][2];
+#pragma unroll
+        for (int t = 0; t < 9; ++t)
+#pragma unroll
+            for (int kk = 0; kk < 2; ++kk) {
+                af[t][kk] = *reinterpret_cast<const half8*>(st + t * 2048 + fo[kk]);
+                bf[t][kk] = *reinterpret_cast<const half8*>(st + 18 * 1024 + t * 2048 + fo[kk]);
+            }
+#pragma unroll
+        for (int t = 0; t < 9; ++t)
+#pragma unroll
+            for (int kk = 0; kk < 2; ++kk)
+                acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[t][kk], bf[t][kk], acc, 0, 0, 0);
+    }
+    // every chunk has landed and been read (by this wave alone): stage through LDS
+    float* const sT = reinterpret_cast<float*>(smem);
+    stage_block(sT, 36, 0, 0, acc, lane);
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");
+    __builtin_amdgcn_s_waitcnt(0xC07F);   // lgkmcnt 0
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");
+    double part[2][8];
+    finish_staged<32>(
+        a, sT, 32, oc0, lane, 64, [&](int pl) { return p0 + pl < a.npix ? p0 + pl : -1; }, part, 0);
+}
+
+void launch_slim_split(const ConvArgs& a, hipStream_t s) {
+    hipLaunchKernelGGL(conv3x3_slim_split_kernel, dim3(cdiv(a.npix, 32), cdiv(a.OC, 32)), dim3(320), 0, s, a);
+}
+
 template <int BM, int BN, int WM, int WN, int KC>
 void launch_igemm(const ConvArgs& a, hipStream_t s) {
     constexpr int NT = (BM / WM) * (BN / WN) * 64;
@@ -2919,7 +3030,8 @@ struct TileCfg {
 // with the prologue / segment-sum variants, 92-101 the GEMM kernel's tiles for
 // launches that leave the chip partly idle (deep rings of 64- and 128-channel
 // chunks; pick_small_tile), 102 the band kernels' sums on 32 x 32 tiles, 103-108
-// the producer / compute band kernel on column segments of any map (pick_band).
+// the producer / compute band kernel on column segments of any map (pick_band),
+// 109 the halo kernel's split-f16 sums on 32 x 32 tiles.
 
 // Tile table.  Wave tiles are WM x WN = (bm / waves_m) x (bn / waves_n) with
 // 4 waves per workgroup; entries are selected per layer by pick_tile().
@@ -3033,6 +3145,7 @@ const TileCfg kTiles[] = {
     {128, 128, 16, launch_bandws<3, 38, 2, 2, 2, 4>, true, 0, 1 << 20},  // 106
     {128, 96, 16, launch_bandws<1, 75, 4, 3, 1, 4>, true, 0, 1 << 20},   // 107: one-row bands
     {128, 64, 16, launch_bandws<1, 38, 4, 1, 2, 4>, true, 0, 1 << 20},   // 108
+    {32, 32, 32, launch_slim_split, true},                // 109: the halo kernel's split-f16 sums on 32 x 32 tiles
 };
 constexpr int kNumTiles = (int)(sizeof(kTiles) / sizeof(kTiles[0]));
 
@@ -3040,6 +3153,7 @@ bool is_s1_3x3(const ConvArgs& a) {
     return a.KH == 3 && a.KW == 3 && a.sh == 1 && a.sw == 1 && a.ph == 1 && a.pw == 1 && a.dh == 1 && a.dw == 1;
 }
 
+constexpr int kFirstSlimSplit = 109;   // the split-f16 3x3 kernel for small launches
 constexpr int kFirstSmall = 92;   // the GEMM kernel's small-launch tiles
 constexpr int kFirstDma = 14;   // then the halo tiles from 26, 8-wave DMA tiles from 33
 
@@ -3086,6 +3200,11 @@ bool tile_fits(const TileCfg& t, const ConvArgs& a) {
     // the in-image tap range for a single row of taps; longer 2-D kernels
     // take the register-staged kernel
     if (a.KH * a.KW > 32 && a.KH != 1 && !igemm_tile(idx)) return false;
+    if (idx >= kFirstSlimSplit) {
+        const auto al = [](const void* p) { return ((uintptr_t)p & 15) == 0; };
+        return a.split && a.IC % 32 == 0 && !a.reflect && !a.segsum && !a.wq && !a.in_scale && a.xs % 8 == 0 &&
+               a.x_lo % 8 == 0 && a.xgs % 8 == 0 && al(a.x) && al(a.w);
+    }
     if (t.sp_ic) return a.IC == t.sp_ic && a.OC == t.bm && split_epilogue(a);
     // the GEMM kernel: channel groups whole per chunk, split-f16 plane terms
     // as consecutive chunks of a tap (2-D taps: the small-launch tiles; prologue / segment sums: the EXT tiles, 1x1 without padding, up to
@@ -3333,6 +3452,17 @@ int pick_tile(const ConvArgs& a) {
     // in the model fcm_conv1 + fcm_conv2 0.256 -> 0.219 ms per step)
     if (!a.split && is_s1_3x3(a) && a.IC == 32 && a.OC == 32 && a.res && tile_fits(kTiles[69], a)) return 69;
     if (a.split && is_s1_3x3(a)) {   // ERes2Net's split-f16 group convs (random-data sweeps)
+        // the layers whose kernels below sum in the halo kernel's order, up to two
+        // 32 x 32 tiles per CU (launches of 4.5 us included: 2 x 10 x 91, 128 ->
+        // 128 24.5 -> 11.7 us; 2 x 20 x 182, 64 -> 64 17.2 -> 12.3, 1 x 20 x 150
+        // 16.8 -> 9.1; 1 x 40 x 100, 32 -> 32 12.6 -> 7.8; 910 tiles: 13.3 -> 14.4)
+        const bool wide = a.IC == 128 && a.OC == 128 && a.H <= 10;
+        if ((a.OC == 32 || a.OC == 64 || wide) && (long)cdiv(a.npix, 32) * cdiv(a.OC, 32) <= 512 &&
+            tile_fits(kTiles[109], a))
+            return 109;
+        // then 32-column tiles while the 64-column ones leave CUs idle (8 x 10 x 38: 23.2 -> 17.2 us)
+        if (wide && (long)(a.npix / (a.Ho * a.Wo)) * cdiv(a.H, 4) * cdiv(a.W, 64) * 4 < 256 && tile_fits(kTiles[28], a))
+            return 28;
         // f16-exact weights: the split-f16 register-weight kernel
         if (a.OC == 16 && a.IC == 32 && tile_fits(kTiles[70], a)) return 70;
         if (a.OC == 16 && a.IC == 16 && tile_fits(kTiles[71], a)) return 71;
