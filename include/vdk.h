@@ -222,6 +222,9 @@ int vdk_conv_set_autotune(int on);
  * tuned it. */
 int vdk_conv_tuned_tile(const vdk_conv_desc* d);
 int vdk_conv2d_tile_fits_ex(int tile, const vdk_conv_desc* desc);
+/* Host: the tile a call with tile = -1 takes without run-time tuning, or -1
+ * when no tile takes it (pointers count by presence only). */
+int vdk_conv2d_pick(const vdk_conv_desc* desc);
 
 /* Same contract with an explicit kernel/tile choice (index into the library's
  * tile table; vdk_conv2d_tile_fits tells which apply to a shape).  For

@@ -1,0 +1,64 @@
+"""The conv dispatch on the host (vdk_conv2d_pick, vdk_conv2d_tile_fits_ex): which
+tile takes which call, over shapes, layouts and batches, with no GPU."""
+import itertools
+
+import pytest
+
+from vdamd import lib
+
+BATCHES = (1, 2, 5, 16, 24, 64, 256, 1500, 12000)
+
+
+def desc(B, H, W, IC, OC, K=3, stride=1, pad=1, out_w=0, split=0, group=0, res=False, act=lib.ACT_RELU):
+    d = lib.ConvDesc()
+    d.batch, d.H, d.W, d.IC, d.OC, d.KH, d.KW = B, H, W, IC, OC, K, K
+    d.stride_h = d.stride_w = stride
+    d.pad_h = d.pad_w = pad
+    d.dil_h = d.dil_w = 1
+    d.out_w, d.act = out_w, act
+    d.residual = 16 if res else None   # only its presence matters
+    d.split = split
+    if split:
+        d.x_stride, d.x_lo, d.y_stride, d.y_lo, d.res_lo = 2 * IC, IC, 2 * OC, OC, OC
+        d.res_stride = 2 * OC if res else 0
+    if group:
+        d.x_group = d.y_group = d.x_lo = d.y_lo = group
+        d.x_group_stride = d.y_group_stride = 2 * group
+    return d
+
+
+def fits(t, d):
+    return bool(lib.lib().vdk_conv2d_tile_fits_ex(t, d))
+
+
+def too_large(d):
+    return d.batch * d.H * d.W * (d.x_stride or d.IC) >= 1 << 30 or d.batch * d.H * d.W * (d.y_stride or d.OC) >= 1 << 31
+
+
+# the register-weight, split-f16 register-weight, band and 32 x 32 3x3 kernels:
+# they store every row as wide as they read it
+WHOLE_ROWS = list(range(53, 60)) + list(range(64, 80)) + list(range(102, 110))
+
+
+@pytest.mark.parametrize("split,group", [(0, 0), (1, 0), (2, 0), (2, 32)])
+def test_cropped_3x3_never_on_whole_row_kernels(split, group):
+    """out_w < W: no kernel that stores whole rows takes the call (it would
+    write past y), explicitly or by default, and some kernel does."""
+    L, n = lib.lib(), 0
+    for IC, OC, H, W, res, act in itertools.product((32, 64, 128, 256), (32, 64, 128, 256), (1, 10, 20, 40),
+                                                    (20, 38, 75, 77, 126, 300), (False, True),
+                                                    (lib.ACT_RELU, lib.ACT_NONE)):
+        if group and res:
+            continue
+        whole = desc(1, H, W, IC, OC, split=split, group=group, res=res, act=act)
+        n += sum(fits(t, whole) for t in WHOLE_ROWS if t < L.vdk_conv2d_tile_count())
+        for out_w in (1, W - 7, W - 1):
+            d = desc(1, H, W, IC, OC, out_w=out_w, split=split, group=group, res=res, act=act)
+            for t in range(L.vdk_conv2d_tile_count()):
+                assert not (t in WHOLE_ROWS and fits(t, d)), (t, IC, OC, H, W, out_w)
+            for B in BATCHES:
+                d.batch = B
+                if not too_large(d):
+                    t = L.vdk_conv2d_pick(d)
+                    assert t >= 0 and t not in WHOLE_ROWS, (t, B, IC, OC, H, W, out_w)
+    assert n > 100   # they do take the uncropped calls

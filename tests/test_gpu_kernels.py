@@ -830,3 +830,76 @@ def test_conv_autotune_same_bits_and_cached(B, H, W, IC, OC, K, res):
         lib.check(L.vdk_conv_set_autotune(0))
     assert np.array_equal(outs[1], outs[0]) and np.array_equal(outs[2], outs[0])
     assert t >= 0 and L.vdk_conv2d_tile_fits_ex(t, d)
+
+
+@pytest.mark.parametrize("B,H,W,out_w,IC,OC,res,split,group", [
+    (2, 5, 77, 70, 128, 128, True, 0, 0),     # wide map: bands of column segments when whole
+    (1, 7, 40, 39, 256, 256, False, 0, 0),
+    (1, 6, 20, 1, 128, 128, True, 0, 0),      # narrow: the 32 x 32 tiles when whole
+    (1, 9, 33, 30, 64, 64, True, 0, 0),       # the register-weight kernel's layers
+    (2, 5, 33, 20, 32, 32, True, 0, 0),
+    (1, 10, 40, 33, 128, 128, False, 2, 0),   # split-f16
+    (1, 8, 45, 44, 64, 64, False, 2, 0),
+    (1, 7, 37, 30, 32, 32, False, 2, 32),     # ... in 32-channel groups
+    (1, 7, 37, 30, 32, 32, False, 1, 0),
+])
+def test_conv3x3_cropped_columns(B, H, W, out_w, IC, OC, res, split, group):
+    """out_w < W on stride-1 3x3 convs: the default pick writes exactly the
+    first out_w columns of each row (guard bytes after y stay), residual and y
+    indexed by the cropped width."""
+    rng = np.random.default_rng(H * W + out_w + IC + OC)
+    announce(f"conv3x3 crop {W}->{out_w} {IC}->{OC} split={split} group={group}")
+    x = rng.standard_normal((B, H, W, IC)).astype(np.float32 if split else np.float16)
+    w = (rng.standard_normal((OC, 3, 3, IC)) * np.sqrt(2.0 / (9 * IC))).astype(np.float32)
+    if split != 1:
+        w = w.astype(np.float16).astype(np.float32)
+    b = rng.uniform(-0.5, 0.5, OC).astype(np.float32)
+    r = rng.standard_normal((B, H, out_w, OC)).astype(np.float16)
+
+    def halves(v):
+        hi = v.astype(np.float16)
+        return hi, (v - hi.astype(np.float32)).astype(np.float16)
+
+    wh, wl = halves(w)
+    pack = {0: [wh], 1: [wh, wh, wl], 2: [wh, wh]}[split]
+    xd = np.concatenate(halves(x), axis=3) if split else x
+    keep = [lib.DeviceBuffer.from_array(np.ascontiguousarray(v)) for v in (xd, np.concatenate(pack, axis=3), b, r)]
+    d = lib.ConvDesc()
+    d.x, d.batch, d.H, d.W, d.IC = keep[0].ptr, B, H, W, IC
+    d.w, d.OC, d.KH, d.KW = keep[1].ptr, OC, 3, 3
+    d.stride_h = d.stride_w = d.pad_h = d.pad_w = d.dil_h = d.dil_w = 1
+    d.bias, d.act, d.out_w, d.tile, d.split = keep[2].ptr, lib.ACT_RELU, out_w, -1, split
+    if res:
+        d.residual = keep[3].ptr
+    ys = 2 * OC if split else OC
+    if split:
+        d.x_stride, d.x_lo, d.y_stride, d.y_lo = 2 * IC, IC, ys, OC
+    if group:
+        d.x_group = d.y_group = d.x_lo = d.y_lo = group
+        d.x_group_stride = d.y_group_stride = 2 * group
+    n, guard = B * H * out_w * ys, 1 << 16
+    dy = lib.DeviceBuffer.from_array(np.full(n + guard, 0x5A5A, np.uint16))
+    d.y = dy.ptr
+    assert lib.lib().vdk_conv2d_pick(d) < 53 or 59 < lib.lib().vdk_conv2d_pick(d) < 64   # LDS-DMA, halo, register-staged
+    lib.check(lib.lib().vdk_conv2d_ex(d, None))
+    lib.check(lib.lib().vdk_synchronize())
+    raw = dy.to_array(np.uint16, (n + guard,))
+    assert (raw[n:] == 0x5A5A).all()
+    o = raw[:n].reshape(B, H, out_w, ys).view(np.float16).astype(np.float64)
+    got = o[..., :OC] + o[..., OC:] if split else o
+    xp = np.pad(x.astype(np.float64), ((0, 0), (1, 1), (1, 1), (0, 0)))
+    want, mag = b + np.zeros((B, H, out_w, OC)), np.abs(b) + np.zeros((B, H, out_w, OC))
+    for kh in range(3):
+        for kw in range(3):
+            xs = xp[:, kh:kh + H, kw:kw + out_w]
+            want += xs @ w[:, kh, kw].astype(np.float64).T
+            mag += np.abs(xs) @ np.abs(w[:, kh, kw].astype(np.float64)).T
+    if res:
+        want += r
+        mag += np.abs(r)
+    want = np.maximum(want, 0)
+    # f32 sums of (2 or 3 times) 9 * IC products, half an ulp each; the store
+    # to f16, or to hi + lo (the terms the split leaves out: 2^-22 of each product)
+    store = 2.0 ** -21 if split else 2.0 ** -11
+    assert (np.abs(got - want) <= ((split + 1) * 9 * IC * 2.0 ** -24 + (2.0 ** -21 if split else 0)) * mag +
+            store * np.abs(want) + 2.0 ** -24).all()

@@ -3183,6 +3183,9 @@ bool igemm_tile(int idx) { return idx < kFirstDma || idx == 62 || idx == 63 || i
 bool tile_fits(const TileCfg& t, const ConvArgs& a) {
     const int idx = (int)(&t - kTiles);
     if (t.halo && !is_s1_3x3(a)) return false;
+    // the register-weight, band and 32 x 32 3x3 kernels store the rows they
+    // read, whole: no cropped outputs (the halo tiles take those)
+    if (a.Wo != a.W && (t.rw_ic || t.sp_ic || t.band_w || idx >= kFirstSlimSplit)) return false;
     // the input prologue lives in the register-staged kernel's operand loads
     // and the LDS-DMA kernel's B fragments (up to 1024 input channels: their
     // scale / shift stage in LDS)
@@ -3520,7 +3523,7 @@ int pick_tile(const ConvArgs& a) {
         if (a.IC == 256 && a.OC == 512) return 40;
     }
     // (up to 256 64 x 64 tiles: the GEMM kernel's, the same bits; batch 1 10.2 -> 8.8 us)
-    if (is_s1_3x3(a) && a.IC == 64 && a.OC == 64 && plain_epilogue(a))
+    if (is_s1_3x3(a) && a.IC == 64 && a.OC == 64 && tile_fits(kTiles[66], a))
         return cdiv(a.npix, 64) <= 256 && tile_fits(kTiles[98], a) ? 98 : 66;   // 66: 3-stage ring
     const int band = pick_band(a);
     if (band >= 0) return band;
@@ -4037,6 +4040,10 @@ ConvArgs shape_args(const vdk_conv_desc& d) {
     a.ph = d.pad_h; a.pw = d.pad_w;
     a.dh = d.dil_h ? d.dil_h : 1; a.dw = d.dil_w ? d.dil_w : 1;
     a.H = d.H; a.W = d.W;
+    a.Ho = (d.H + 2 * d.pad_h - (d.KH - 1) * a.dh - 1) / a.sh + 1;
+    a.Wo = d.out_w > 0 ? d.out_w : (d.W + 2 * d.pad_w - (d.KW - 1) * a.dw - 1) / a.sw + 1;
+    a.npix = d.batch * a.Ho * a.Wo;
+    a.npix_in = d.batch * d.H * d.W;
     a.xs = d.x_stride ? d.x_stride : d.IC;
     a.ys = d.y_stride ? d.y_stride : d.OC;
     a.rs = d.res_stride ? d.res_stride : d.OC;
@@ -4064,6 +4071,7 @@ ConvArgs shape_args(const vdk_conv_desc& d) {
     a.ygl = d.y_group == 32 ? 5 : 4;
     a.xgs = d.x_group_stride ? d.x_group_stride : 1 << a.xgl;
     a.ygs = d.y_group_stride ? d.y_group_stride : 1 << a.ygl;
+    a.x_lo = d.x_lo; a.r_lo = d.res_lo; a.y_lo = d.y_lo;
     return a;
 }
 
@@ -4115,13 +4123,7 @@ extern "C" int vdk_conv_set_autotune(int on) {
 
 extern "C" int vdk_conv_tuned_tile(const vdk_conv_desc* d) {
     if (!d || d->batch <= 0) return -1;
-    ConvArgs a = shape_args(*d);   // + the fields conv_impl derives
-    const int ekh = (d->KH - 1) * a.dh + 1, ekw = (d->KW - 1) * a.dw + 1;
-    a.Ho = (d->H + 2 * d->pad_h - ekh) / a.sh + 1;
-    const int Wo_full = (d->W + 2 * d->pad_w - ekw) / a.sw + 1;
-    a.Wo = d->out_w > 0 ? d->out_w : Wo_full;
-    a.npix = d->batch * a.Ho * a.Wo;
-    a.npix_in = d->batch * d->H * d->W;
+    ConvArgs a = shape_args(*d);
     a.bias = d->bias;
     a.wc = static_cast<const half_t*>(d->w_chunked);
     TuneCache& tc = tune_cache();
@@ -4133,6 +4135,13 @@ extern "C" int vdk_conv_tuned_tile(const vdk_conv_desc* d) {
 extern "C" int vdk_conv2d_tile_fits_ex(int tile, const vdk_conv_desc* d) {
     if (tile < 0 || tile >= kNumTiles || !d) return 0;
     return tile_fits(kTiles[tile], shape_args(*d)) ? 1 : 0;
+}
+
+extern "C" int vdk_conv2d_pick(const vdk_conv_desc* d) {
+    if (!d || d->batch <= 0) return -1;
+    const ConvArgs a = shape_args(*d);
+    const int t = pick_tile(a);
+    return t >= 0 && tile_fits(kTiles[t], a) ? t : -1;
 }
 
 extern "C" int vdk_stem_conv3x3_ex(const float* d_feats, const float* d_row_mean, int batch, int H, int W,
