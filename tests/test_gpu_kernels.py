@@ -903,3 +903,35 @@ def test_conv3x3_cropped_columns(B, H, W, out_w, IC, OC, res, split, group):
     store = 2.0 ** -21 if split else 2.0 ** -11
     assert (np.abs(got - want) <= ((split + 1) * 9 * IC * 2.0 ** -24 + (2.0 ** -21 if split else 0)) * mag +
             store * np.abs(want) + 2.0 ** -24).all()
+
+
+@pytest.mark.parametrize("W,C,relu", [(20, 128, False), (20, 128, True), (75, 128, True), (38, 256, False),
+                                      (126, 128, False), (126, 128, True), (37, 64, False)])
+def test_conv3x3_nonfinite_residual_stays_in_its_channel(W, C, relu):
+    """An infinite and a NaN residual change their own output only: every
+    other channel and pixel keeps the bits of the run with finite residuals, on
+    every tile that takes the shape."""
+    rng = np.random.default_rng(W + C)
+    H, B = 7, 2
+    x = rng.standard_normal((B, H, W, C)).astype(np.float16)
+    w = (rng.standard_normal((C, C, 3, 3)) * np.sqrt(2.0 / (9 * C))).astype(np.float16)
+    b = rng.uniform(-0.5, 0.5, C).astype(np.float32)
+    res = rng.standard_normal((B, H, W, C)).astype(np.float16)
+    bad = res.copy()
+    at = np.zeros(res.shape, bool)
+    for (c, h, ww, ch), v in (((0, 0, 0, 5), np.inf), ((1, H - 1, W - 1, C - 1), np.nan), ((0, 3, W // 2, 33), -np.inf)):
+        bad[c, h, ww, ch] = v
+        at[c, h, ww, ch] = True
+    n = 0
+    for t in [-1] + list(range(lib.lib().vdk_conv2d_tile_count())):
+        if t >= 0 and not tile_fits(t, B, H, W, C, C, 3, 1, 1, relu=relu):
+            continue
+        announce(f"non-finite residual tile {t} W={W} C={C} relu={relu}")
+        want = conv_gpu(x, w, b, res, 1, 1, relu, tile=t)
+        got = conv_gpu(x, w, b, bad, 1, 1, relu, tile=t)
+        assert np.array_equal(got.view(np.uint16)[~at], want.view(np.uint16)[~at]), f"tile {t}"
+        assert np.isposinf(got[0, 0, 0, 5])
+        assert got[0, 3, W // 2, 33] == (0 if relu else -np.inf)
+        assert relu or np.isnan(got[1, H - 1, W - 1, C - 1])
+        n += 1
+    assert n >= 3

@@ -2486,6 +2486,42 @@ __device__ __forceinline__ int div_small(int n, float inv_d) {
     return (int)(((float)n + 0.5f) * inv_d);
 }
 
+// acc + residual of a 32-channel x 32-pixel block through MFMAs with identity A
+// operands (products r x 1, one rounding): lane (lrow, lhalf) passes channels
+// h * 16 + lhalf * 8 .. + 7 of pixel lrow in rv[h].  An infinite or NaN residual
+// would reach the pixel's other channels too (0 x Inf), in every accumulator:
+// such a block runs again with finite residuals, and each lane adds the others
+// to its own outputs (own(g): the residuals of registers g*4 .. + 3).
+template <class Own>
+__device__ __forceinline__ float16v add_residual_block(const half8* rv, const float16v& acc, int lrow, int lhalf, Own own) {
+    half8 eye[2];
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int e = 0; e < 8; ++e) eye[h][e] = (half_t)((lrow == h * 16 + lhalf * 8 + e) ? 1.0f : 0.0f);
+    float16v sum = acc;
+#pragma unroll
+    for (int h = 0; h < 2; ++h) sum = __builtin_amdgcn_mfma_f32_32x32x16_f16(eye[h], rv[h], sum, 0, 0, 0);
+    if (__any(!__builtin_isfinite(sum[0]))) {
+        sum = acc;
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            half8 f = rv[h];
+#pragma unroll
+            for (int e = 0; e < 8; ++e) f[e] = __builtin_isfinite((float)f[e]) ? f[e] : (half_t)0.0f;
+            sum = __builtin_amdgcn_mfma_f32_32x32x16_f16(eye[h], f, sum, 0, 0, 0);
+        }
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+            const half4 r = own(g);
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                if (!__builtin_isfinite((float)r[e])) sum[g * 4 + e] += (float)r[e];
+        }
+    }
+    return sum;
+}
+
 // SEG: maps of several column segments (one segment: the arithmetic of the
 // columns compiles away, 3 % of the 5-row bands at batch 64)
 template <int TH, int MAXW, int WMG, int WNG, int NJ, int NP, bool SEG>
@@ -2675,25 +2711,21 @@ __global__ __launch_bounds__((WMG * WNG + NP) * 64) void conv3x3_bandws_kernel(C
     // the residual rows, then the wave's channel range of its pixel rows out
     // as 16-byte chunks.
     const bool relu = a.act == VDK_ACT_RELU;
-    half8 eye[2];
-#pragma unroll
-    for (int h = 0; h < 2; ++h)
-#pragma unroll
-        for (int e = 0; e < 8; ++e) eye[h][e] = (half_t)((lrow == h * 16 + lhalf * 8 + e) ? 1.0f : 0.0f);
 #pragma unroll
     for (int i = 0; i < MI; ++i) {
         const int cw = cg0 + i * 32;
 #pragma unroll
         for (int j = 0; j < NJ; ++j) {
             uint8_t* const prow = rrow((pg * NJ + j) * 32 + lrow);
-            if (has_res) {
-#pragma unroll
-                for (int h = 0; h < 2; ++h) {
-                    const half8 rv = *reinterpret_cast<const half8*>(prow + (cw + h * 16 + lhalf * 8) * 2);
-                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(eye[h], rv, acc[i][j], 0, 0, 0);
-                }
-            }
             uint8_t* const row = prow + (cw + lhalf * 4) * 2;
+            if (has_res) {
+                half8 rv[2];
+#pragma unroll
+                for (int h = 0; h < 2; ++h)
+                    rv[h] = *reinterpret_cast<const half8*>(prow + (cw + h * 16 + lhalf * 8) * 2);
+                acc[i][j] = add_residual_block(rv, acc[i][j], lrow, lhalf,
+                                               [&](int g) { return *reinterpret_cast<const half4*>(row + g * 16); });
+            }
 #pragma unroll
             for (int g = 0; g < 4; ++g) {
                 half4 hv;
@@ -2836,15 +2868,10 @@ __global__ __launch_bounds__(192) void conv3x3_slim_kernel(ConvArgs a) {
 #pragma unroll
         for (int t = 0; t < 9; ++t) acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[t], bf[t], acc, 0, 0, 0);
     }
-    if (a.res) {
-#pragma unroll
-        for (int h = 0; h < 2; ++h) {
-            half8 eye;
-#pragma unroll
-            for (int e = 0; e < 8; ++e) eye[e] = (half_t)((lrow == h * 16 + lhalf * 8 + e) ? 1.0f : 0.0f);
-            acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(eye, rv[h], acc, 0, 0, 0);
-        }
-    }
+    if (a.res)
+        acc = add_residual_block(rv, acc, lrow, lhalf, [&](int g) {
+            return ok ? *reinterpret_cast<const half4*>(a.res + (size_t)P * a.rs + oc0 + g * 8 + lhalf * 4) : half4{};
+        });
     // f16, then the lane halves trade 4-channel pieces, so each lane stores
     // two whole 8-channel chunks of its pixel
     const bool relu = a.act == VDK_ACT_RELU;
