@@ -62,3 +62,36 @@ def test_cropped_3x3_never_on_whole_row_kernels(split, group):
                     t = L.vdk_conv2d_pick(d)
                     assert t >= 0 and t not in WHOLE_ROWS, (t, B, IC, OC, H, W, out_w)
     assert n > 100   # they do take the uncropped calls
+
+
+# tiles by the order their sums run in: the halo kernel's split-f16 order (plane
+# terms, 32-channel chunks, taps) and the band kernels' (16-channel chunks, taps,
+# bias first); the rest run taps first, but for the 16-row MFMA tiles
+def sum_order(t, d):
+    if t in (70, 71, 73):
+        return f"16-row MFMA, tile {t}"
+    if t in (72, 74, 75, 109) or (26 <= t <= 32 and (d.split or d.IC > 32)):
+        return "halo"
+    if t in (57, 58, 59):
+        return "band, bias last"
+    if t in (64, 65) or 76 <= t <= 79 or 102 <= t <= 108:
+        return "band"
+    return "taps"
+
+
+@pytest.mark.parametrize("split,group", [(1, 0), (1, 16), (1, 32), (2, 0), (2, 16), (2, 32)])
+def test_split_3x3_order_does_not_depend_on_the_batch(split, group):
+    """Every batch of a split-f16 3x3 shape runs its sums in the same order, so a
+    clip's bits do not depend on the batch it is in."""
+    L = lib.lib()
+    for IC, OC, H, W, act in itertools.product((16, 32, 64, 128), (16, 32, 64, 128), (1, 10, 20, 40),
+                                               (13, 49, 91, 150, 998, 1998), (lib.ACT_RELU, lib.ACT_SILU)):
+        if IC == 16 and (split != 2 or OC != 16) or (group == 32 and (IC % 32 or OC % 32)):
+            continue
+        seen = {}
+        for B in BATCHES:
+            d = desc(B, H, W, IC, OC, split=split, group=group, act=act)
+            if not too_large(d):
+                t = L.vdk_conv2d_pick(d)
+                seen.setdefault(sum_order(t, d) if t >= 0 else "refused", []).append((B, t))
+        assert len(seen) == 1, (IC, OC, H, W, act, seen)

@@ -73,3 +73,16 @@ def test_eres2net_f32_weights():
     ctx = lib.Context(path)
     _check(ctx, O.OracleEres2net(g), synth.clips(640, 2, 48000), (0, 1), "eres2net f32")
     ctx.close()
+
+
+def test_eres2net_f32_weights_batch_invariance():
+    """Three-term weights over grouped chunks: a clip's embedding keeps its bits
+    in a batch whose layers are past the small-launch limits."""
+    path, _ = _model(synth.write_eres2net, "eres2net_f32.gguf", seed=64, wtype=gguf.GGML_F32, f16_exact=False)
+    announce("f32 weights: eres2net 1 s alone and in batches of 12")
+    ctx = lib.Context(path)
+    pcm = synth.clips(641, 12, 16000)
+    emb = ctx.embed_batch(pcm)
+    for c in (0, 5, 11):
+        assert np.array_equal(ctx.embed_batch(pcm[c:c + 1])[0], emb[c]), f"clip {c}"
+    ctx.close()

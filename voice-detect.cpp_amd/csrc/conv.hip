@@ -20,6 +20,7 @@
 #include <atomic>
 #include <climits>
 #include <cstdlib>
+#include <initializer_list>
 #include <mutex>
 #include <string>
 #include <type_traits>
@@ -3486,14 +3487,18 @@ int pick_tile(const ConvArgs& a) {
     // in the model fcm_conv1 + fcm_conv2 0.256 -> 0.219 ms per step)
     if (!a.split && is_s1_3x3(a) && a.IC == 32 && a.OC == 32 && a.res && tile_fits(kTiles[69], a)) return 69;
     if (a.split && is_s1_3x3(a)) {   // ERes2Net's split-f16 group convs (random-data sweeps)
-        // the layers whose kernels below sum in the halo kernel's order, up to two
-        // 32 x 32 tiles per CU (launches of 4.5 us included: 2 x 10 x 91, 128 ->
-        // 128 24.5 -> 11.7 us; 2 x 20 x 182, 64 -> 64 17.2 -> 12.3, 1 x 20 x 150
+        // the layers whose kernels below sum in the halo kernel's order (not the
+        // channel groups that only the LDS-DMA tiles take, e.g. with three-term
+        // weights: a clip's bits would depend on its batch), up to two 32 x 32
+        // tiles per CU (launches of 4.5 us included: 2 x 10 x 91, 128 -> 128
+        // 24.5 -> 11.7 us; 2 x 20 x 182, 64 -> 64 17.2 -> 12.3, 1 x 20 x 150
         // 16.8 -> 9.1; 1 x 40 x 100, 32 -> 32 12.6 -> 7.8; 910 tiles: 13.3 -> 14.4)
+        const auto any = [&](std::initializer_list<int> ts) {
+            return std::any_of(ts.begin(), ts.end(), [&](int t) { return tile_fits(kTiles[t], a); });
+        };
         const bool wide = a.IC == 128 && a.OC == 128 && a.H <= 10;
-        if ((a.OC == 32 || a.OC == 64 || wide) && (long)cdiv(a.npix, 32) * cdiv(a.OC, 32) <= 512 &&
-            tile_fits(kTiles[109], a))
-            return 109;
+        const bool halo_order = a.OC == 32 ? any({28, 72, 74}) : (a.OC == 64 ? any({30, 75}) : wide && any({26}));
+        if (halo_order && (long)cdiv(a.npix, 32) * cdiv(a.OC, 32) <= 512 && tile_fits(kTiles[109], a)) return 109;
         // then 32-column tiles while the 64-column ones leave CUs idle (8 x 10 x 38: 23.2 -> 17.2 us)
         if (wide && (long)(a.npix / (a.Ho * a.Wo)) * cdiv(a.H, 4) * cdiv(a.W, 64) * 4 < 256 && tile_fits(kTiles[28], a))
             return 28;
