@@ -95,3 +95,20 @@ def test_split_3x3_order_does_not_depend_on_the_batch(split, group):
                 t = L.vdk_conv2d_pick(d)
                 seen.setdefault(sum_order(t, d) if t >= 0 else "refused", []).append((B, t))
         assert len(seen) == 1, (IC, OC, H, W, act, seen)
+
+
+def test_plain_3x3_order_does_not_depend_on_the_batch():
+    """The same for f16 3x3 layers, up to the largest launch (outputs of 2^31
+    elements)."""
+    L, large = lib.lib(), 0
+    for IC, OC, H, W, res in itertools.product((16, 32, 64, 128, 256), (32, 64, 128, 256, 384), (5, 10, 20, 80),
+                                               (13, 38, 75, 77, 126, 300), (False, True)):
+        seen = {}
+        for B in BATCHES + (4000, 6000, 9000):
+            d = desc(B, H, W, IC, OC, res=res)
+            if not too_large(d):
+                t = L.vdk_conv2d_pick(d)
+                seen.setdefault(sum_order(t, d) if t >= 0 else "refused", []).append((B, t))
+                large += OC % 128 == 0 and B * H * W * OC >= 1 << 30
+        assert len(seen) == 1, (IC, OC, H, W, res, seen)
+    assert large > 50

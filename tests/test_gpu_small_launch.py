@@ -322,3 +322,41 @@ def test_slim_split_bitwise(B, H, W, IC, OC, split, groups):
                                 bias=bias, f64=True) for c in range(B)])
     want = np.clip(want, 0, 20)
     assert np.abs(got.transpose(0, 3, 1, 2) - want).max() <= 2e-6 * max(np.abs(want).max(), 1.0)
+
+
+def test_band_output_past_two_gigabytes():
+    """16 -> 128 channels over 5600 clips of 20 x 75 (output and residual of 2.15
+    GB): the first and last clips have the bits they have in a batch of three."""
+    B, H, W, IC, OC, n = 5600, 20, 75, 16, 128, 3
+    rng = np.random.default_rng(5600)
+    announce(f"band output of {B * H * W * OC * 2 / 2**30:.2f} GiB")
+    x, r = (rng.standard_normal((n, H, W, c)).astype(np.float16) for c in (IC, OC))
+    w = (rng.standard_normal((OC, 3, 3, IC)) * np.sqrt(2.0 / (9 * IC))).astype(np.float16)
+    b = rng.uniform(-0.5, 0.5, OC).astype(np.float32)
+    L, dw, db = lib.lib(), lib.DeviceBuffer.from_array(w), lib.DeviceBuffer.from_array(b)
+
+    def run(batch):
+        clip = H * W * 2
+        dx, dr, dy = (lib.DeviceBuffer(batch * clip * c) for c in (IC, OC, OC))
+        dx.copy_from(np.resize(x, (batch, H, W, IC)))
+        for c0 in range(0, batch, 300):   # (300 % n == 0)
+            part = np.resize(r, (min(300, batch - c0), H, W, OC))
+            lib.check(L.vdk_memcpy_h2d(dr.ptr + c0 * clip * OC, part.ctypes.data, part.nbytes))
+        d = lib.ConvDesc()
+        d.x, d.batch, d.H, d.W, d.IC = dx.ptr, batch, H, W, IC
+        d.w, d.OC, d.KH, d.KW = dw.ptr, OC, 3, 3
+        d.stride_h = d.stride_w = d.pad_h = d.pad_w = d.dil_h = d.dil_w = 1
+        d.bias, d.residual, d.act, d.y, d.tile = db.ptr, dr.ptr, lib.ACT_RELU, dy.ptr, -1
+        lib.check(L.vdk_conv2d_ex(d, None))
+        lib.check(L.vdk_synchronize())
+        out = {}
+        for c in range(n), range(batch - n, batch):
+            for i in c:
+                o = np.empty((H, W, OC), np.uint16)
+                lib.check(L.vdk_memcpy_d2h(o.ctypes.data, dy.ptr + i * clip * OC, o.nbytes))
+                out[i] = o
+        return out
+
+    want, got = run(n), run(B)
+    for i, o in got.items():
+        assert np.array_equal(o, want[i % n]), f"clip {i}"

@@ -3330,7 +3330,7 @@ long round_cost(const ConvArgs& a, int t) {
 // 10 x 38 x 256 16.8 -> 10.8 at batch 1 (102), 27.9 -> 22.6 at batch 16 (106);
 // 10 x 63 x 256 at batch 64 68.8 -> 53.3 (103).
 int pick_band(const ConvArgs& a) {
-    if (!is_s1_3x3(a) || a.OC % 128 != 0 || !plain_epilogue(a) || (long)a.npix * a.OC >= (1L << 30)) return -1;
+    if (!is_s1_3x3(a) || a.OC % 128 != 0 || !plain_epilogue(a)) return -1;
     struct BandCost { int tile, th, maxw; float base, per; };
     static const BandCost kBands[] = {
         {103, 5, 75, 9.5f, 1.56f}, {104, 5, 38, 6.0f, 1.06f}, {105, 3, 75, 7.5f, 1.06f},
