@@ -112,3 +112,18 @@ def test_plain_3x3_order_does_not_depend_on_the_batch():
                 large += OC % 128 == 0 and B * H * W * OC >= 1 << 30
         assert len(seen) == 1, (IC, OC, H, W, res, seen)
     assert large > 50
+
+
+@pytest.mark.parametrize("IC,OC,seg_len,taken", [
+    (128, 128, 100, True), (64, 128, 64, True), (1024, 512, 100, True), (96, 128, 100, True),
+    (64, 128, 40, False),    # segments shorter than the wide tile's 64 pixels
+    (32, 32, 100, False), (64, 8, 100, False), (96, 40, 100, False),   # 128-pixel tiles for narrow outputs
+])
+def test_segment_sums_taken_or_refused_at_every_batch(IC, OC, seg_len, taken):
+    """seg_sum calls: whether a shape is taken does not depend on the batch (the
+    small-launch tiles would take shorter segments)."""
+    for B, T in itertools.product((1, 2, 8, 32), (1, 49, 249, 499)):
+        d = desc(B, 1, T, IC, OC, K=1, pad=0)
+        d.in_scale = d.in_shift = d.seg_sum = 16
+        d.seg_len = seg_len
+        assert (lib.lib().vdk_conv2d_pick(d) >= 0) == taken, (B, T)

@@ -3362,11 +3362,7 @@ int pick_band(const ConvArgs& a) {
 // implicit GEMM with the widest OC tile that divides OC; IC % 32 != 0: the
 // register-staged kernel with KC = 16).  OC that no tile divides runs on
 // 32-wide tiles with the surplus rows masked.
-int pick_tile(const ConvArgs& a) {
-    const int o = tile_override();
-    if (o >= 0 && o < kNumTiles && tile_fits(kTiles[o], a)) return o;
-    const int small = pick_small_tile(a);
-    if (small >= 0) return small;
+int pick_wide_tile(const ConvArgs& a) {
     const int bm = a.OC % 128 == 0 ? 128 : (a.OC % 64 == 0 ? 64 : 32);
     if (a.in_scale) {
         // CAM++'s 1024 -> 512 transits (B=32 x 499 frames): the GEMM kernel's
@@ -3590,6 +3586,17 @@ int pick_tile(const ConvArgs& a) {
     if (a.split) return -1;
     if (a.IC % 16 == 0) return bm == 128 ? 13 : (bm == 64 ? 12 : 11);
     return -1;
+}
+
+int pick_tile(const ConvArgs& a) {
+    const int o = tile_override();
+    if (o >= 0 && o < kNumTiles && tile_fits(kTiles[o], a)) return o;
+    const int small = pick_small_tile(a);
+    if (small >= 0 && !a.segsum) return small;
+    // segment sums: what the wide tile refuses (a pixel tile wider than a
+    // segment) is refused at any size, not accepted for small batches only
+    const int wide = pick_wide_tile(a);
+    return small >= 0 && wide >= 0 && tile_fits(kTiles[wide], a) ? small : wide;
 }
 
 template <int OC>
