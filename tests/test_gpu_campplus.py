@@ -427,11 +427,11 @@ def test_linear1_segment_sums_feed_cam_local(batch, T, c_in):
 
 
 @pytest.mark.parametrize("batch,T,c_in", [(B, TP, 320), (B, TP, 1024), (3, 257, 160), (8, 149, 288),
-                                          (8, 49, 160), (16, 101, 256), (12, 3, 128)])
+                                          (8, 49, 160), (16, 101, 256), (12, 3, 128), (2, 131, 576)])
 def test_linear1_tiles_bitwise(batch, T, c_in):
     """linear1 (BN + ReLU prologue, bias, ReLU, segment sums) on the GEMM
-    kernel's narrow tiles with producer / compute waves: the register-staged
-    tiles' bits, outputs and f64 segment sums alike (same operand rounding,
+    kernel's narrow and small-launch tiles with producer / compute waves: the
+    register-staged tiles' bits, outputs and f64 segment sums alike (same operand rounding,
     K order and exact sums), including pixel tiles that reach three
     segments."""
     rng = np.random.default_rng(11 * T + c_in)
@@ -446,7 +446,7 @@ def test_linear1_tiles_bitwise(batch, T, c_in):
     bias = (rng.standard_normal(BC, dtype=np.float32) * 0.1).astype(np.float32)
     dd, ds1, dt1, dw, db = (lib.DeviceBuffer.from_array(a) for a in (dense, s1, t1, w, bias))
     outs = {}
-    for tile in (63, 80, 85, 86, 87, 88):
+    for tile in (63, 80, 85, 86, 87, 88, 92, 93, 94, 96, 98):
         d = lib.ConvDesc()
         d.x, d.batch, d.H, d.W, d.IC, d.x_stride = dd.ptr, batch, 1, T, c_in, CMAX
         d.w, d.OC, d.KH, d.KW = dw.ptr, BC, 1, 1
@@ -462,7 +462,8 @@ def test_linear1_tiles_bitwise(batch, T, c_in):
         lib.check(L.vdk_conv2d_ex(d, None))
         _sync()
         outs[tile] = (dh.to_array(np.uint16, (batch, T, BC)), seg.to_array(np.float64, (batch, nseg, BC)))
-    assert 63 in outs and sum(t >= 85 for t in outs) >= 3, sorted(outs)
+    assert 63 in outs and sum(t >= 85 for t in outs) >= 3 and sum(t >= 92 for t in outs) >= 1 + 2 * (c_in % 64 == 0), \
+        sorted(outs)
     for t, (h, sg) in outs.items():
         assert np.array_equal(h, outs[63][0]), f"tile {t} outputs"
         assert np.array_equal(sg, outs[63][1]), f"tile {t} segment sums"
