@@ -37,7 +37,7 @@ def too_large(d):
 
 # the register-weight, split-f16 register-weight, band and 32 x 32 3x3 kernels:
 # they store every row as wide as they read it
-WHOLE_ROWS = list(range(53, 60)) + list(range(64, 80)) + list(range(102, 110))
+WHOLE_ROWS = list(range(53, 60)) + list(range(64, 80)) + [102]
 
 
 @pytest.mark.parametrize("split,group", [(0, 0), (1, 0), (2, 0), (2, 32)])
@@ -70,11 +70,9 @@ def test_cropped_3x3_never_on_whole_row_kernels(split, group):
 def sum_order(t, d):
     if t in (70, 71, 73):
         return f"16-row MFMA, tile {t}"
-    if t in (72, 74, 75, 109) or (26 <= t <= 32 and (d.split or d.IC > 32)):
+    if t in (72, 74, 75, 102) or (26 <= t <= 32 and (d.split or d.IC > 32)):
         return "halo"
-    if t in (57, 58, 59):
-        return "band, bias last"
-    if t in (64, 65) or 76 <= t <= 79 or 102 <= t <= 108:
+    if t in (57, 58, 59, 64, 65) or 76 <= t <= 79:
         return "band"
     return "taps"
 

@@ -17,6 +17,7 @@ from vdamd import lib
 pytestmark = pytest.mark.gpu
 
 SMALL = list(range(92, 102))
+BANDS = [57, 58, 59, 64, 65, 76, 77, 78, 79]
 
 
 def run_tiles(d, dy, shape, tiles):
@@ -215,13 +216,13 @@ def test_band_tiles_bitwise(B, H, W, IC, OC, res, relu):
         d.residual = keep[3].ptr
     dy = lib.DeviceBuffer(B * H * W * OC * 2)
     d.y = dy.ptr
-    outs = run_tiles(d, dy, (B, H, W, OC), [-1] + list(range(102, 109)))
-    assert len(outs) == 8, sorted(outs)
+    outs = run_tiles(d, dy, (B, H, W, OC), [-1] + BANDS)
+    assert len(outs) == 10, sorted(outs)
     d.w_chunked = keep[4].ptr
-    chunked = run_tiles(d, dy, (B, H, W, OC), [-1] + list(range(102, 109)))
+    chunked = run_tiles(d, dy, (B, H, W, OC), [-1] + BANDS)
     for o in (outs, chunked):
         for t in o:
-            assert np.array_equal(o[t], outs[103]), f"tile {t}"
+            assert np.array_equal(o[t], outs[64]), f"tile {t}"
     xp = np.pad(x.astype(np.float64), ((0, 0), (1, 1), (1, 1), (0, 0)))
     want, mag = b + np.zeros((B, H, W, OC)), np.abs(b) + np.zeros((B, H, W, OC))
     for kh in range(3):
@@ -312,11 +313,11 @@ def test_slim_split_bitwise(B, H, W, IC, OC, split, groups):
         d.x_group, d.x_group_stride, d.y_group, d.y_group_stride = 32, 64, 32, 64
     dy = lib.DeviceBuffer(B * H * W * 2 * OC * 2)
     d.y, d.y_stride, d.y_lo = dy.ptr, 2 * OC, OC
-    outs = run_tiles(d, dy, (B, H, W, 2 * OC), [-1, 26, 28, 30, 72, 74, 75, 109])
-    assert 109 in outs and len(outs) >= 3, sorted(outs)
+    outs = run_tiles(d, dy, (B, H, W, 2 * OC), [-1, 26, 28, 30, 72, 74, 75, 102])
+    assert 102 in outs and len(outs) >= 3, sorted(outs)
     for t, o in outs.items():
-        assert np.array_equal(o, outs[109]), f"tile {t}"
-    o = outs[109].view(np.float16).astype(np.float64)
+        assert np.array_equal(o, outs[102]), f"tile {t}"
+    o = outs[102].view(np.float16).astype(np.float64)
     got = o[..., :OC] + o[..., OC:]
     want = np.stack([O.conv2d_g(x[c].transpose(2, 0, 1), np.ascontiguousarray(w.transpose(0, 3, 1, 2)), ph=1, pw=1,
                                 bias=bias, f64=True) for c in range(B)])

@@ -2169,262 +2169,6 @@ void launch_sp(const ConvArgs& a, hipStream_t s) {
 }
 
 // ---------------------------------------------------------------------------
-// conv3x3_band_kernel: stride-1 3x3 conv (pad 1) for the wide layers
-// (IC % 16 == 0, OC % 128 == 0).  A workgroup of 8 waves owns a band of TH
-// full image rows of one clip and 128 output channels; the band's pixels,
-// flattened row-major, form NB = 2*NBW MFMA column blocks of 32 (so a
-// 75- or 38-wide map wastes at most a couple of percent of the lanes, where
-// 32-wide row tiles would waste 22-40 %).  Per 16-channel chunk of the input
-// the workgroup DMAs into LDS
-//   * the weights of all 9 taps for its 128 output channels (rows (tap, oc)
-//     of 32 bytes, the two 16-byte halves swapped on every other group of 8
-//     rows so an operand read of 16 consecutive rows hits 16 distinct bank
-//     groups), and
-//   * the band's (TH+2) x (W+2) input halo (48-byte rows: 32 bytes of
-//     channels + 16 of padding, so 16 consecutive rows start in 16 distinct
-//     bank groups and a tap is a constant offset from a lane's base row),
-// double-buffered: chunk k+1 is in flight while chunk k runs 9 taps x NBW
-// MFMAs per wave (wave w: output channels 32*(w%4).., column blocks
-// NBW*(w/4)..).  Every B fragment is read once per tap from the halo instead
-// of being re-fetched per tap as an im2col row.  The epilogue stages each
-// 32x32 block per wave through LDS and runs the shared epilogue (epi8, store8) on
-// 16-byte channel rows.  Products and sums are the other conv kernels'
-// (f16 x f16 -> f32, tap-major / channel-minor within a chunk).
-// ---------------------------------------------------------------------------
-template <int TH, int NBW>
-struct BandTile {
-    static constexpr int NW = 8, OCB = 128;
-    static constexpr int A_BYTES = 9 * OCB * 32, A_INS = A_BYTES / 1024;   // weights of one chunk
-    static constexpr int NB = 2 * NBW;                                    // column blocks per band
-    static constexpr int MAXW = NB * 32 / TH;                             // widest map a band holds
-    static constexpr int XPIX = (TH + 2) * (MAXW + 2);                    // halo pixels, upper bound
-    static constexpr int RB = 48;                                         // halo row bytes
-    static constexpr int X_INS = (XPIX * 3 + 63) / 64;
-    static constexpr int A_IPW = (A_INS + NW - 1) / NW, X_IPW = (X_INS + NW - 1) / NW;
-    static constexpr int STAGE = A_BYTES + X_INS * 1024;                  // one pipeline buffer pair
-    // epilogue: the band's residual rows (128 channels + 16 bytes of padding)
-    // and a 2 KB f16 staging block per wave, in the freed pipeline buffers
-    static constexpr int RRB = 272, RES_BYTES = NB * 32 * RRB, SBLK = 32 * 64;
-    static_assert(RES_BYTES + NW * SBLK <= 2 * STAGE, "the epilogue fits the pipeline buffers");
-};
-
-// Weight slot p of a chunk: row p/2 = (tap, oc), 16-byte half (p & 1) xor
-// ((row >> 3) & 1) of the row's 16 channels; recomputed per chunk from the
-// lane (a few integer ops) rather than held in registers across the loop.
-template <int TH, int NBW>
-__device__ __forceinline__ void band_issue(uint8_t* __restrict__ sa, uint8_t* __restrict__ sx, int c0, int oc0,
-                                           int IC, const int* xoff, __amdgpu_buffer_rsrc_t wr,
-                                           __amdgpu_buffer_rsrc_t xr, int wave, int lane) {
-    using G = BandTile<TH, NBW>;
-    asm volatile("" : "+v"(lane));
-#pragma unroll
-    for (int i = 0; i < G::A_IPW; ++i) {
-        const int ins = wave + i * G::NW;
-        if (ins >= G::A_INS) break;
-        const int p = ins * 64 + lane;
-        const int row = p >> 1, tap = row >> 7, oc = row & 127;
-        const int half = (p & 1) ^ ((row >> 3) & 1);
-        const uint32_t off = (uint32_t)((((oc0 + oc) * 9 + tap) * IC + c0) * 2 + half * 16);
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(wr, (lds_void*)(sa + ins * 1024), 16, off, 0, 0, 0);
-    }
-#pragma unroll
-    for (int i = 0; i < G::X_IPW; ++i) {
-        const int ins = wave + i * G::NW;
-        if (ins >= G::X_INS) break;
-        const uint32_t off = xoff[i] < 0 ? kOOB : (uint32_t)(xoff[i] + c0 * 2);
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(xr, (lds_void*)(sx + ins * 1024), 16, off, 0, 0, 0);
-    }
-}
-
-// One chunk: the next chunk's DMA (into the other buffer pair, passed as
-// distinct __restrict__ pointers so the reads below are not made to wait for
-// it), then 9 taps x NBW MFMAs with the fragment reads one tap ahead.
-template <int TH, int NBW>
-__device__ __forceinline__ void band_chunk(const uint8_t* __restrict__ sa, const uint8_t* __restrict__ sx,
-                                           uint8_t* __restrict__ sa_n, uint8_t* __restrict__ sx_n, bool prefetch,
-                                           int c0n, int oc0, int IC, const int* xoff, __amdgpu_buffer_rsrc_t wr,
-                                           __amdgpu_buffer_rsrc_t xr, int abase, int* bb, int hw,
-                                           float16v* acc, int wave, int lane) {
-    using G = BandTile<TH, NBW>;
-    if (prefetch) band_issue<TH, NBW>(sa_n, sx_n, c0n, oc0, IC, xoff, wr, xr, wave, lane);
-    // the B bases go behind an empty asm per chunk: otherwise the 9 x NBW
-    // (base + tap offset) sums are hoisted out of the chunk loop and spill
-#pragma unroll
-    for (int j = 0; j < NBW; ++j) asm volatile("" : "+v"(bb[j]));
-    // the 9 x NBW MFMAs as one sequence of steps (tap-major); B fragments are
-    // read D steps ahead through a D-slot ring, the next tap's A fragment at
-    // the first step of the current tap
-    constexpr int S = 9 * NBW, D = NBW > 4 ? 2 : 3;
-    half8 aq[2], bq[D];
-    auto load_a = [&](int tap, int slot) {
-        aq[slot] = *reinterpret_cast<const half8*>(sa + abase + tap * G::OCB * 32);
-    };
-    auto load_b = [&](int st, int slot) {
-        const int tap = st / NBW, j = st - tap * NBW;
-        const int kh = tap / 3, kw = tap - kh * 3;
-        bq[slot] = *reinterpret_cast<const half8*>(sx + bb[j] + (kh * hw + kw) * G::RB);
-    };
-    load_a(0, 0);
-#pragma unroll
-    for (int st = 0; st < D; ++st) load_b(st, st);
-    __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-    for (int st = 0; st < S; ++st) {
-        const int tap = st / NBW, j = st - tap * NBW;
-        const half8 cur = bq[st % D];
-        if (st + D < S) load_b(st + D, st % D);
-        if (j == 0 && tap + 1 < 9) load_a(tap + 1, (tap + 1) & 1);
-        __builtin_amdgcn_sched_barrier(0);
-        acc[j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(aq[tap & 1], cur, acc[j], 0, 0, 0);
-    }
-}
-
-template <int TH, int NBW>
-__global__ __launch_bounds__(512) void conv3x3_band_kernel(ConvArgs a) {
-    using G = BandTile<TH, NBW>;
-    __shared__ __attribute__((aligned(1024))) uint8_t smem[2 * G::STAGE];
-    uint8_t* const sa0 = smem;
-    uint8_t* const sx0 = smem + G::A_BYTES;
-    uint8_t* const sa1 = smem + G::STAGE;
-    uint8_t* const sx1 = sa1 + G::A_BYTES;
-
-    const int tid = threadIdx.x, lane = tid & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int lrow = lane & 31, lhalf = lane >> 5;
-    const int H = a.H, W = a.W, IC = a.IC, HW = W + 2;
-    const int bands = (H + TH - 1) / TH;
-    const int b = blockIdx.x / bands, r0 = (blockIdx.x - b * bands) * TH;
-    const int oc0 = blockIdx.y * G::OCB;
-    const int mb = wave & 3, ng = wave >> 2;
-    const int npx = TH * W;   // band pixels (rows past H are computed and dropped)
-
-    // this lane's halo DMA slots, as byte offsets at channel 0 (add 2*c0 per chunk)
-    int xoff[G::X_IPW];
-#pragma unroll
-    for (int i = 0; i < G::X_IPW; ++i) {
-        const int p = (wave + i * G::NW) * 64 + lane;
-        const int hrow = p / 3, s = p - hrow * 3;
-        const int hr = hrow / HW, hc = hrow - hr * HW;
-        const int ih = r0 - 1 + hr, iw = hc - 1;
-        const bool ok = s < 2 && hr < TH + 2 && ih >= 0 && ih < H && iw >= 0 && iw < W;
-        xoff[i] = ok ? (int)(((size_t)(b * H + ih) * W + iw) * a.xs * 2) + s * 16 : -1;
-    }
-    // operand read bases: A row (tap, mb*32 + lrow) with its halves swapped
-    // on odd groups of 8 rows; B halo row of pixel p = block*32 + lrow
-    const int abase = (mb * 32 + lrow) * 32 + ((lhalf ^ ((lrow >> 3) & 1)) * 16);
-    int bbase[NBW];
-#pragma unroll
-    for (int j = 0; j < NBW; ++j) {
-        int p = (ng * NBW + j) * 32 + lrow;
-        if (p >= npx) p = 0;   // masked lane: any valid row, result dropped
-        const int r = p / W, c = p - r * W;
-        bbase[j] = (r * HW + c) * G::RB + lhalf * 16;
-    }
-    const __amdgpu_buffer_rsrc_t wr =
-        __builtin_amdgcn_make_buffer_rsrc((void*)a.w, 0, (int)((size_t)a.OC * 9 * IC * 2), 0x00020000);
-    const __amdgpu_buffer_rsrc_t xr =
-        __builtin_amdgcn_make_buffer_rsrc((void*)a.x, 0, (int)(((size_t)(a.npix_in - 1) * a.xs + IC) * 2), 0x00020000);
-
-    float16v acc[NBW];
-#pragma unroll
-    for (int j = 0; j < NBW; ++j)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) acc[j][r] = 0.0f;
-
-    const int nk = IC / 16;
-    band_issue<TH, NBW>(sa0, sx0, 0, oc0, IC, xoff, wr, xr, wave, lane);
-#pragma unroll 1
-    for (int k = 0; k < nk; ++k) {
-        // chunk k: this wave's DMA has landed (nothing else is outstanding),
-        // then every wave's has, and chunk k-1's reads of the other pair are
-        // done.  One chunk per trip with the buffer pair picked per chunk (the
-        // inlined chunk keeps its distinct __restrict__ views, so its reads
-        // still do not wait for the other pair's DMA), which keeps the
-        // accumulators in one set of registers.
-        __builtin_amdgcn_s_waitcnt(0);
-        lds_barrier();
-        const bool odd = k & 1;
-        band_chunk<TH, NBW>(odd ? sa1 : sa0, odd ? sx1 : sx0, odd ? sa0 : sa1, odd ? sx0 : sx1, k + 1 < nk,
-                            (k + 1) * 16, oc0, IC, xoff, wr, xr, abase, bbase, HW, acc, wave, lane);
-    }
-    lds_barrier();   // every wave is done reading the buffers the epilogue reuses
-
-    // Epilogue y = act(acc + bias [+ residual]) in the MFMA layout (register
-    // g*4+e of a lane: channel 8g + 4*lhalf + e of its 32-channel block,
-    // pixel lrow of the column block).  The band's residual rows arrive in one
-    // DMA burst into the freed pipeline buffers and the bias sits in
-    // registers, so no global load waits behind a store; each finished 32x32
-    // block goes through the wave's f16 staging block to 16-byte channel-row
-    // stores.
-    const bool has_res = a.res != nullptr;
-    uint8_t* const sres = smem;
-    uint8_t* const sstg = smem + G::RES_BYTES + wave * G::SBLK;
-    const int ocw = oc0 + mb * 32;                   // this wave's first output channel
-    float bias[16];
-#pragma unroll
-    for (int g = 0; g < 4; ++g)
-#pragma unroll
-        for (int e = 0; e < 4; ++e) bias[g * 4 + e] = a.bias ? a.bias[ocw + g * 8 + lhalf * 4 + e] : 0.0f;
-    if (has_res) {
-        const __amdgpu_buffer_rsrc_t rr = __builtin_amdgcn_make_buffer_rsrc(
-            (void*)a.res, 0, (int)(((size_t)(a.npix - 1) * a.rs + a.OC) * 2), 0x00020000);
-        constexpr int SPR = G::RRB / 16;             // 17 slots per row, the last is padding
-        const int nins = (npx * SPR + 63) / 64;
-        for (int ins = wave; ins < nins; ins += G::NW) {
-            const int p = ins * 64 + lane;
-            const int px = p / SPR, ch = p - px * SPR;
-            const int r = px / W, c = px - r * W;
-            const bool ok = ch < 16 && px < npx && r0 + r < H;
-            const uint32_t off =
-                ok ? (uint32_t)((((size_t)(b * H + r0 + r) * W + c) * a.rs + oc0) * 2 + ch * 16) : kOOB;
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(rr, (lds_void*)(sres + ins * 1024), 16, off, 0, 0, 0);
-        }
-    }
-    __builtin_amdgcn_s_waitcnt(0);
-    lds_barrier();
-    half_t* const y = static_cast<half_t*>(a.y);
-    const bool relu = a.act == VDK_ACT_RELU;
-#pragma unroll
-    for (int j = 0; j < NBW; ++j) {
-        const int p0 = (ng * NBW + j) * 32;
-        int pr = p0 + lrow;
-        pr = pr < npx ? pr : npx - 1;
-        const uint8_t* const rrow = sres + pr * G::RRB + (mb * 32 + lhalf * 4) * 2;
-        uint8_t* const srow = sstg + lrow * 64 + lhalf * 8;
-        // the block's 4 residual reads go out together (zero without a residual)
-        half4 r4[4];
-#pragma unroll
-        for (int g = 0; g < 4; ++g) {
-            r4[g] = has_res ? *reinterpret_cast<const half4*>(rrow + g * 16) : half4{};
-        }
-#pragma unroll
-        for (int g = 0; g < 4; ++g) {
-            half4 h;
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                const float v = acc[j][g * 4 + e] + bias[g * 4 + e] + (float)r4[g][e];
-                h[e] = (half_t)(relu ? fmaxf(v, 0.0f) : v);
-            }
-            *reinterpret_cast<half4*>(srow + (swz<32>(lrow, g) * 16)) = h;
-        }
-#pragma unroll
-        for (int hp = 0; hp < 2; ++hp) {
-            const int pix = hp * 16 + (lane >> 2), ch = lane & 3;
-            const half8 v8 = *reinterpret_cast<const half8*>(sstg + pix * 64 + swz<32>(pix, ch) * 16);
-            const int p = p0 + pix, r = p / W, c = p - r * W;
-            if (p < npx && r0 + r < H)
-                *reinterpret_cast<half8*>(y + ((size_t)(b * H + r0 + r) * W + c) * a.ys + ocw + ch * 8) = v8;
-        }
-    }
-}
-
-template <int TH, int NBW>
-void launch_band(const ConvArgs& a, hipStream_t s) {
-    const int B = a.npix / (a.Ho * a.Wo);
-    hipLaunchKernelGGL((conv3x3_band_kernel<TH, NBW>), dim3(B * cdiv(a.H, TH), a.OC / 128), dim3(512), 0, s, a);
-}
-
-// ---------------------------------------------------------------------------
 // conv3x3_bandws_kernel: stride-1 3x3 conv (pad 1) for OC % 128 == 0, one
 // workgroup per band of TH rows x 128 output channels (flattened 32-pixel MFMA
 // blocks); maps wider than MAXW are cut into column segments of equal width,
@@ -3037,7 +2781,7 @@ struct TileCfg {
     void (*launch)(const ConvArgs&, hipStream_t);
     bool halo;       // 3x3 stride-1 pad-1 dilation-1 only
     int rw_ic = 0;   // register-weight kernels: exactly IC = rw_ic and OC = bm, plain epilogue
-    int band_w = 0;  // band kernels: W <= band_w, OC % 128 == 0, IC % 16 == 0
+    bool band = false;   // band kernels and the 32 x 32 tiles of their sums: OC % bm == 0, IC % 16 == 0
     int sp_ic = 0;   // split-f16 register-weight kernels: exactly IC = sp_ic and OC = bm, split 2
     bool gemm = false;   // the GEMM kernel with producer / compute waves: no reflect / q8_0
     bool gemm_ext = false;   // ... and its prologue / segment-sum variants (1x1, no padding)
@@ -3046,20 +2790,17 @@ struct TileCfg {
 // Entries 0-13 are the register-staged kernel (any layout; the only one with
 // KC=16 for IC % 32 != 0), 14-25 the LDS-DMA kernel, 26-32 the halo kernel,
 // 33-52 LDS-DMA tiles with 8 waves per workgroup, 53-56 the register-weight
-// persistent 3x3 kernel, 57-59 the band kernel for wide 3x3 layers, 60-61
-// narrow LDS-DMA tiles, 62-63 narrow register-staged tiles, 64-65 the band
-// kernel with producer / compute waves (128-channel groups, maps up to 75 /
-// 38 wide), 66-69 the register-weight kernel with 3- and 4-stage rings,
-// 70-75 the split-f16 register-weight kernel (ERes2Net's group convs), 76-79
-// the producer / compute band kernel on one-row bands (the same sums in the
-// same order as its 5-row bands, so the same bits, on 5x the workgroups), 80
+// persistent 3x3 kernel, 57-59, 64-65 and 76-79 the band kernel with producer /
+// compute waves (maps of any width in column segments of up to 75 / 38) on
+// three-, five- and one-row bands and its sums on 32 x 32 tiles (59), all the
+// same bits (pick_band), 60-61 narrow LDS-DMA tiles, 62-63 narrow
+// register-staged tiles, 66-69 the register-weight kernel with 3- and 4-stage
+// rings, 70-75 the split-f16 register-weight kernel (ERes2Net's group convs), 80
 // the register-staged 64x64 tile with 64-channel chunks, 81-84 the 1x1 GEMM
 // kernel with producer / compute waves, 85-88 narrow tiles of that kernel
 // with the prologue / segment-sum variants, 92-101 the GEMM kernel's tiles for
 // launches that leave the chip partly idle (deep rings of 64- and 128-channel
-// chunks; pick_small_tile), 102 the band kernels' sums on 32 x 32 tiles, 103-108
-// the producer / compute band kernel on column segments of any map (pick_band),
-// 109 the halo kernel's split-f16 sums on 32 x 32 tiles.
+// chunks; pick_small_tile), 102 the halo kernel's split-f16 sums on 32 x 32 tiles.
 
 // Tile table.  Wave tiles are WM x WN = (bm / waves_m) x (bn / waves_n) with
 // 4 waves per workgroup; entries are selected per layer by pick_tile().
@@ -3121,59 +2862,52 @@ const TileCfg kTiles[] = {
     {64, 192, 64, launch_rw<64, 64, 6, 8, 2>, true, 64},  // 54
     {64, 64, 64, launch_rw<64, 64, 2, 8, 2>, true, 64},   // 55
     {32, 128, 32, launch_rw<32, 32, 4, 8, 2>, true, 32},  // 56
-    {128, 384, 16, launch_band<5, 6>, true, 0, BandTile<5, 6>::MAXW},   // 57: band kernels
-    {128, 192, 16, launch_band<5, 3>, true, 0, BandTile<5, 3>::MAXW},   // 58
-    {128, 320, 16, launch_band<4, 5>, true, 0, BandTile<4, 5>::MAXW},   // 59
+    {128, 256, 16, launch_bandws<3, 75, 2, 4, 2, 4>, true, 0, true},   // 57: three-row bands
+    {128, 128, 16, launch_bandws<3, 38, 2, 2, 2, 4>, true, 0, true},   // 58
+    {32, 32, 16, launch_slim, true, 0, true},                          // 59: the bands' sums on 32 x 32 tiles
     {32, 64, 32, launch_dma<32, 64, 32, 32, 32, 2>},      // 60: narrow DMA tiles (OC = 32, few pixels)
     {32, 128, 32, launch_dma<32, 128, 32, 32, 32, 2>},    // 61
     {128, 32, 32, launch_igemm<128, 32, 64, 32, 32>},     // 62: register-staged, more workgroups
     {64, 64, 32, launch_igemm<64, 64, 32, 32, 32>},       // 63
-    {128, 384, 16, launch_bandws<5, 75, 2, 4, 3, 4>, true, 0, 75},   // 64: producer / compute band kernels
-    {128, 192, 16, launch_bandws<5, 38, 2, 2, 3, 4>, true, 0, 38},   // 65
+    {128, 384, 16, launch_bandws<5, 75, 2, 4, 3, 4>, true, 0, true},   // 64: five-row bands
+    {128, 192, 16, launch_bandws<5, 38, 2, 2, 3, 4>, true, 0, true},   // 65
     {64, 128, 64, launch_rw<64, 64, 4, 8, 3>, true, 64},  // 66: register-weight kernel, deeper rings
     {64, 64, 64, launch_rw<64, 64, 2, 8, 4>, true, 64},   // 67
     {32, 128, 32, launch_rw<32, 32, 4, 8, 4>, true, 32},  // 68
     {32, 256, 32, launch_rw<32, 32, 8, 8, 3>, true, 32},  // 69
-    {16, 256, 32, launch_sp<32, 16, 8, 8, 3, true>, true, 0, 0, 32},    // 70: split-f16 register-weight 3x3
-    {16, 256, 16, launch_sp<16, 16, 8, 8, 4, true>, true, 0, 0, 16},    // 71
-    {32, 256, 32, launch_sp<32, 32, 8, 8, 3, false>, true, 0, 0, 32},   // 72
-    {32, 64, 64, launch_sp<64, 32, 2, 4, 4, true>, true, 0, 0, 64},     // 73
-    {32, 128, 64, launch_sp<64, 32, 4, 4, 2, false>, true, 0, 0, 64},   // 74
-    {64, 128, 64, launch_sp<64, 64, 4, 8, 2, false>, true, 0, 0, 64},   // 75
-    {128, 96, 16, launch_bandws<1, 75, 4, 1, 3, 4>, true, 0, 75},   // 76: one-row bands (small batches)
-    {128, 96, 16, launch_bandws<1, 75, 4, 3, 1, 4>, true, 0, 75},   // 77
-    {128, 64, 16, launch_bandws<1, 38, 4, 1, 2, 4>, true, 0, 38},   // 78
-    {128, 64, 16, launch_bandws<1, 38, 4, 2, 1, 4>, true, 0, 38},   // 79
+    {16, 256, 32, launch_sp<32, 16, 8, 8, 3, true>, true, 0, false, 32},    // 70: split-f16 register-weight 3x3
+    {16, 256, 16, launch_sp<16, 16, 8, 8, 4, true>, true, 0, false, 16},    // 71
+    {32, 256, 32, launch_sp<32, 32, 8, 8, 3, false>, true, 0, false, 32},   // 72
+    {32, 64, 64, launch_sp<64, 32, 2, 4, 4, true>, true, 0, false, 64},     // 73
+    {32, 128, 64, launch_sp<64, 32, 4, 4, 2, false>, true, 0, false, 64},   // 74
+    {64, 128, 64, launch_sp<64, 64, 4, 8, 2, false>, true, 0, false, 64},   // 75
+    {128, 96, 16, launch_bandws<1, 75, 4, 1, 3, 4>, true, 0, true},   // 76: one-row bands (small batches)
+    {128, 96, 16, launch_bandws<1, 75, 4, 3, 1, 4>, true, 0, true},   // 77
+    {128, 64, 16, launch_bandws<1, 38, 4, 1, 2, 4>, true, 0, true},   // 78
+    {128, 64, 16, launch_bandws<1, 38, 4, 2, 1, 4>, true, 0, true},   // 79
     {64, 64, 64, launch_igemm<64, 64, 32, 32, 64>},       // 80: register-staged, 64-channel chunks
-    {128, 256, 64, launch_gemm_ws<128, 256, 2, 4, 64, 3, 4>, false, 0, 0, 0, true},   // 81: 1x1 GEMMs, producer / compute waves
-    {128, 384, 32, launch_gemm_ws<128, 384, 2, 4, 32, 4, 4>, false, 0, 0, 0, true},   // 82
-    {256, 128, 64, launch_gemm_ws<256, 128, 4, 2, 64, 3, 4>, false, 0, 0, 0, true},   // 83
-    {128, 288, 64, launch_gemm_ws<128, 288, 2, 3, 64, 3, 4>, false, 0, 0, 0, true},   // 84
-    {128, 64, 32, launch_gemm_ws<128, 64, 2, 2, 32, 4, 2, true>, false, 0, 0, 0, true, true},   // 85: narrow GEMMs
-    {128, 64, 64, launch_gemm_ws<128, 64, 2, 2, 64, 3, 2, true>, false, 0, 0, 0, true, true},   // 86
-    {128, 32, 32, launch_gemm_ws<128, 32, 4, 1, 32, 4, 2, true>, false, 0, 0, 0, true, true},   // 87
-    {64, 64, 32, launch_gemm_ws<64, 64, 2, 2, 32, 4, 2, true>, false, 0, 0, 0, true, true},     // 88
-    {128, 256, 64, launch_gemm_ws<128, 256, 2, 4, 64, 3, 4, true>, false, 0, 0, 0, true, true},   // 89: wide, + prologue
-    {256, 128, 64, launch_gemm_ws<256, 128, 4, 2, 64, 3, 4, true>, false, 0, 0, 0, true, true},   // 90
-    {128, 384, 32, launch_gemm_ws<128, 384, 2, 4, 32, 4, 4, true>, false, 0, 0, 0, true, true},   // 91
-    {32, 32, 128, launch_gemm_ws<32, 32, 1, 1, 128, 4, 4, true>, false, 0, 0, 0, true, true},     // 92: small launches
-    {32, 32, 64, launch_gemm_ws<32, 32, 1, 1, 64, 8, 2, true>, false, 0, 0, 0, true, true},       // 93
-    {32, 32, 32, launch_gemm_ws<32, 32, 1, 1, 32, 16, 2, true>, false, 0, 0, 0, true, true},      // 94
-    {64, 32, 128, launch_gemm_ws<64, 32, 2, 1, 128, 3, 4>, false, 0, 0, 0, true},                 // 95
-    {64, 64, 128, launch_gemm_ws<64, 64, 2, 2, 128, 4, 4, true>, false, 0, 0, 0, true, true},     // 96
-    {64, 64, 128, launch_gemm_ws<64, 64, 2, 2, 128, 2, 4>, false, 0, 0, 0, true},                 // 97
-    {64, 64, 64, launch_gemm_ws<64, 64, 2, 2, 64, 4, 4, true>, false, 0, 0, 0, true, true},       // 98
-    {32, 64, 32, launch_gemm_ws<32, 64, 1, 2, 32, 8, 2>, false, 0, 0, 0, true},                   // 99
-    {128, 64, 128, launch_gemm_ws<128, 64, 2, 2, 128, 3, 4>, false, 0, 0, 0, true},               // 100
-    {128, 128, 64, launch_gemm_ws<128, 128, 4, 2, 64, 4, 4>, false, 0, 0, 0, true},               // 101
-    {32, 32, 16, launch_slim, true, 0, 1 << 20},       // 102: the band kernels' sums on 32 x 32 tiles
-    {128, 384, 16, launch_bandws<5, 75, 2, 4, 3, 4>, true, 0, 1 << 20},  // 103: bands of column segments (wide maps)
-    {128, 192, 16, launch_bandws<5, 38, 2, 2, 3, 4>, true, 0, 1 << 20},  // 104
-    {128, 256, 16, launch_bandws<3, 75, 2, 4, 2, 4>, true, 0, 1 << 20},  // 105: three-row bands
-    {128, 128, 16, launch_bandws<3, 38, 2, 2, 2, 4>, true, 0, 1 << 20},  // 106
-    {128, 96, 16, launch_bandws<1, 75, 4, 3, 1, 4>, true, 0, 1 << 20},   // 107: one-row bands
-    {128, 64, 16, launch_bandws<1, 38, 4, 1, 2, 4>, true, 0, 1 << 20},   // 108
-    {32, 32, 32, launch_slim_split, true},                // 109: the halo kernel's split-f16 sums on 32 x 32 tiles
+    {128, 256, 64, launch_gemm_ws<128, 256, 2, 4, 64, 3, 4>, false, 0, false, 0, true},   // 81: 1x1 GEMMs, producer / compute waves
+    {128, 384, 32, launch_gemm_ws<128, 384, 2, 4, 32, 4, 4>, false, 0, false, 0, true},   // 82
+    {256, 128, 64, launch_gemm_ws<256, 128, 4, 2, 64, 3, 4>, false, 0, false, 0, true},   // 83
+    {128, 288, 64, launch_gemm_ws<128, 288, 2, 3, 64, 3, 4>, false, 0, false, 0, true},   // 84
+    {128, 64, 32, launch_gemm_ws<128, 64, 2, 2, 32, 4, 2, true>, false, 0, false, 0, true, true},   // 85: narrow GEMMs
+    {128, 64, 64, launch_gemm_ws<128, 64, 2, 2, 64, 3, 2, true>, false, 0, false, 0, true, true},   // 86
+    {128, 32, 32, launch_gemm_ws<128, 32, 4, 1, 32, 4, 2, true>, false, 0, false, 0, true, true},   // 87
+    {64, 64, 32, launch_gemm_ws<64, 64, 2, 2, 32, 4, 2, true>, false, 0, false, 0, true, true},     // 88
+    {128, 256, 64, launch_gemm_ws<128, 256, 2, 4, 64, 3, 4, true>, false, 0, false, 0, true, true},   // 89: wide, + prologue
+    {256, 128, 64, launch_gemm_ws<256, 128, 4, 2, 64, 3, 4, true>, false, 0, false, 0, true, true},   // 90
+    {128, 384, 32, launch_gemm_ws<128, 384, 2, 4, 32, 4, 4, true>, false, 0, false, 0, true, true},   // 91
+    {32, 32, 128, launch_gemm_ws<32, 32, 1, 1, 128, 4, 4, true>, false, 0, false, 0, true, true},     // 92: small launches
+    {32, 32, 64, launch_gemm_ws<32, 32, 1, 1, 64, 8, 2, true>, false, 0, false, 0, true, true},       // 93
+    {32, 32, 32, launch_gemm_ws<32, 32, 1, 1, 32, 16, 2, true>, false, 0, false, 0, true, true},      // 94
+    {64, 32, 128, launch_gemm_ws<64, 32, 2, 1, 128, 3, 4>, false, 0, false, 0, true},                 // 95
+    {64, 64, 128, launch_gemm_ws<64, 64, 2, 2, 128, 4, 4, true>, false, 0, false, 0, true, true},     // 96
+    {64, 64, 128, launch_gemm_ws<64, 64, 2, 2, 128, 2, 4>, false, 0, false, 0, true},                 // 97
+    {64, 64, 64, launch_gemm_ws<64, 64, 2, 2, 64, 4, 4, true>, false, 0, false, 0, true, true},       // 98
+    {32, 64, 32, launch_gemm_ws<32, 64, 1, 2, 32, 8, 2>, false, 0, false, 0, true},                   // 99
+    {128, 64, 128, launch_gemm_ws<128, 64, 2, 2, 128, 3, 4>, false, 0, false, 0, true},               // 100
+    {128, 128, 64, launch_gemm_ws<128, 128, 4, 2, 64, 4, 4>, false, 0, false, 0, true},               // 101
+    {32, 32, 32, launch_slim_split, true},                // 102: the halo kernel's split-f16 sums on 32 x 32 tiles
 };
 constexpr int kNumTiles = (int)(sizeof(kTiles) / sizeof(kTiles[0]));
 
@@ -3181,7 +2915,7 @@ bool is_s1_3x3(const ConvArgs& a) {
     return a.KH == 3 && a.KW == 3 && a.sh == 1 && a.sw == 1 && a.ph == 1 && a.pw == 1 && a.dh == 1 && a.dw == 1;
 }
 
-constexpr int kFirstSlimSplit = 109;   // the split-f16 3x3 kernel for small launches
+constexpr int kFirstSlimSplit = 102;   // the split-f16 3x3 kernel for small launches
 constexpr int kFirstSmall = 92;   // the GEMM kernel's small-launch tiles
 constexpr int kFirstDma = 14;   // then the halo tiles from 26, 8-wave DMA tiles from 33
 
@@ -3213,11 +2947,11 @@ bool tile_fits(const TileCfg& t, const ConvArgs& a) {
     if (t.halo && !is_s1_3x3(a)) return false;
     // the register-weight, band and 32 x 32 3x3 kernels store the rows they
     // read, whole: no cropped outputs (the halo tiles take those)
-    if (a.Wo != a.W && (t.rw_ic || t.sp_ic || t.band_w || idx >= kFirstSlimSplit)) return false;
+    if (a.Wo != a.W && (t.rw_ic || t.sp_ic || t.band || idx >= kFirstSlimSplit)) return false;
     // the input prologue lives in the register-staged kernel's operand loads
     // and the LDS-DMA kernel's B fragments (up to 1024 input channels: their
     // scale / shift stage in LDS)
-    if (a.in_scale && (t.halo || t.rw_ic || t.band_w || a.IC > 1024)) return false;
+    if (a.in_scale && (t.halo || t.rw_ic || t.band || a.IC > 1024)) return false;
     // reflect padding lives in the LDS-DMA kernel's pixel offsets (one row
     // of at most 32 taps)
     if (a.reflect && (igemm_tile(idx) || t.halo || a.KH * a.KW > 32)) return false;
@@ -3250,12 +2984,12 @@ bool tile_fits(const TileCfg& t, const ConvArgs& a) {
                (!a.split || a.x_lo % 8 == 0);
     }
     // 16-channel group strides: the LDS-DMA kernel's offsets and the shared store
-    if ((a.xgs != (1 << a.xgl) || a.ygs != (1 << a.ygl)) && (igemm_tile(idx) || t.halo || t.rw_ic || t.band_w))
+    if ((a.xgs != (1 << a.xgl) || a.ygs != (1 << a.ygl)) && (igemm_tile(idx) || t.halo || t.rw_ic || t.band))
         return false;
     // a DMA chunk covers whole groups
     if (a.xgl == 5 && t.kc % 32 != 0) return false;
     if (t.rw_ic) return a.IC == t.rw_ic && a.OC == t.bm && plain_epilogue(a);
-    if (t.band_w) return plain_epilogue(a) && a.W <= t.band_w && a.OC % t.bm == 0 && a.IC % 16 == 0;
+    if (t.band) return plain_epilogue(a) && a.OC % t.bm == 0 && a.IC % 16 == 0;
     // split: the DMA and halo kernels only (IC % kc == 0 below keeps a chunk inside one plane)
     if (a.split && (igemm_tile(idx) || idx >= 62)) return false;
     return a.IC % t.kc == 0;
@@ -3325,16 +3059,16 @@ long round_cost(const ConvArgs& a, int t) {
 // measured at 128 and 256 channels, single launches with inputs flushed to
 // HBM); the least total wins.  Against the rule before (5-row bands, one-row
 // ones under 48 workgroups, LDS-DMA tiles on maps wider than 75 / 38): 20 x 75
-// x 128 14.6 -> 8.8 us at batch 1 (102), 27.4 -> 16.8 at batch 16 (106), 29.2
-// -> 22.4 at batch 32 (104); 20 x 126 x 128 at batch 16 34.7 -> 22.1 (104);
-// 10 x 38 x 256 16.8 -> 10.8 at batch 1 (102), 27.9 -> 22.6 at batch 16 (106);
-// 10 x 63 x 256 at batch 64 68.8 -> 53.3 (103).
+// x 128 14.6 -> 8.8 us at batch 1 (59), 27.4 -> 16.8 at batch 16 (58), 29.2
+// -> 22.4 at batch 32 (65); 20 x 126 x 128 at batch 16 34.7 -> 22.1 (65);
+// 10 x 38 x 256 16.8 -> 10.8 at batch 1 (59), 27.9 -> 22.6 at batch 16 (58);
+// 10 x 63 x 256 at batch 64 68.8 -> 53.3 (64).
 int pick_band(const ConvArgs& a) {
     if (!is_s1_3x3(a) || a.OC % 128 != 0 || !plain_epilogue(a)) return -1;
     struct BandCost { int tile, th, maxw; float base, per; };
     static const BandCost kBands[] = {
-        {103, 5, 75, 9.5f, 1.56f}, {104, 5, 38, 6.0f, 1.06f}, {105, 3, 75, 7.5f, 1.06f},
-        {106, 3, 38, 4.5f, 0.81f}, {107, 1, 75, 3.5f, 0.81f}, {108, 1, 38, 3.1f, 0.64f},
+        {64, 5, 75, 9.5f, 1.56f}, {65, 5, 38, 6.0f, 1.06f}, {57, 3, 75, 7.5f, 1.06f},
+        {58, 3, 38, 4.5f, 0.81f}, {77, 1, 75, 3.5f, 0.81f}, {78, 1, 38, 3.1f, 0.64f},
     };
     const int chunks = a.IC / 16, B = a.npix / (a.Ho * a.Wo);
     const auto rounds = [](long wgs) { return (float)((wgs + 255) / 256); };
@@ -3348,15 +3082,14 @@ int pick_band(const ConvArgs& a) {
     // the 32 x 32 tiles: two workgroups share a CU
     const long w32 = (long)cdiv(a.npix, 32) * (a.OC / 32);
     const float slim = w32 <= 256 ? 2.3f + 0.25f * chunks : rounds(w32) * (1.0f + 0.275f * chunks);
-    if (best >= 0 && tile_fits(kTiles[102], a) && slim < cost) best = 102;
+    if (best >= 0 && tile_fits(kTiles[59], a) && slim < cost) best = 59;
     return best;
 }
 
 // Per-layer-class defaults, from a sweep of every ResNet34 conv shape at
 // batch 64 on MI355X (64-channel 3x3 stride-1 layers with the plain
-// epilogue: the register-weight kernel; 128-channel ones whose map is 39-76
-// wide: the band kernel, 256+-channel ones on maps up to 38 wide: the
-// 3-block band; the strided / 1x1 32 -> 64 convs: the register-staged 64x128
+// epilogue: the register-weight kernel; ones with 128-channel output groups:
+// the band kernels (pick_band); the strided / 1x1 32 -> 64 convs: the register-staged 64x128
 // tile; other narrow 3x3 stride-1 layers: the 32-channel halo tile;
 // 128 output channels: the 128x128 DMA tile with KC = 32; the rest: DMA
 // implicit GEMM with the widest OC tile that divides OC; IC % 32 != 0: the
@@ -3494,7 +3227,7 @@ int pick_wide_tile(const ConvArgs& a) {
         };
         const bool wide = a.IC == 128 && a.OC == 128 && a.H <= 10;
         const bool halo_order = a.OC == 32 ? any({28, 72, 74}) : (a.OC == 64 ? any({30, 75}) : wide && any({26}));
-        if (halo_order && (long)cdiv(a.npix, 32) * cdiv(a.OC, 32) <= 512 && tile_fits(kTiles[109], a)) return 109;
+        if (halo_order && (long)cdiv(a.npix, 32) * cdiv(a.OC, 32) <= 512 && tile_fits(kTiles[102], a)) return 102;
         // then 32-column tiles while the 64-column ones leave CUs idle (8 x 10 x 38: 23.2 -> 17.2 us)
         if (wide && (long)(a.npix / (a.Ho * a.Wo)) * cdiv(a.H, 4) * cdiv(a.W, 64) * 4 < 256 && tile_fits(kTiles[28], a))
             return 28;
@@ -3555,9 +3288,11 @@ int pick_wide_tile(const ConvArgs& a) {
         return cdiv(a.npix, 64) <= 256 && tile_fits(kTiles[98], a) ? 98 : 66;   // 66: 3-stage ring
     const int band = pick_band(a);
     if (band >= 0) return band;
-    // ResNet's stride-2 convs at small batches (under 8192 output pixels, e.g.
-    // batch 1), measured: the 3x3s from 64 / 128 channels on the 128x32 DMA
-    // tile (18.8 -> 9.6 / 13.7 us), the rest on the 64x64 register-staged tile
+    // stride-2 convs under 8192 output pixels that are past the small-launch
+    // limits (more output channels than ResNet34's own, which run there): the
+    // tiles that were the fastest of these kernels on ResNet34's at batch 1,
+    // the 128x32 DMA one for 3x3s from 64 / 128 channels (18.8 -> 9.6 / 13.7
+    // us against the 128x128 one), the 64x64 register-staged one for the rest
     // (32 -> 64 3x3 10.8 -> 7.0 us, the 1x1 shortcuts 9.1 -> 4.5 and 7.3 -> 5.1)
     if (!a.split && a.KH == a.KW && a.sh == 2 && a.sw == 2 && a.npix < 8192 && a.IC % 32 == 0 && a.OC % 64 == 0) {
         if (a.KH == 3 && a.IC % 64 == 0 && a.OC % 128 == 0 && tile_fits(kTiles[52], a)) return 52;
