@@ -4,8 +4,10 @@
  * Every entry point takes device pointers, plain sizes and a HIP stream
  * (`void* stream`, NULL = the default stream), enqueues its kernels and
  * returns 0, or a nonzero code with a message from vdk_last_error().  Nothing
- * here allocates device memory except vdk_malloc.  Shapes are checked on the
- * host before any launch.
+ * here allocates device memory except vdk_malloc, vdk_fbank (the workspace that
+ * vdk_fbank_ex takes from its caller), vdk_res2_block in place on clips of
+ * several time tiles (vdk_res2_block_out does not) and the opt-in tile tuning.
+ * Shapes are checked on the host before any launch.
  *
  * Layouts: PCM [B][n] f32; FBank features feat-major [B][n_mels][T] f32 (the
  * reference's [n_mels, T] per clip); activations NHWC f16 [B][H=freq][W=time][C];
@@ -320,7 +322,7 @@ int vdk_linear_ex_noalloc(const float* d_x, int batch, int in_dim, const float* 
 int vdk_feats_tmajor(const float* d_feats, const float* d_row_mean, int batch, int n_mels, int T, int pad,
                      int c_pad, void* d_out, void* stream);
 /* All scale - 1 dependent group convs of one SE-Res2Net block's Res2Net
- * (src/encoder.cpp:174-200) in one launch.  buf [B][T][stride] f16 holds
+ * (src/encoder.cpp:174-200), in place.  buf [B][T][stride] f16 holds
  * the block's groups in slots of G channels: x_m (tdnn1's output chunk m) in
  * slot m + 1; group j (1 .. scale-1) = conv_j(in_j) with in_1 = x_1 and
  * in_j = f16(v_{j-1} + x_j), conv_j the k = 3 dilated conv with reflect
@@ -328,7 +330,12 @@ int vdk_feats_tmajor(const float* d_feats, const float* d_row_mean, int batch, i
  * stored as f16 to slot 0 (j = 1) or slot j.  Weights [G][3][G] f16 (16-byte
  * aligned); scale / shift may be NULL (1 / 0).  The same bits as the groups
  * run one conv at a time (vdk_conv2d_ex with reflect_pad and the second
- * output).  G = 128, scale <= 8, T > dil, (scale - 1) * dil <= 64. */
+ * output).  G = 128, scale <= 8, T > dil, (scale - 1) * dil <= 64.
+ * One launch where a clip is one time tile (T <= 160 - 2 (scale - 1) dil).
+ * Longer clips are cut into tiles, and y_j's slot holds x_{j-1}, which a
+ * neighbouring tile still reads: their results go through a side buffer of
+ * batch * T * scale * G halfs, taken from the stream's memory pool and given
+ * back on the stream, and a second launch copies them in place. */
 typedef struct {
     const void* w[7]; const float* bias[7]; const float* scale[7]; const float* shift[7];
 } vdk_res2_weights;
@@ -336,8 +343,7 @@ int vdk_res2_block(void* d_buf, int stride, int batch, int T, int G, int scale, 
                    const vdk_res2_weights* w, void* stream);
 /* The same block into a buffer of its own: y [B][T][y_stride] = [y_1 | x_0 |
  * y_2 .. y_{scale-1}] in slots 0 .. scale - 1, x left as it was; x and y must
- * not overlap, y 16-byte aligned.  (In place, clips of several time tiles go
- * through a side buffer, allocated and freed on the stream.) */
+ * not overlap, y 16-byte aligned.  One launch at any T, and no allocation. */
 int vdk_res2_block_out(const void* d_x, int stride, int batch, int T, int G, int scale, int dil,
                        const vdk_res2_weights* w, void* d_y, int y_stride, void* stream);
 /* out [B][T+2*pad][G] = reflect_pad(a (+ b)) over time: the Res2Net group

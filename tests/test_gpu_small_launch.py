@@ -187,6 +187,41 @@ def test_res2_block_out_tiles(batch, T, dil, scale):
     assert (err <= 3 * G * 2.0 ** -24 * mag + 2.0 ** -11 * np.abs(want) + 2.0 ** -24).all()
 
 
+def pool_used():
+    """Bytes in use of the device's stream-ordered memory pool."""
+    hip, pool, used = lib.lib(), ctypes.c_void_p(), ctypes.c_uint64()
+    assert hip.hipDeviceGetDefaultMemPool(ctypes.byref(pool), 0) == 0
+    assert hip.hipMemPoolGetAttribute(pool, 7, ctypes.byref(used)) == 0   # hipMemPoolAttrUsedMemCurrent
+    return used.value
+
+
+def test_res2_block_in_place_gives_its_side_buffer_back():
+    """In place over several time tiles the results go through a side buffer
+    of the stream's pool: given back after the call, also when it fails on the
+    way (here on an error that an earlier HIP call left behind)."""
+    G, scale, T, dil, L = 128, 8, 400, 2, lib.lib()
+    announce("res2 block in place: the side buffer")
+    w, b = lib.DeviceBuffer.from_array(np.zeros((G, 3, G), np.float16)), lib.DeviceBuffer.from_array(np.zeros(G, np.float32))
+    rw = lib.Res2Weights()
+    for j in range(scale - 1):
+        rw.w[j], rw.bias[j] = w.ptr, b.ptr
+    S = (scale + 1) * G
+    buf = lib.DeviceBuffer.from_array(np.zeros((4, T, S), np.float16))
+    lib.check(L.vdk_synchronize())
+    used = pool_used()
+    lib.check(L.vdk_res2_block(buf.ptr, S, 4, T, G, scale, dil, rw, None))
+    lib.check(L.vdk_synchronize())
+    assert pool_used() == used
+    assert L.hipSetDevice(1 << 20) != 0
+    rc = L.vdk_res2_block(buf.ptr, S, 4, T, G, scale, dil, rw, None)
+    L.hipGetLastError()
+    lib.check(L.vdk_synchronize())
+    assert rc != 0
+    assert pool_used() == used
+    lib.check(L.vdk_res2_block(buf.ptr, S, 4, T, G, scale, dil, rw, None))
+    lib.check(L.vdk_synchronize())
+
+
 @pytest.mark.parametrize("B,H,W,IC,OC,res,relu", [
     (1, 20, 75, 128, 128, True, True),      # one segment, the 5-row band's own width
     (2, 7, 76, 128, 128, False, True),      # just past it: two segments of 38

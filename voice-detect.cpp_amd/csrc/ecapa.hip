@@ -839,16 +839,20 @@ extern "C" int vdk_res2_block(void* d_buf, int stride, int batch, int T, int G, 
         }
         // several tiles: y_j's slot holds x_{j-1}, which a neighbour that starts
         // late still reads on its halo, so the results go through a side buffer
-        void* tmp = nullptr;
+        // of the stream's pool, given back on every way out
+        struct Side {
+            hipStream_t s;
+            void* p = nullptr;
+            ~Side() { if (p) (void)hipFreeAsync(p, s); }
+        } side{s};
         const long rows = (long)batch * T;
-        VDK_HIP(hipMallocAsync(&tmp, (size_t)rows * scale * G * 2, s));
-        a.y = static_cast<half_t*>(tmp);
+        VDK_HIP(hipMallocAsync(&side.p, (size_t)rows * scale * G * 2, s));
+        a.y = static_cast<half_t*>(side.p);
         a.ys = scale * G;
         launch_res2(a, batch, s);
         hipLaunchKernelGGL(res2_copy_kernel, dim3(cdiv(rows * scale * (G / 8), 256)), dim3(256), 0, s, a.y,
                            static_cast<half_t*>(d_buf), rows, a.L, stride);
         VDK_HIP(hipGetLastError());
-        VDK_HIP(hipFreeAsync(tmp, s));
     });
 }
 
