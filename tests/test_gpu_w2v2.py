@@ -17,6 +17,7 @@ test_age_gender.cpp: age_raw and gender logits 1e-2, probabilities 1e-3),
 applied relative to the rms of each tensor.
 """
 import json
+import ctypes
 import os
 import tempfile
 import zlib
@@ -346,6 +347,34 @@ def test_analyze_small_matches_oracle(kind, dims):
         assert np.array_equal(solo[0], raw[1])
     finally:
         ctx.close()
+
+
+def test_kept_states_memory_comes_with_the_first_small_call():
+    """The hidden states that small calls keep (4 x 4096 rows of 256 here) take
+    memory from the first such call on, not in a context of large calls; the
+    results are those of a context of its own."""
+    path = _model("emotion", 5, SMALL)
+    pcm = synth.clips(33, 171, 8000)
+    free = ctypes.c_size_t(), ctypes.c_size_t()
+
+    def free_bytes():
+        lib.check(lib.lib().vdk_synchronize())
+        assert lib.lib().hipMemGetInfo(ctypes.byref(free[0]), ctypes.byref(free[1])) == 0
+        return free[0].value
+
+    ctx, own = lib.Context(path), lib.Context(path)
+    try:
+        assert 171 * ctx.analyze_frames(8000) > 4096
+        announce("analyze emotion small: 171 clips, then one")
+        want = own.analyze_pcm(pcm[1:2])
+        large = ctx.analyze_pcm(pcm)
+        before = free_bytes()
+        solo = ctx.analyze_pcm(pcm[1:2])
+        assert before - free_bytes() >= 4 * 4096 * 256 * 2
+        assert np.array_equal(solo, want) and np.array_equal(large[1], want[0])
+    finally:
+        ctx.close()
+        own.close()
 
 
 @pytest.mark.parametrize("kind", ["emotion", "age_gender"])

@@ -313,6 +313,7 @@ private:
     void upload_w2v2();
     void ensure_workspace(int batch, int n_samples);
     void alloc_w2v2_workspace(int batch, int n_samples);
+    bool reserve_states();
     void analyze_forward(const float* d_pcm, int batch, int n_samples, float* d_raw);
     void alloc_resnet_workspace(int batch, int T);
     void alloc_ecapa_workspace(int batch, int T);

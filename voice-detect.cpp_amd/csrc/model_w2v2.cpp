@@ -282,11 +282,9 @@ void Model::alloc_w2v2_workspace(int batch, int n) {
     w.wh1 = ws_alloc(2 * BT * H);
     // small launches of the post-norm stack keep every hidden state and pool
     // them in one launch at the end; larger ones pool state by state (their
-    // launches are long, and 13 states of 64 x 10 s would be 0.6 GB)
-    if (!c.stable_layer_norm && c.n_layers + 1 <= 32 && H % 8 == 0) {
-        w.state_rows = std::min<size_t>(BT, 4096);
-        w.wstates = ws_alloc(2 * w.state_rows * H * (c.n_layers + 1));
-    }
+    // launches are long, and 13 states of 64 x 10 s would be 0.6 GB).  The
+    // states' memory comes with the first call that keeps them.
+    if (!c.stable_layer_norm && c.n_layers + 1 <= 32 && H % 8 == 0) w.state_rows = std::min<size_t>(BT, 4096);
     w.qkv = ws_alloc(2 * BT * 3 * H);
     w.att = ws_alloc(2 * BT * H);
     w.ffb = ws_alloc(2 * BT * c.ff);
@@ -300,6 +298,24 @@ void Model::alloc_w2v2_workspace(int batch, int n) {
     fcw = std::max(fcw, vdk_linear_workspace_size(batch, H, 1));
     w.fc_work_bytes = fcw;
     w.fc_work = ws_alloc(fcw);
+}
+
+// The memory of the kept hidden states (82 MB for 4096 rows of base).  Without
+// it (none left, or the stream is being captured) the call pools state by
+// state, the same values.
+bool Model::reserve_states() {
+    if (ws_.wstates) return true;
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    VDK_HIP(hipStreamIsCapturing(stream_, &cap));
+    if (cap != hipStreamCaptureStatusNone) return false;
+    const size_t bytes = 2 * ws_.state_rows * cfg_.w2v2.hidden * (cfg_.w2v2.n_layers + 1);
+    if (hipMalloc(&ws_.wstates, bytes) != hipSuccess) {
+        (void)hipGetLastError();
+        ws_.wstates = nullptr;
+        return false;
+    }
+    ws_.allocs.push_back(ws_.wstates);
+    return true;
 }
 
 void Model::analyze_forward(const float* d_pcm, int batch, int n, float* d_raw) {
@@ -433,7 +449,8 @@ void Model::analyze_forward(const float* d_pcm, int batch, int n, float* d_raw) 
     } else {
         // post-norm (src/analyze_w2v2.cpp:429-468): hidden_states[0] is the
         // encoder LN of (projection + pos conv), then every layer's output
-        const bool keep = (size_t)BT <= w.state_rows && std::count(sw.begin(), sw.end(), 0.0f) + 1 < (long)sw.size();
+        const bool keep = (size_t)BT <= w.state_rows && std::count(sw.begin(), sw.end(), 0.0f) + 1 < (long)sw.size() &&
+                          reserve_states();
         auto state = [&](int i) -> void* {
             return keep ? static_cast<uint8_t*>(w.wstates) + 2 * w.state_rows * H * i : w.wh;
         };
