@@ -9,9 +9,10 @@
 // of the f64 sum.  Ranking: highest score first, equal scores by the lower row
 // index, so the result is deterministic.
 //
-// registry_score_kernel: the scores on f64 MFMA (v_mfma_f64_16x16x4), a
-// workgroup's chunk of rows staged in LDS and its best k rows per query picked
-// there; one sorted candidate list per query and chunk goes out.
+// registry_score_kernel: the scores on f64 MFMA (v_mfma_f64_16x16x4) from rows
+// and queries loaded straight to registers; the scores of a workgroup's chunk
+// of rows are staged in LDS and the best k rows per query picked there, one
+// candidate list per query and chunk (in no particular order for k > 16).
 // registry_merge_kernel: one workgroup per query picks the best k of its
 // candidates.
 #include <cfloat>
