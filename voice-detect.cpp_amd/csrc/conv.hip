@@ -2188,10 +2188,9 @@ void launch_sp(const ConvArgs& a, hipStream_t s) {
 //  * weights read from the chunk-major copy ([IC/16][9][OC][16],
 //    vdk_conv_desc.w_chunked) when there is one, so a DMA instruction's 64
 //    slots are one contiguous kilobyte instead of pieces of 32 cache lines;
-//  * accumulators that start at the bias; the residual added by two MFMAs per
-//    32x32 block with identity A operands (products r x 1, one rounding of
-//    acc + r), then [ReLU], f16, written over the residual rows, and stored
-//    as 16-byte channel chunks.
+//  * accumulators that start at the bias; the residual added in f32 by the lane
+//    that holds the output (one rounding of acc + r), then [ReLU], f16, written
+//    over the residual rows, and stored as 16-byte channel chunks.
 // Products are f16 x f16 with f32 accumulation in tap-major, channel-minor
 // order, like the other conv kernels, with the bias entering first.
 // ---------------------------------------------------------------------------
@@ -2229,42 +2228,6 @@ __device__ __forceinline__ uint32_t band_woff(int p, int c0, int oc0, int IC, in
 // at least 1/(2d) away from an integer, far beyond the float rounding error.
 __device__ __forceinline__ int div_small(int n, float inv_d) {
     return (int)(((float)n + 0.5f) * inv_d);
-}
-
-// acc + residual of a 32-channel x 32-pixel block through MFMAs with identity A
-// operands (products r x 1, one rounding): lane (lrow, lhalf) passes channels
-// h * 16 + lhalf * 8 .. + 7 of pixel lrow in rv[h].  An infinite or NaN residual
-// would reach the pixel's other channels too (0 x Inf), in every accumulator:
-// such a block runs again with finite residuals, and each lane adds the others
-// to its own outputs (own(g): the residuals of registers g*4 .. + 3).
-template <class Own>
-__device__ __forceinline__ float16v add_residual_block(const half8* rv, const float16v& acc, int lrow, int lhalf, Own own) {
-    half8 eye[2];
-#pragma unroll
-    for (int h = 0; h < 2; ++h)
-#pragma unroll
-        for (int e = 0; e < 8; ++e) eye[h][e] = (half_t)((lrow == h * 16 + lhalf * 8 + e) ? 1.0f : 0.0f);
-    float16v sum = acc;
-#pragma unroll
-    for (int h = 0; h < 2; ++h) sum = __builtin_amdgcn_mfma_f32_32x32x16_f16(eye[h], rv[h], sum, 0, 0, 0);
-    if (__any(!__builtin_isfinite(sum[0]))) {
-        sum = acc;
-#pragma unroll
-        for (int h = 0; h < 2; ++h) {
-            half8 f = rv[h];
-#pragma unroll
-            for (int e = 0; e < 8; ++e) f[e] = __builtin_isfinite((float)f[e]) ? f[e] : (half_t)0.0f;
-            sum = __builtin_amdgcn_mfma_f32_32x32x16_f16(eye[h], f, sum, 0, 0, 0);
-        }
-#pragma unroll
-        for (int g = 0; g < 4; ++g) {
-            const half4 r = own(g);
-#pragma unroll
-            for (int e = 0; e < 4; ++e)
-                if (!__builtin_isfinite((float)r[e])) sum[g * 4 + e] += (float)r[e];
-        }
-    }
-    return sum;
 }
 
 // SEG: maps of several column segments (one segment: the arithmetic of the
@@ -2452,8 +2415,8 @@ __global__ __launch_bounds__((WMG * WNG + NP) * 64) void conv3x3_bandws_kernel(C
     }
     if (has_res) lds_barrier();                       // the producers' residual tile has landed
 
-    // Epilogue: the residual through identity-operand MFMAs, [ReLU], f16 over
-    // the residual rows, then the wave's channel range of its pixel rows out
+    // Epilogue: + residual (each lane its own outputs'), [ReLU], f16 over the
+    // residual rows, then the wave's channel range of its pixel rows out
     // as 16-byte chunks.
     const bool relu = a.act == VDK_ACT_RELU;
 #pragma unroll
@@ -2461,15 +2424,14 @@ __global__ __launch_bounds__((WMG * WNG + NP) * 64) void conv3x3_bandws_kernel(C
         const int cw = cg0 + i * 32;
 #pragma unroll
         for (int j = 0; j < NJ; ++j) {
-            uint8_t* const prow = rrow((pg * NJ + j) * 32 + lrow);
-            uint8_t* const row = prow + (cw + lhalf * 4) * 2;
+            uint8_t* const row = rrow((pg * NJ + j) * 32 + lrow) + (cw + lhalf * 4) * 2;
             if (has_res) {
-                half8 rv[2];
 #pragma unroll
-                for (int h = 0; h < 2; ++h)
-                    rv[h] = *reinterpret_cast<const half8*>(prow + (cw + h * 16 + lhalf * 8) * 2);
-                acc[i][j] = add_residual_block(rv, acc[i][j], lrow, lhalf,
-                                               [&](int g) { return *reinterpret_cast<const half4*>(row + g * 16); });
+                for (int g = 0; g < 4; ++g) {
+                    const half4 rv = *reinterpret_cast<const half4*>(row + g * 16);
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) acc[i][j][g * 4 + e] += (float)rv[e];
+                }
             }
 #pragma unroll
             for (int g = 0; g < 4; ++g) {
@@ -2519,7 +2481,7 @@ void launch_bandws(const ConvArgs& args, hipStream_t s) {
 // the 16-byte halves swapped on odd groups of 8 rows as in the band kernels),
 // from lane offsets that stay fixed over the chunks.  The sums run in the band
 // kernels' order (chunks, taps; accumulators from the bias; the residual
-// through identity-operand MFMAs), so the results are the same bits.
+// added in f32), so the results are the same bits.
 // Bound by the latency of a chunk's way through LDS.
 // ---------------------------------------------------------------------------
 constexpr int kSlimStages = 4;   // 72 KB: two workgroups per CU (8 stages, one per CU: 9.6 -> 13.7 us at batch 2)
@@ -2585,11 +2547,11 @@ __global__ __launch_bounds__(192) void conv3x3_slim_kernel(ConvArgs a) {
     const int lrow = lane & 31, lhalf = lane >> 5;
     const int P = p0 + lrow;
     const bool ok = P < a.npix;
-    half8 rv[2] = {};
+    half4 rv[4] = {};
     if (a.res && ok) {
 #pragma unroll
-        for (int h = 0; h < 2; ++h)
-            rv[h] = *reinterpret_cast<const half8*>(a.res + (size_t)P * a.rs + oc0 + h * 16 + lhalf * 8);
+        for (int g = 0; g < 4; ++g)
+            rv[g] = *reinterpret_cast<const half4*>(a.res + (size_t)P * a.rs + oc0 + g * 8 + lhalf * 4);
     }
     float16v acc;   // register g*4+e of a lane: channel 8g + 4*lhalf + e
 #pragma unroll
@@ -2613,10 +2575,12 @@ __global__ __launch_bounds__(192) void conv3x3_slim_kernel(ConvArgs a) {
 #pragma unroll
         for (int t = 0; t < 9; ++t) acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[t], bf[t], acc, 0, 0, 0);
     }
-    if (a.res)
-        acc = add_residual_block(rv, acc, lrow, lhalf, [&](int g) {
-            return ok ? *reinterpret_cast<const half4*>(a.res + (size_t)P * a.rs + oc0 + g * 8 + lhalf * 4) : half4{};
-        });
+    if (a.res) {
+#pragma unroll
+        for (int g = 0; g < 4; ++g)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) acc[g * 4 + e] += (float)rv[g][e];
+    }
     // f16, then the lane halves trade 4-channel pieces, so each lane stores
     // two whole 8-channel chunks of its pixel
     const bool relu = a.act == VDK_ACT_RELU;
