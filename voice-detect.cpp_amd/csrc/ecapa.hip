@@ -314,12 +314,6 @@ __device__ __forceinline__ void asp_logits(const uint8_t* st, const half8* wf, i
     }
 }
 
-// x (4 channels: register group g of this lane's channel block) of frame
-// row `row` of a stage's swizzled x rows.
-__device__ __forceinline__ half4 asp_x4(const uint8_t* xs_lds, int row, int cb, int g, int lhalf) {
-    return *reinterpret_cast<const half4*>(xs_lds + row * 128 + (((cb * 4 + g) ^ (row & 7)) * 16) + lhalf * 8);
-}
-
 // Online-softmax state: running max and the sums scaled by exp(-m).
 struct AspState {
     float m;
