@@ -377,6 +377,39 @@ def test_kept_states_memory_comes_with_the_first_small_call():
         own.close()
 
 
+def test_analyze_captured_without_kept_states():
+    """One clip captured into a HIP graph in a context that has seen a large
+    call only: capture takes no memory (the states are pooled one by one), and
+    every replay, with eager calls between, gives the eager result."""
+    path = _model("emotion", 5, SMALL)
+    pcm = synth.clips(33, 171, 8000)
+    L, ctx, own = lib.lib(), lib.Context(path), lib.Context(path)
+    L.hipStreamBeginCapture.argtypes = [ctypes.c_void_p, ctypes.c_int]
+    L.hipStreamEndCapture.argtypes = [ctypes.c_void_p, ctypes.c_void_p]
+    L.hipGraphInstantiate.argtypes = [ctypes.c_void_p] * 4 + [ctypes.c_size_t]
+    L.hipGraphLaunch.argtypes = [ctypes.c_void_p, ctypes.c_void_p]
+    try:
+        announce("analyze emotion small: one clip captured after 171")
+        want = [own.analyze_pcm(pcm[c:c + 1]) for c in range(3)]
+        ctx.analyze_pcm(pcm)
+        stream = L.voicedetect_gpu_stream(ctx.ctx)
+        d_pcm, d_raw = lib.DeviceBuffer.from_array(pcm[:1]), lib.DeviceBuffer(want[0].nbytes)
+        graph, ex = ctypes.c_void_p(), ctypes.c_void_p()
+        assert L.hipStreamBeginCapture(stream, 1) == 0   # thread-local
+        ctx.analyze_device_async(d_pcm.ptr, 1, 8000, d_raw.ptr)
+        assert L.hipStreamEndCapture(stream, ctypes.byref(graph)) == 0
+        assert L.hipGraphInstantiate(ctypes.byref(ex), graph, None, None, 0) == 0
+        for c in (0, 1, 2, 0):
+            d_pcm.copy_from(pcm[c:c + 1])
+            assert L.hipGraphLaunch(ex, stream) == 0
+            ctx.synchronize()
+            assert np.array_equal(d_raw.to_array(np.float32, want[c].shape), want[c]), f"clip {c}"
+            assert np.array_equal(ctx.analyze_pcm(pcm[c:c + 1]), want[c])
+    finally:
+        ctx.close()
+        own.close()
+
+
 @pytest.mark.parametrize("kind", ["emotion", "age_gender"])
 def test_analyze_full_size(kind):
     """The published shapes (base: 768 x 12 layers; large-robust: 1024 x 24)
