@@ -1039,8 +1039,9 @@ __global__ __launch_bounds__((WMG * WNG + NP) * 64) void gemm_ws_kernel(ConvArgs
         for (int k = 0; k < nk; ++k) {
             lds_barrier();   // chunk k has landed; chunk k-1's reads are done
             const uint8_t* const sa = smem + (k % NST) * G::STAGE;
-// Wave tiles of one or two blocks have too few MFMAs to hide a
-            // fragment read behind: the chunk's reads all go out first.  Larger ones read one k-step ahead, between the MFMAs.
+            // Wave tiles of one or two blocks have too few MFMAs to hide a
+            // fragment read behind: the chunk's reads all go out first.
+            // Larger ones read one k-step ahead, between the MFMAs.
             constexpr bool kAll = TM * TN <= 2;
             constexpr int NB = kAll ? KS : 2;
             half8 af[NB][TM], bf[NB][TN];
@@ -2936,8 +2937,9 @@ bool tile_fits(const TileCfg& t, const ConvArgs& a) {
     }
     if (t.sp_ic) return a.IC == t.sp_ic && a.OC == t.bm && split_epilogue(a);
     // the GEMM kernel: channel groups whole per chunk, split-f16 plane terms
-    // as consecutive chunks of a tap (2-D taps: the small-launch tiles; prologue / segment sums: the EXT tiles, 1x1 without padding, up to
-    // 1024 input channels, pixel tiles at most seg_len wide)
+    // as consecutive chunks of a tap (2-D taps: the small-launch tiles;
+    // prologue / segment sums: the EXT tiles, 1x1 without padding, up to 1024
+    // input channels, pixel tiles at most seg_len wide)
     if (t.gemm) {
         const bool one = a.KH * a.KW == 1 && a.ph == 0 && a.pw == 0;
         if ((a.in_scale || a.segsum) && !(t.gemm_ext && one && !a.split)) return false;
